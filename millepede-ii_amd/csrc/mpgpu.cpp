@@ -147,6 +147,8 @@ struct mpgpu_ctx {
     DBuf<int64_t> d_inc_ptr;     // per batch: (nblock+1) pointers into d_inc_src
     DBuf<int64_t> d_inc_src;     // buffer offsets of the records' values for each block
     DBuf<double> d_cbuf;         // update buffer (largest batch)
+    RowStruct rows;              // records in row form; the others are in d_order
+    int64_t ngen = 0;            // records in d_order
     int band_grid = 0;
     int band_lfitbb = -1;
     int64_t nrec = 0;
@@ -1077,9 +1079,6 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         c->d_ccol_ptr.swap(blk.ccol_ptr);
         c->d_cc_off.swap(blk.cc_off);
         c->d_cc_fn.swap(blk.cc_fn);
-        // per record: block id of each segment pair
-        st_pair_blocks(sin, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, max_seg, d_rst, pm, c->d_rec_pb,
-                       c->d_pair_blk, s);
     } else {
         int64_t n = c->nall;
         c->nstored = n * (n + 1) / 2;
@@ -1149,6 +1148,66 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     std::vector<int64_t> order;
     st_order(nrec, c->ngroup, d_rst, c->d_order, order, s);
     phase("processing order");
+    // ---- records in row form leave d_order: every record whose equations each touch one small
+    // group and whose local fit has at most 5 parameters (k_rows_class); with residual monitoring
+    // the record kernel takes all of them ----
+    if (c->nband > 0) c->d_band_info.upload(binfo, s);
+    c->ngen = nrec;
+    std::vector<int64_t> row_upd;      // update sizes of the records in row form, when a batch size is set
+    if (sparse && c->opt.monitor == 0) {
+        std::vector<int32_t> tg_of(ntot), tg_t0, tg_v0;
+        std::vector<uint32_t> tg_mask;
+        for (int32_t t = 0; t < ntot; t++) {
+            if (bnd[t]) {
+                tg_t0.push_back(t);
+                tg_v0.push_back(0);
+                tg_mask.push_back(0);
+            }
+            tg_of[t] = (int32_t)tg_t0.size() - 1;
+            if (c->var_index[t] > 0) {
+                if (tg_v0.back() == 0) tg_v0.back() = c->var_index[t];
+                if (t - tg_t0.back() < 32) tg_mask.back() |= 1u << (t - tg_t0.back());
+            }
+        }
+        tg_t0.push_back(ntot);
+        // columns of a group: its variable parameters, then the fixed ones
+        std::vector<int32_t> col(ntot), ptix(ntot);
+        bool moved = false;
+        for (size_t g = 0; g + 1 < tg_t0.size(); g++) {
+            int32_t a = 0;
+            for (int pass = 0; pass < 2; pass++)
+                for (int32_t t = tg_t0[g]; t < tg_t0[g + 1]; t++)
+                    if ((c->var_index[t] > 0) == (pass == 0)) {
+                        col[t] = a;
+                        ptix[tg_t0[g] + a] = t;
+                        moved = moved || a != t - tg_t0[g];
+                        a++;
+                    }
+        }
+        if (moved) c->rows.ptix.upload(ptix, s);
+        DBuf<int32_t> d_of, d_t0, d_v0, d_col;
+        d_col.upload(col, s);
+        DBuf<uint32_t> d_mask;
+        d_of.upload(tg_of, s);
+        d_t0.upload(tg_t0, s);
+        d_v0.upload(tg_v0, s);
+        d_mask.upload(tg_mask, s);
+        const RowGroups Q{d_of.p, d_t0.p, c->d_var.p, d_col.p, d_mask.p, d_v0.p};
+        std::vector<uint8_t> cls;
+        rows_classify(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->nband > 0 ? c->d_band_info.p : nullptr, Q, c->rows, cls, s);
+        std::vector<int64_t> fast, gen;
+        fast.reserve(nrec);
+        for (int64_t q = 0; q < nrec; q++) (cls[order[q]] ? fast : gen).push_back(order[q]);
+        if (std::getenv("MPGPU_UPDATE_BUFFER_GB"))
+            for (int64_t r : fast) row_upd.push_back(cnt_r[r]);
+        for (int64_t r : fast) cnt_r[r] = 0;
+        rows_build(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, Q, fast, c->rows, s);
+        c->ngen = (int64_t)gen.size();
+        c->d_order.upload(gen, s);
+        HIPCHK(hipStreamSynchronize(s));     // the tables above end here
+        order.swap(gen);
+        phase("records in row form");
+    }
     // ---- two-phase build index (group-block storage) ----
     // Each record writes its update of every segment pair (r-major block, lower triangle for the
     // diagonal pairs) contiguously into a buffer; the block gather sums, for every stored block,
@@ -1172,9 +1231,15 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             else (void)hipGetLastError();
         }
         const int64_t budget = std::max<int64_t>(1 << 20, (int64_t)(gb * (1ull << 30) / 8.0));
+        rows_incidence(c->rows, c->d_group_of.p, pm, c->nblock, budget, row_upd, s);
+        phase("row incidence lists");
+        // the other records: per record the block id of each segment pair
+        if (c->ngen > 0)
+            st_pair_blocks(sin, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, max_seg, d_rst, pm, c->d_rec_pb,
+                           c->d_pair_blk, s);
         std::vector<int64_t> bat_inc;                   // incidences of every batch
         int64_t q0 = 0, acc = 0, ninc = 0;
-        for (int64_t q = 0; q < nrec; q++) {
+        for (int64_t q = 0; q < c->ngen; q++) {
             const int64_t r = order[q];
             if (acc + cnt_r[r] > budget && q > q0) {
                 c->batches.push_back({q0, q, 0, acc, 0});
@@ -1188,8 +1253,8 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             acc += cnt_r[r];
             if (cnt_r[r] > 0) ninc += (int64_t)st_nseg[r] * (st_nseg[r] + 1) / 2;
         }
-        if (nrec > q0 || c->batches.empty()) {
-            c->batches.push_back({q0, nrec, 0, acc, 0});
+        if (c->ngen > q0) {
+            c->batches.push_back({q0, c->ngen, 0, acc, 0});
             bat_inc.push_back(ninc);
         }
         c->d_rec_cb.upload(rec_cb, s);
@@ -1201,7 +1266,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             c->batches[bt].inc0 = inc_total;
             inc_total += bat_inc[bt];
         }
-        c->d_inc_ptr.alloc((size_t)nbat * (nb + 1));
+        c->d_inc_ptr.alloc(std::max<size_t>((size_t)nbat * (nb + 1), 1));
         c->d_inc_src.alloc(std::max<int64_t>(inc_total, 1));
         for (int64_t bt = 0; bt < nbat; bt++) {
             const auto &B = c->batches[bt];
@@ -1235,9 +1300,8 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     if (c->nband > 0) {
         std::vector<int64_t> ids;
         ids.reserve(c->nband);
-        for (int64_t q = 0; q < nrec; q++) if (binfo[order[q]]) ids.push_back(order[q]);
+        for (int64_t q = 0; q < c->ngen; q++) if (binfo[order[q]]) ids.push_back(order[q]);
         c->d_band_ids.upload(ids, s);
-        c->d_band_info.upload(binfo, s);
         c->d_band_scratch.alloc((size_t)c->band_grid * c->bplan.vinv_stride);
     } else {
         c->d_band_ids.release();
@@ -1479,9 +1543,29 @@ extern "C" int mpgpu_loopn(mpgpu_ctx *c, int32_t icalcm, int32_t nloopn, float c
         mon = MonCtx{c->d_mon_grp.p, c->d_mon_res.p, c->d_mon_hist.p, c->mon_bins, c->opt.monitor};
         c->d_mon_hist.zero(s);   // histograms of this pass only (src/pede.f90:2607)
     }
-    int grid = (int)std::min<int64_t>(c->nrec, 256 * 40);
+    int grid = (int)std::min<int64_t>(c->ngen, 256 * 40);
     HIPCHK(hipEventRecord(e1, s));
-    if (c->nrec > 0) {
+    if (c->rows.nq > 0) {
+        // records in row form
+        const RowStruct &S = c->rows;
+        RowDev D{S.hdr.p, S.rows.p, S.eq_t0.p, S.eq_pos.p, S.seq.p, S.seg.p, S.ptix.p, c->ntot, 0, S.unit.p, S.side.p};
+        const bool build = icalcm == 1;
+        for (size_t bt = 0; bt < (build ? S.batches.size() : 1); bt++) {
+            const int64_t q0 = build ? S.batches[bt].q0 : 0, q1 = build ? S.batches[bt].q1 : S.nq;
+            if (build) D.ub = S.batches[bt].unit0;
+            auto tr = timed(t_rec);
+            HIPCHK(hipEventRecord(tr.first, s));
+            HIPCHK(launch_rows(S, D, M, o, out, build, q0, q1, s));
+            HIPCHK(hipEventRecord(tr.second, s));
+            if (!build) break;
+            auto tg = timed(t_gat);
+            HIPCHK(hipEventRecord(tg.first, s));
+            HIPCHK(launch_rows_gather(S, bt, c->ngroup, c->nblock, c->d_brow.p, c->d_boff.p, c->d_brg.p, c->d_bcol.p,
+                                      c->d_gfirst.p, c->d_mat.p, c->d_vec.p, c->d_cnt.p, s));
+            HIPCHK(hipEventRecord(tg.second, s));
+        }
+    }
+    if (c->ngen > 0) {
         if (icalcm == 1 && c->opt.matsto == MPGPU_SPARSE) {
             // two-phase build: each batch of records writes its updates, then the blocks gather them
             for (size_t bt = 0; bt < c->batches.size(); bt++) {
@@ -1502,7 +1586,7 @@ extern "C" int mpgpu_loopn(mpgpu_ctx *c, int32_t icalcm, int32_t nloopn, float c
         } else {
             auto tr = timed(t_rec);
             HIPCHK(hipEventRecord(tr.first, s));
-            HIPCHK(launch_records(R, M, o, out, c->plan, 0, c->nrec, std::max(grid, 1), s, mon));
+            HIPCHK(launch_records(R, M, o, out, c->plan, 0, c->ngen, std::max(grid, 1), s, mon));
             HIPCHK(hipEventRecord(tr.second, s));
         }
     }

@@ -75,6 +75,37 @@ struct RecOut {
                      // 8 needs bordered-band local fit, 9 exceeds kernel limits, 20 bad record
 };
 
+// ---- records in row form (k_rows.hip) ---------------------------------------------------
+// one record: first row (equation), first entry of its group table and first unit over all such
+// records in processing order
+struct RowHdr {
+    int64_t row0, seg0, unit0, rec;
+    int32_t neq, nseg, nalc, nunit;
+};
+// parameter groups over all total indices
+struct RowGroups {
+    const int32_t *of;      // [ntot] group of a total index
+    const int32_t *t0;      // [ngroups + 1] first total index
+    const int32_t *var;     // [ntot] variable index (1-based) or <= 0
+    const int32_t *col;     // [ntot] column in its group: the variable parameters first
+    const uint32_t *mask;   // [ngroups] which of its parameters are variable (groups of up to 8)
+    const int32_t *v0;      // [ngroups] first variable index (1-based)
+};
+struct RowDev {
+    const RowHdr *hdr;
+    const void *rows;       // one row per equation (RowLayout)
+    const int32_t *eq_t0;   // first total index of the equation's group, -1: no global parameters
+    const uint16_t *eq_pos; // place of the equation in the record's units
+    const uint16_t *seq;    // equations of each group of a record
+    const int4 *seg;        // group table: first variable, equations (first | count << 16),
+                            // variables, units (first | count << 16)
+    const int32_t *ptix;    // total index of column j of the group at t0: ptix[t0 + j] (null: t0 + j)
+    int32_t ntot;
+    int64_t ub;             // first unit of the batch
+    void *unit;             // units (UnitLayout) of the batch
+    double *side;           // per unit: w of its two equations, w x residual of both
+};
+
 // LDS plan of the record kernel (all counts in elements)
 struct LdsPlan {
     int32_t max_gl, max_eq, nalc_max, max_var, max_pair;

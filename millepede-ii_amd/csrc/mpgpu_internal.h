@@ -331,6 +331,37 @@ void st_incidence(const StructIn &in, const DBuf<int64_t> &rec_gl, const DBuf<in
                   const DBuf<int32_t> &pair_blk, const DBuf<int64_t> &rec_cb, int64_t q0, int64_t q1, int64_t nblock,
                   int64_t *ptr, int64_t *src, int64_t nsrc, hipStream_t s);
 
+// ---- records in row form (k_rows.hip) ----
+struct RowStruct {
+    struct Batch { int64_t q0, q1, unit0, nunit, inc0, npair; };
+    int64_t nq = 0, nrow = 0, nseg = 0, nunit = 0, npair = 0;
+    int kp = 4, gp = 6, max_eq = 0;   // local and group columns of a row, most equations of a record
+    bool dbl = false;
+    DBuf<int32_t> n;                  // per record counts (k_rows_class)
+    DBuf<int64_t> order, c;           // processing order; running sums of the counts in that order
+    DBuf<RowHdr> hdr;
+    DBuf<uint8_t> rows;
+    DBuf<int32_t> eq_t0, ptix;
+    DBuf<uint16_t> eq_pos, seq;
+    DBuf<int4> seg;
+    std::vector<Batch> batches;       // matrix build: batches of records and their incidence lists
+    DBuf<uint32_t> ptr;
+    DBuf<uint2> src;
+    DBuf<uint8_t> unit;               // units and side array of the largest batch
+    DBuf<double> side;
+};
+void rows_classify(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix,
+                   const int32_t *band, const RowGroups &Q, RowStruct &S, std::vector<uint8_t> &cls, hipStream_t s);
+void rows_build(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix,
+                const RowGroups &Q, const std::vector<int64_t> &order, RowStruct &S, hipStream_t s);
+void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, int64_t nblock, int64_t budget,
+                    const std::vector<int64_t> &upd, hipStream_t s);
+hipError_t launch_rows(const RowStruct &S, const RowDev &R, const DevModel &M, const PassOpts &o, const RecOut &out, bool build,
+                       int64_t q0, int64_t q1, hipStream_t s);
+hipError_t launch_rows_gather(const RowStruct &S, size_t batch, int32_t ngroup, int64_t nblock, const int64_t *brow,
+                              const int64_t *boff, const int32_t *brg, const int32_t *bcol, const int32_t *gfirst, double *mat,
+                              double *vec, unsigned long long *cnt, hipStream_t s);
+
 // ---- constraint elimination (mpgpu_qldec.cpp, k_qlelim.hip) ----
 // device view of the reflectors: rows over parameter ranges, the transpose per parameter, the WY
 // factor T and two m-vectors of scratch
