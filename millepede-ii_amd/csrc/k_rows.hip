@@ -34,6 +34,7 @@ namespace mpgpu {
 #define MAXEQ 128                // equations per record: two per lane
 #define MAXGRP 8                 // parameters of a group (fixed ones included)
 #define MAXSEG 128               // groups, and units, per record
+#define PERM_WINDOW 4096         // blocks whose order the gather may change
 #define MAXSEQ 4                 // equations of one group in a record
 
 __device__ __forceinline__ void rsync()
@@ -175,11 +176,19 @@ template <typename T, int KP, int GP> struct RowLayout {
     static constexpr int V = 16 / (int)sizeof(T);                   // values per 16 bytes
     static constexpr int RS = (2 + KP + GP + V - 1) / V * V;        // row stride
 };
-// a unit: q of its two equations, their group derivatives, the signs S (bit k: D_k < 0)
+// A unit in pieces of 16 bytes: q of its two equations (NQ pieces each), then the two halves of the
+// group derivatives (NH pieces each: HM values of the first equation, HM of the second, and the
+// signs S, bit k: D_k < 0).  Four lanes load a unit in whole lines, one piece each at a time, and
+// exchange pieces (k_rows_gather).
 template <typename T, int KP, int GP> struct UnitLayout {
-    static constexpr int G = 2 * KP * 8;                            // byte offsets
-    static constexpr int SG = G + 2 * GP * (int)sizeof(T);
-    static constexpr int BYTES = (SG + 4 + 15) / 16 * 16;
+    static constexpr int HM = GP / 2;
+    static constexpr int NQ = KP / 2;
+    static constexpr int SG = 2 * HM * (int)sizeof(T);              // signs, byte offset in a half
+    static constexpr int NH = (SG + 4 + 15) / 16;
+    static constexpr int NP = 2 * (NQ + NH);
+    static constexpr int BYTES = 16 * NP;
+    static __host__ __device__ constexpr int q(int e) { return 16 * NQ * e; }
+    static __host__ __device__ constexpr int h(int x) { return 16 * (2 * NQ + NH * x); }
 };
 
 // One wavefront per record: its header, rows, group table, the equations of each group and the
@@ -346,6 +355,29 @@ __global__ void k_rows_ptr(int64_t n, const uint32_t *key, int64_t nk, uint32_t 
         const int64_t hi = i == n ? nk : (int64_t)key[i];
         for (int64_t k = lo + 1; k <= hi; k++) ptr[k] = (uint32_t)i;
     }
+}
+
+// Slots that share a block in the gather, by the length of its list: with one slot a list of 32
+// pairs takes 32 steps, longer ones are split so that no wavefront runs much longer than the rest.
+__device__ __forceinline__ int len_class(uint32_t n) { return n >= 128u ? 0 : n >= 32u ? 1 : 2; }
+
+// sort key of a block: its class (3: diagonal or empty), its window of neighbouring blocks, then
+// descending list length
+__global__ void k_rows_len(int64_t nb, const uint32_t *ptr, const int32_t *brg, const int32_t *bcol, uint64_t *key,
+                           uint32_t *val, unsigned long long *ncls)
+{
+    __shared__ unsigned s_n[4];
+    if (threadIdx.x < 4) s_n[threadIdx.x] = 0u;
+    __syncthreads();
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < nb; k += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t n = ptr[k + 1] - ptr[k];
+        const int c = n == 0 || brg[k] == bcol[k] ? 3 : len_class(n);
+        key[k] = ((uint64_t)c << 36) | ((uint64_t)(k / PERM_WINDOW) << 12) | (uint64_t)(4095u - min(n, 4095u));
+        val[k] = (uint32_t)k;
+        atomicAdd(&s_n[c], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 && s_n[threadIdx.x]) atomicAdd(&ncls[threadIdx.x], (unsigned long long)s_n[threadIdx.x]);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -684,22 +716,28 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
             }
             const int un = (int)((pos & 0x7fffu) >> 1), half = (int)(pos & 1u);
             char *u = U + (int64_t)un * UL::BYTES;
-            double *uq = (double *)u + half * KP;
-            T *ug = (T *)(u + UL::G) + half * GP;
+            double *uq = (double *)(u + UL::q(half));
 #pragma unroll
             for (int k = 0; k < KP; k += 2) *(double2 *)&uq[k] = make_double2(qv[k], qv[k + 1]);
             const T *row = rows + (h.row0 + i) * RS + 2 + KP;
 #pragma unroll
-            for (int j = 0; j < GP; j++) ug[j] = row[j];
-            if (half == 0) *(int *)(u + UL::SG) = sg;
+            for (int x = 0; x < 2; x++) {
+                T *ug = (T *)(u + UL::h(x)) + half * UL::HM;
+#pragma unroll
+                for (int j = 0; j < UL::HM; j++) ug[j] = row[x * UL::HM + j];
+                if (half == 0) *(int *)(u + UL::h(x) + UL::SG) = sg;
+            }
             S[4 * un + half] = wght;
             S[4 * un + 2 + half] = wght * rmeas;
             if (pos & 0x8000u) {
                 // no second equation in this unit
+                double *u1 = (double *)(u + UL::q(1));
 #pragma unroll
-                for (int k = 0; k < KP; k += 2) *(double2 *)&uq[KP + k] = make_double2(0.0, 0.0);
+                for (int k = 0; k < KP; k += 2) *(double2 *)&u1[k] = make_double2(0.0, 0.0);
 #pragma unroll
-                for (int j = 0; j < GP; j++) ug[GP + j] = (T)0;
+                for (int x = 0; x < 2; x++)
+#pragma unroll
+                    for (int j = 0; j < UL::HM; j++) ((T *)(u + UL::h(x)))[UL::HM + j] = (T)0;
                 S[4 * un + 1] = 0.0;
                 S[4 * un + 3] = 0.0;
             }
@@ -757,113 +795,160 @@ template <int R> __device__ __forceinline__ double row_ror(double v)
     return __hiloint2double(hi, lo);
 }
 
-// One pair of units, four lanes (e, f) or (ti, tj): a lane forms s_ef, the four exchange theirs,
-// and each has a quarter of the 2HM x 2HM contribution sum_ef g_e s_ef g_f^T: rows ti*HM..,
-// columns tj*HM...
-template <typename T, int KP, int GP, int HM> struct UnitPair {
+// one dword of lane A (even half) / lane B (odd half) of the four; HI: the half is bit 1 of the
+// lane, else bit 0.  Pieces 0, 1, ... lie in loads 0, 0, 0, 0, 1, ... of lanes 0, 1, 2, 3, 0, ...
+template <int PERM> __device__ __forceinline__ int quad_i(int v) { return __builtin_amdgcn_mov_dpp(v, PERM, 0xf, 0xf, true); }
+template <int A, int B, bool HI, int NI> __device__ __forceinline__ int4 piece(const int4 (&w)[NI], bool odd)
+{
+    constexpr int a = A & 3, b = B & 3;
+    if constexpr (A / 4 == B / 4) {
+        constexpr int P = HI ? a | a << 2 | b << 4 | b << 6 : a | b << 2 | a << 4 | b << 6;
+        const int4 v = w[A / 4];
+        return make_int4(quad_i<P>(v.x), quad_i<P>(v.y), quad_i<P>(v.z), quad_i<P>(v.w));
+    } else {
+        constexpr int P = a * 0x55, Q = b * 0x55;
+        const int4 v = w[A / 4], u = w[B / 4];
+        // both exchanges by all lanes, then the choice
+        const int4 x = make_int4(quad_i<P>(v.x), quad_i<P>(v.y), quad_i<P>(v.z), quad_i<P>(v.w));
+        const int4 y = make_int4(quad_i<Q>(u.x), quad_i<Q>(u.y), quad_i<Q>(u.z), quad_i<Q>(u.w));
+        return odd ? y : x;
+    }
+}
+// pieces BASE.. (even half) or BASE + N.. (odd half)
+template <int BASE, int N, bool HI, int NI, int I = 0>
+__device__ __forceinline__ void pieces(const int4 (&w)[NI], bool odd, int4 *out)
+{
+    if constexpr (I < N) {
+        out[I] = piece<BASE + I, BASE + N + I, HI>(w, odd);
+        pieces<BASE, N, HI, NI, I + 1>(w, odd, out);
+    }
+}
+
+// One pair of units a, b on four lanes (hi, lo): lane (e, f) forms s_ef, the four exchange theirs,
+// and each has a quarter of the contribution sum_ef g_e m_ef g_f^T: rows hi*HM.., columns lo*HM...
+template <typename T, int KP, int GP> struct UnitRaw {
     typedef UnitLayout<T, KP, GP> UL;
-    double2 qa[KP / 2], qb[KP / 2];
-    T ga[2][HM], gb[2][HM];
-    int sg;
-    __device__ __forceinline__ void load(const char *unit, uint2 p, int hi, int lo)
+    static constexpr int NI = (UL::NP + 3) / 4;
+    int4 w[NI];
+    __device__ __forceinline__ void load(const char *unit, uint32_t p, int lane)
     {
-        const char *a = unit + (int64_t)p.x * UL::BYTES, *b = unit + (int64_t)p.y * UL::BYTES;
-        const double2 *x = (const double2 *)a + hi * (KP / 2), *y = (const double2 *)b + lo * (KP / 2);
+        const int4 *u = (const int4 *)(unit + (int64_t)p * UL::BYTES);
 #pragma unroll
-        for (int k = 0; k < KP / 2; k++) { qa[k] = x[k]; qb[k] = y[k]; }
-        const T *g = (const T *)(a + UL::G) + hi * HM, *h = (const T *)(b + UL::G) + lo * HM;
-#pragma unroll
-        for (int e = 0; e < 2; e++)
-#pragma unroll
-            for (int k = 0; k < HM; k++) { ga[e][k] = g[e * GP + k]; gb[e][k] = h[e * GP + k]; }
-        sg = *(const int *)(a + UL::SG);
-    }
-    __device__ __forceinline__ double dot() const
-    {
-        double s = 0.0;
-        if (__any(sg != 0)) {
-#pragma unroll
-            for (int k = 0; k < KP / 2; k++) {
-                s += (sg >> (2 * k)) & 1 ? -qa[k].x * qb[k].x : qa[k].x * qb[k].x;
-                s += (sg >> (2 * k + 1)) & 1 ? -qa[k].y * qb[k].y : qa[k].y * qb[k].y;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < KP / 2; k++) s = s + qa[k].x * qb[k].x + qa[k].y * qb[k].y;
-        }
-        return s;
-    }
-    // acc += sum_ef g_e m_ef g_f^T
-    __device__ __forceinline__ void add(double m00, double m01, double m10, double m11, double (&acc)[HM][HM]) const
-    {
-        double b0[HM], b1[HM];
-#pragma unroll
-        for (int y = 0; y < HM; y++) { b0[y] = (double)gb[0][y]; b1[y] = (double)gb[1][y]; }
-#pragma unroll
-        for (int x = 0; x < HM; x++) {
-            const double g0 = (double)ga[0][x], g1 = (double)ga[1][x];
-            const double t0 = g0 * m00 + g1 * m10, t1 = g0 * m01 + g1 * m11;
-#pragma unroll
-            for (int y = 0; y < HM; y++) acc[x][y] = acc[x][y] + t0 * b0[y] + t1 * b1[y];
-        }
+        for (int t = 0; t < NI; t++) w[t] = u[min(4 * t + (lane & 3), UL::NP - 1)];
     }
 };
+template <typename T, int KP, int GP, bool HI> struct UnitHalf {
+    typedef UnitLayout<T, KP, GP> UL;
+    union { int4 v[UL::NQ]; double d[KP]; } q;
+    union { int4 v[UL::NH]; T d[UL::NH * 16 / sizeof(T)]; int i[UL::NH * 4]; } g;
+    __device__ __forceinline__ void take(const UnitRaw<T, KP, GP> &r, bool odd)
+    {
+        pieces<0, UL::NQ, HI>(r.w, odd, q.v);
+        pieces<2 * UL::NQ, UL::NH, HI>(r.w, odd, g.v);
+    }
+};
+template <typename T, int KP, int GP>
+__device__ __forceinline__ double unit_dot(const UnitHalf<T, KP, GP, true> &a, const UnitHalf<T, KP, GP, false> &b)
+{
+    const int sg = a.g.i[UnitLayout<T, KP, GP>::SG / 4];
+    double s = 0.0;
+    if (__any(sg != 0)) {
+#pragma unroll
+        for (int k = 0; k < KP; k++) s += (sg >> k) & 1 ? -a.q.d[k] * b.q.d[k] : a.q.d[k] * b.q.d[k];
+    } else {
+#pragma unroll
+        for (int k = 0; k < KP; k++) s = s + a.q.d[k] * b.q.d[k];
+    }
+    return s;
+}
+template <typename T, int KP, int GP>
+__device__ __forceinline__ void unit_add(const UnitHalf<T, KP, GP, true> &a, const UnitHalf<T, KP, GP, false> &b, double m00,
+                                         double m01, double m10, double m11, double (&acc)[GP / 2][GP / 2])
+{
+    constexpr int HM = GP / 2;
+    double b0[HM], b1[HM];
+#pragma unroll
+    for (int y = 0; y < HM; y++) { b0[y] = (double)b.g.d[y]; b1[y] = (double)b.g.d[HM + y]; }
+#pragma unroll
+    for (int x = 0; x < HM; x++) {
+        const double g0 = (double)a.g.d[x], g1 = (double)a.g.d[HM + x];
+        const double t0 = g0 * m00 + g1 * m10, t1 = g0 * m01 + g1 * m11;
+#pragma unroll
+        for (int y = 0; y < HM; y++) acc[x][y] = acc[x][y] + t0 * b0[y] + t1 * b1[y];
+    }
+}
 
-// Off-diagonal blocks: SL slots of four lanes per block (64 / (4 SL) blocks per wavefront), a slot
-// takes every SL-th pair of units of the block; the slots' sums are added in a fixed order at the
-// end.  The next pair's values are loaded before the current one is used.
+// Off-diagonal blocks: SL slots of four lanes per block (16 / SL blocks per wavefront), a slot takes
+// every SL-th pair of units of the block; the slots' sums are added in a fixed order at the end.
+// Blocks are taken in `perm`'s order: by list length within a window of neighbouring blocks, so the
+// blocks of a wavefront have lists of like length.  Units are loaded two pairs ahead.
 template <typename T, int KP, int GP, int SL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rows_gather(int64_t nblock, const int64_t *boff, const int32_t *brg,
-                                                     const int32_t *bcol, const int32_t *gfirst, const uint32_t *ptr,
-                                                     const uint2 *src, const char *unit, double *mat)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+void k_rows_gather(int64_t nblock /* of this class */, const uint32_t *perm, const int64_t *boff, const int32_t *brg, const int32_t *bcol,
+                   const int32_t *gfirst, const uint32_t *ptr, const uint2 *src, const char *unit, double *mat)
 {
     constexpr int HM = GP / 2;
     const int lane = threadIdx.x & 63;
-    const int64_t k = (xcd_run(blockIdx.x, gridDim.x, 64) * 256 + threadIdx.x) / (4 * SL);
+    const int64_t p = (xcd_run(blockIdx.x, gridDim.x, 64) * 256 + threadIdx.x) / (4 * SL);
     const int slot = (lane >> 2) & (SL - 1), hi = (lane >> 1) & 1, lo = lane & 1;
-    uint32_t i0 = 0, i1 = 0;
+    uint32_t i0 = 0, i1 = 0, k = 0;
     int ga = 0, gb = 0;
-    if (k < nblock) {
+    if (p < nblock) {
+        k = perm[p];
         ga = brg[k];
         gb = bcol[k];
-        if (ga != gb) { i0 = ptr[k]; i1 = ptr[k + 1]; }
+        i0 = ptr[k];
+        i1 = ptr[k + 1];
     }
     double acc[HM][HM];
 #pragma unroll
     for (int x = 0; x < HM; x++)
 #pragma unroll
         for (int y = 0; y < HM; y++) acc[x][y] = 0.0;
-    UnitPair<T, KP, GP, HM> cur, nxt;
+    // a0, b0: the current pair; a1, b1: the next; n2: the places of the one after
+    UnitRaw<T, KP, GP> a0, b0, a1, b1;
     uint32_t i = i0 + slot;
-    uint2 pn = make_uint2(0, 0);
-    if (i < i1) cur.load(unit, src[i], hi, lo);
-    if (i + SL < i1) pn = src[i + SL];
-    while (__any(i < i1)) {
-        const bool more = i + SL < i1;
-        if (more) nxt.load(unit, pn, hi, lo);
-        if (i + 2 * SL < i1) pn = src[i + 2 * SL];
-        if (i < i1) {
-            const double s = cur.dot();
-            cur.add(quad<0x00>(s), quad<0x55>(s), quad<0xaa>(s), quad<0xff>(s), acc);
-        }
-        if (more) cur = nxt;
+    uint2 n2 = make_uint2(0, 0);
+    const uint32_t last = i1 > 0 ? i1 - 1 : 0;
+    if (i1 > i0) {
+        const uint2 x = src[min(i, last)], y = src[min(i + SL, last)];
+        n2 = src[min(i + 2 * SL, last)];
+        a0.load(unit, x.x, lane);
+        b0.load(unit, x.y, lane);
+        a1.load(unit, y.x, lane);
+        b1.load(unit, y.y, lane);
+    }
+    while (i < i1) {
+        UnitHalf<T, KP, GP, true> A;
+        UnitHalf<T, KP, GP, false> B;
+        A.take(a0, hi);
+        B.take(b0, lo);
+        a0 = a1;
+        b0 = b1;
+        a1.load(unit, n2.x, lane);
+        b1.load(unit, n2.y, lane);
+        n2 = src[min(i + 3 * SL, last)];
+        const double s = unit_dot<T, KP, GP>(A, B);
+        unit_add<T, KP, GP>(A, B, quad<0x00>(s), quad<0x55>(s), quad<0xaa>(s), quad<0xff>(s), acc);
         i += SL;
     }
     const int nr = gfirst[ga + 1] - gfirst[ga], nc = gfirst[gb + 1] - gfirst[gb];
-    double *B = k < nblock ? mat + boff[k] : nullptr;
+    double *Bk = mat + (p < nblock ? boff[k] : 0);
 #pragma unroll
     for (int x = 0; x < HM; x++)
 #pragma unroll
         for (int y = 0; y < HM; y++) {
             double v = acc[x][y];
-            v += row_ror<4>(v);
-            v += row_ror<8>(v);
+            if (SL > 1) {
+                v += row_ror<4>(v);
+                v += row_ror<8>(v);
+            }
             if (SL > 4) {
                 v += __shfl_xor(v, 16, WV);
                 v += __shfl_xor(v, 32, WV);
             }
             const int rr = hi * HM + x, cc = lo * HM + y;
-            if (i1 > i0 && slot == ((x * HM + y) & (SL - 1)) && rr < nr && cc < nc) B[rr * nc + cc] -= v;
+            if (i1 > i0 && slot == ((x * HM + y) & (SL - 1)) && rr < nr && cc < nc) Bk[rr * nc + cc] -= v;
         }
 }
 
@@ -894,26 +979,33 @@ __global__ __launch_bounds__(256) void k_rows_gather_diag(int32_t ngroup, const 
 #pragma unroll
         for (int y = 0; y < HM; y++) acc[x][y] = 0.0;
     }
-    UnitPair<T, KP, GP, HM> u;
+    UnitRaw<T, KP, GP> a, b;
+    UnitHalf<T, KP, GP, true> A;
+    UnitHalf<T, KP, GP, false> B;
     for (uint32_t i = i0 + wv * 16 + slot; i < i1; i += 64) {
         const uint2 p = src[i];
-        u.load(unit, p, hi, lo);
-        const double s = -u.dot();
+        a.load(unit, p.x, lane);
+        if (p.x == p.y) b = a;
+        else b.load(unit, p.y, lane);
+        A.take(a, hi);
+        B.take(b, lo);
+        const double s = -unit_dot<T, KP, GP>(A, B);
         double m00 = quad<0x00>(s), m01 = quad<0x55>(s), m10 = quad<0xaa>(s), m11 = quad<0xff>(s);
         if (p.x == p.y) {
             const double2 w = ((const double2 *)side)[2 * (int64_t)p.x], wr = ((const double2 *)side)[2 * (int64_t)p.x + 1];
             m00 += w.x;
             m11 += w.y;
-            u.add(m00, m01, m10, m11, acc);
+            unit_add<T, KP, GP>(A, B, m00, m01, m10, m11, acc);
 #pragma unroll
             for (int x = 0; x < HM; x++) {
-                v[x] = v[x] + wr.x * (double)u.ga[0][x] + wr.y * (double)u.ga[1][x];
-                c[x] += (u.ga[0][x] != (T)0) + (u.ga[1][x] != (T)0);
+                v[x] = v[x] + wr.x * (double)A.g.d[x] + wr.y * (double)A.g.d[HM + x];
+                c[x] += (A.g.d[x] != (T)0) + (A.g.d[HM + x] != (T)0);
             }
         } else {
-            u.add(m00, m01, m10, m11, acc);
-            u.load(unit, make_uint2(p.y, p.x), hi, lo);
-            u.add(m00, m10, m01, m11, acc);
+            unit_add<T, KP, GP>(A, B, m00, m01, m10, m11, acc);
+            A.take(b, hi);
+            B.take(a, lo);
+            unit_add<T, KP, GP>(A, B, m00, m10, m01, m11, acc);
         }
     }
 #pragma unroll
@@ -1048,15 +1140,15 @@ template <typename T> static int unit_bytes_t(const RowStruct &S)
 // buffers of the pairs (24 bytes each) of a batch within `budget` doubles, at most 2^30 pairs.
 // upd (when not empty): the size of each record's update, held against the budget instead (a
 // budget set by MPGPU_UPDATE_BUFFER_GB counts updates, as it does for the other records)
-void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, int64_t nblock, int64_t budget,
-                    const std::vector<int64_t> &upd, hipStream_t s)
+void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, int64_t nblock, const int32_t *brg,
+                    const int32_t *bcol, int64_t budget, const std::vector<int64_t> &upd, hipStream_t s)
 {
     S.batches.clear();
     if (S.nq == 0) return;
     const int ubytes = S.dbl ? unit_bytes_t<double>(S) : unit_bytes_t<float>(S);
     const int64_t n1 = S.nq + 1, maxpair = (int64_t)1 << 30, ud = ubytes / 8 + 4;
     if (upd.empty() && ud * S.nunit + 3 * S.npair <= budget && S.npair <= maxpair) {
-        S.batches.push_back({0, S.nq, 0, S.nunit, 0, S.npair});
+        S.batches.push_back({0, S.nq, 0, S.nunit, 0, S.npair, {0, 0, 0}});
     } else {
         std::vector<int64_t> c(2 * n1);
         HIPCHK(hipMemcpyAsync(c.data(), S.c.p + 2 * n1, sizeof(int64_t) * 2 * n1, hipMemcpyDeviceToHost, s));
@@ -1066,14 +1158,14 @@ void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, in
         for (int64_t q = 0; q < S.nq; q++) {
             const int64_t d = upd.empty() ? ud * (cu[q + 1] - cu[q]) + 3 * (cp[q + 1] - cp[q]) : upd[q];
             if (q > q0 && (size + d > budget || cp[q + 1] - cp[q0] > maxpair)) {
-                S.batches.push_back({q0, q, cu[q0], cu[q] - cu[q0], inc, cp[q] - cp[q0]});
+                S.batches.push_back({q0, q, cu[q0], cu[q] - cu[q0], inc, cp[q] - cp[q0], {0, 0, 0}});
                 inc += cp[q] - cp[q0];
                 q0 = q;
                 size = 0;
             }
             size += d;
         }
-        S.batches.push_back({q0, S.nq, cu[q0], S.nunit - cu[q0], inc, S.npair - cp[q0]});
+        S.batches.push_back({q0, S.nq, cu[q0], S.nunit - cu[q0], inc, S.npair - cp[q0], {0, 0, 0}});
     }
     int64_t mu = 1, mp = 1;
     for (const auto &B : S.batches) {
@@ -1105,6 +1197,31 @@ void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, in
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(s));
+    // order of the blocks in the gather, per batch
+    S.perm.alloc(S.batches.size() * (size_t)nblock);
+    {
+        DBuf<uint64_t> q0, q1;
+        DBuf<uint32_t> p0;
+        DBuf<unsigned long long> nc;
+        DBuf<uint8_t> t2;
+        q0.alloc(nblock);
+        q1.alloc(nblock);
+        p0.alloc(nblock);
+        nc.alloc(3 * S.batches.size());
+        nc.zero(s);
+        HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, q0.p, q1.p, p0.p, S.perm.p, (int)nblock, 0, 38, s));
+        t2.alloc(std::max<size_t>(bytes, 1));
+        for (size_t b = 0; b < S.batches.size(); b++) {
+            hipLaunchKernelGGL(k_rows_len, dim3(rows_grid(nblock, 256, 2048)), dim3(256), 0, s, nblock, S.ptr.p + b * (nblock + 1), brg,
+                               bcol, q0.p, p0.p, nc.p + 3 * b);
+            HIPCHK(hipcub::DeviceRadixSort::SortPairs(t2.p, bytes, q0.p, q1.p, p0.p, S.perm.p + b * nblock, (int)nblock, 0, 38, s));
+        }
+        std::vector<unsigned long long> h(3 * S.batches.size());
+        nc.download(h.data(), h.size(), s);
+        HIPCHK(hipStreamSynchronize(s));
+        for (size_t b = 0; b < S.batches.size(); b++)
+            for (int x = 0; x < 3; x++) S.batches[b].ncls[x] = (int64_t)h[3 * b + x];
+    }
     S.unit.alloc((size_t)mu * ubytes);
     S.side.alloc((size_t)mu * 4);
     S.c.release();
@@ -1157,17 +1274,16 @@ hipError_t launch_rows_gather(const RowStruct &S, size_t batch, int32_t ngroup, 
     const auto &B = S.batches[batch];
     const uint32_t *ptr = S.ptr.p + batch * (nblock + 1);
     const uint2 *src = S.src.p + B.inc0;
-    // four slots per block, sixteen when the blocks' lists are long (few blocks)
-    const bool wide = B.npair > 64 * nblock;
-    const dim3 grid((unsigned)((nblock + (wide ? 3 : 15)) / (wide ? 4 : 16)));
+    const uint32_t *perm = S.perm.p + batch * nblock;
+#define ROWS_GS(T_, KP_, GP_, SL_, N_)                                                                                     \
+    if ((N_) > 0) {                                                                                                       \
+        hipLaunchKernelGGL((k_rows_gather<T_, KP_, GP_, SL_>), dim3((unsigned)(((N_) * 4 * SL_ + 255) / 256)), dim3(256), \
+                           0, s, N_, perm, boff, brg, bcol, gfirst, ptr, src, (const char *)S.unit.p, mat);               \
+        perm += (N_);                                                                                                     \
+    }
 #define ROWS_G(T_, KP_, GP_)                                                                                               \
     if (S.kp == KP_ && S.gp == GP_) {                                                                                     \
-        if (wide)                                                                                                         \
-            hipLaunchKernelGGL((k_rows_gather<T_, KP_, GP_, 16>), grid, dim3(256), 0, s, nblock, boff, brg, bcol, gfirst, \
-                               ptr, src, (const char *)S.unit.p, mat);                                                    \
-        else                                                                                                              \
-            hipLaunchKernelGGL((k_rows_gather<T_, KP_, GP_, 4>), grid, dim3(256), 0, s, nblock, boff, brg, bcol, gfirst,  \
-                               ptr, src, (const char *)S.unit.p, mat);                                                    \
+        ROWS_GS(T_, KP_, GP_, 16, B.ncls[0]) ROWS_GS(T_, KP_, GP_, 4, B.ncls[1]) ROWS_GS(T_, KP_, GP_, 1, B.ncls[2])      \
         hipLaunchKernelGGL((k_rows_gather_diag<T_, KP_, GP_>), dim3(ngroup), dim3(256), 0, s, ngroup, brow, boff, gfirst, \
                            ptr, src, (const char *)S.unit.p, S.side.p, mat, vec, cnt);                                    \
     }
@@ -1176,6 +1292,7 @@ hipError_t launch_rows_gather(const RowStruct &S, size_t batch, int32_t ngroup, 
     ROWS_G(T_, 6, 2) ROWS_G(T_, 6, 6) ROWS_G(T_, 6, 8)
     if (S.dbl) { ROWS_GT(double) } else { ROWS_GT(float) }
 #undef ROWS_G
+#undef ROWS_GS
 #undef ROWS_GT
     return hipGetLastError();
 }

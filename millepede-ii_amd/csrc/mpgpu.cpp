@@ -1231,7 +1231,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             else (void)hipGetLastError();
         }
         const int64_t budget = std::max<int64_t>(1 << 20, (int64_t)(gb * (1ull << 30) / 8.0));
-        rows_incidence(c->rows, c->d_group_of.p, pm, c->nblock, budget, row_upd, s);
+        rows_incidence(c->rows, c->d_group_of.p, pm, c->nblock, c->d_brg.p, c->d_bcol.p, budget, row_upd, s);
         phase("row incidence lists");
         // the other records: per record the block id of each segment pair
         if (c->ngen > 0)

@@ -333,7 +333,8 @@ void st_incidence(const StructIn &in, const DBuf<int64_t> &rec_gl, const DBuf<in
 
 // ---- records in row form (k_rows.hip) ----
 struct RowStruct {
-    struct Batch { int64_t q0, q1, unit0, nunit, inc0, npair; };
+    // ncls: off-diagonal blocks whose lists are long, medium, short (k_rows_gather)
+    struct Batch { int64_t q0, q1, unit0, nunit, inc0, npair, ncls[3]; };
     int64_t nq = 0, nrow = 0, nseg = 0, nunit = 0, npair = 0;
     int kp = 4, gp = 6, max_eq = 0;   // local and group columns of a row, most equations of a record
     bool dbl = false;
@@ -345,7 +346,7 @@ struct RowStruct {
     DBuf<uint16_t> eq_pos, seq;
     DBuf<int4> seg;
     std::vector<Batch> batches;       // matrix build: batches of records and their incidence lists
-    DBuf<uint32_t> ptr;
+    DBuf<uint32_t> ptr, perm;         // perm: order of the blocks in the gather
     DBuf<uint2> src;
     DBuf<uint8_t> unit;               // units and side array of the largest batch
     DBuf<double> side;
@@ -354,8 +355,8 @@ void rows_classify(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int
                    const int32_t *band, const RowGroups &Q, RowStruct &S, std::vector<uint8_t> &cls, hipStream_t s);
 void rows_build(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix,
                 const RowGroups &Q, const std::vector<int64_t> &order, RowStruct &S, hipStream_t s);
-void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, int64_t nblock, int64_t budget,
-                    const std::vector<int64_t> &upd, hipStream_t s);
+void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, int64_t nblock, const int32_t *brg,
+                    const int32_t *bcol, int64_t budget, const std::vector<int64_t> &upd, hipStream_t s);
 hipError_t launch_rows(const RowStruct &S, const RowDev &R, const DevModel &M, const PassOpts &o, const RecOut &out, bool build,
                        int64_t q0, int64_t q1, hipStream_t s);
 hipError_t launch_rows_gather(const RowStruct &S, size_t batch, int32_t ngroup, int64_t nblock, const int64_t *brow,
