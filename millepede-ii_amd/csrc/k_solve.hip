@@ -117,6 +117,7 @@ __global__ void k_final_sum(int n, const double *part, double *out)
 // workgroup to finish (a counter in part[DOT_CNT], zero between calls) adds the partial sums in
 // k_final_sum's order, so the result is bit-identical to the two-launch form
 #define DOT_CNT 2047
+#define SPK_CH 256     // rows of a chunk of the band solves
 __global__ __launch_bounds__(TPB) void k_dot_fused(int64_t n, const double *a, const double *b, double *part, double *out)
 {
     __shared__ double s[TPB];
@@ -1056,7 +1057,7 @@ __global__ __launch_bounds__(256) void k_bsymv_cols(int32_t ngroup, const int64_
 }
 
 // constraint rows (Lagrange multipliers) in CSR over variable indices:
-// y[nvar+j] += sum c_ji x_i ; y_i += c_ji x[nvar+j]
+// y[nvar+j] = sum c_ji x_i ; y_i += c_ji x[nvar+j]
 __global__ void k_cons_symv(int32_t ncon, int32_t nvar, const int64_t *cptr, const int32_t *cidx,
                             const double *cval, const double *x, double *y)
 {
@@ -1077,7 +1078,7 @@ __global__ void k_cons_symv(int32_t ncon, int32_t nvar, const int64_t *cptr, con
         if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(&y[nvar + j], s[0]);
+    if (threadIdx.x == 0) y[nvar + j] = s[0];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1094,19 +1095,11 @@ __global__ void k_mr_scale(int64_t n, const MrState *st, const double *y, double
     const double sc = 1.0 / st->beta;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) v[i] = sc * y[i];
 }
-// y -= (beta/oldb) r (which = 0) or y -= (alfa/beta) r (which = 1)
-__global__ void k_mr_axpy(int64_t n, const MrState *st, int which, const double *r, double *y)
-{
-    if (st->istop != 0) return;
-    const double c = which == 0 ? st->beta / st->oldb : st->alfa / st->beta;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) y[i] = y[i] - c * r[i];
-}
 // one step of the scalar recurrence (src/minresModule.f90:468-600), the host restatement's
 // operations in the same order, without contraction into fused multiply-adds
-__global__ void k_mr_step(MrState *st)
+__device__ void mr_step(MrState *st)
 {
 #pragma clang fp contract(off)
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (st->istop != 0) { st->upd = 0; return; }
     const double eps = 2.220446049250313e-16;
     const int itn = ++st->itn;
@@ -1183,19 +1176,115 @@ __global__ void k_mr_step(MrState *st)
     st->Acond = Acond;
     st->istop = istop;
 }
-// w1 = w2; w2 = w; w = (v - oldeps*w1 - delta*w2)*denom; x = x + phi*w  (iterations that ran)
-__global__ void k_mr_update(int64_t n, const MrState *st, const double *v, double *w, double *w1, double *w2, double *x)
+// Sum over all workgroups of one value per thread, in the order of k_dot_fused (partial sums per
+// workgroup, the last workgroup adds them); true in thread 0 of the last workgroup, which has the
+// sum.  part: partial sums and the counter, as k_dot_fused's.
+__device__ bool last_sum(double acc, double *part, double &sum)
+{
+    __shared__ double s[TPB];
+    __shared__ int last;
+    s[threadIdx.x] = acc;
+    __syncthreads();
+    for (int o = TPB / 2; o > 0; o >>= 1) {
+        if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+        __syncthreads();
+    }
+    unsigned int *cnt = (unsigned int *)(part + DOT_CNT);
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&part[blockIdx.x], s[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned int done = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        last = done == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return false;
+    double acc2 = 0.0;
+    for (int i = threadIdx.x; i < (int)gridDim.x; i += TPB)
+        acc2 += __hip_atomic_load(&part[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s[threadIdx.x] = acc2;
+    __syncthreads();
+    for (int o = TPB / 2; o > 0; o >>= 1) {
+        if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return false;
+    sum = s[0];
+    __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// An iteration of MINRES around the product and the preconditioner, in four launches (it was eight
+// kernels of 2-5 us each, at or below the time of a launch):
+// after the product: y -= (beta/oldb) r1 (from the second iteration on), alfa = v . y
+__global__ __launch_bounds__(TPB) void k_mr_mid(int64_t n, MrState *st, int first, const double *v, const double *r1, double *y,
+                                                double *part)
+{
+    if (st->istop != 0) return;
+    const double c = first ? 0.0 : st->beta / st->oldb;
+    double acc = 0.0;
+    for (int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
+        double t = y[i];
+        if (!first) {
+            t = t - c * r1[i];
+            y[i] = t;
+        }
+        acc += v[i] * t;
+    }
+    double sum;
+    if (last_sum(acc, part, sum)) st->alfa = sum;
+}
+// r1 <- y - (alfa/beta) r2 (the new r2 in r1's place: the caller swaps them); keep: y holds it too
+__global__ void k_mr_sub(int64_t n, const MrState *st, const double *r2, double *r1, double *y, int keep)
+{
+    if (st->istop != 0) return;
+    const double c = st->alfa / st->beta;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const double t = y[i] - c * r2[i];
+        r1[i] = t;
+        if (keep) y[i] = t;
+    }
+}
+// end of the preconditioner and the scalar recurrence: W > 0: y_i += sum_q Cb_iq t_q (the backward
+// correction of the band solve, rows i < nb of chunks of `ch` rows but the last); beta^2 = r2 . y,
+// then one step of the recurrence
+template <int W>
+__global__ __launch_bounds__(TPB) void k_mr_end(int64_t n, MrState *st, const double *r2, double *y, int nb, int ch,
+                                                const double *Cb, const double *t, double *part)
+{
+    if (st->istop != 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->upd = 0;
+        return;
+    }
+    double acc = 0.0;
+    const int nfix = W > 0 ? (nb - 1) / ch * ch : 0;
+    for (int64_t i = blockIdx.x * (int64_t)TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
+        double v = y[i];
+        if (W > 0 && i < nfix) {
+#pragma unroll
+            for (int q = 0; q < W; q++) v += Cb[i * W + q] * t[i / ch * W + q];
+            y[i] = v;
+        }
+        acc += r2[i] * v;
+    }
+    double sum;
+    if (last_sum(acc, part, sum)) {
+        st->bnew = sum;
+        mr_step(st);
+    }
+}
+// w1 = w2; w2 = w; w = (v - oldeps*w1 - delta*w2)*denom; x = x + phi*w  (iterations that ran), then
+// the next iteration's v = y / beta
+__global__ void k_mr_next(int64_t n, const MrState *st, const double *y, double *v, double *w, double *w2, double *x)
 {
     if (st->upd == 0) return;
-    const double oldeps = st->oldeps, delta = st->delta, denom = st->denom, phi = st->phi;
+    const double oldeps = st->oldeps, delta = st->delta, denom = st->denom, phi = st->phi, sc = 1.0 / st->beta;
+    const bool on = st->istop == 0;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        double a1 = w2[i];
-        double a2 = w[i];
-        w1[i] = a1;
+        const double a1 = w2[i], a2 = w[i];
         w2[i] = a2;
-        double wn = (v[i] - oldeps * a1 - delta * a2) * denom;
+        const double wn = (v[i] - oldeps * a1 - delta * a2) * denom;
         w[i] = wn;
         x[i] = x[i] + phi * wn;
+        if (on) v[i] = sc * y[i];
     }
 }
 
@@ -2038,8 +2127,9 @@ void l_block_symv(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const
                   const double *x, double *y, int32_t nvar, int64_t nall, int32_t maxgrp, const int32_t *cc_blk,
                   double *tb, int32_t ugrp, const int32_t *bcol, int64_t nblock, int variant, hipStream_t s)
 {
-    // rows beyond the parameter groups (Lagrange multipliers) start at zero
-    if (nall > nvar) hipLaunchKernelGGL(k_zero, dim3(nblk(nall - nvar)), dim3(TPB), 0, s, nall - nvar, y + nvar);
+    // rows beyond the parameter groups (Lagrange multipliers) are written by k_cons_symv
+    (void)nall;
+    (void)nvar;
     if (maxgrp <= 8 && tb && cc_blk) {
         // the matrix is read once: rows pass with the transposed block products (tbw values per
         // block), then their sums over the column lists
@@ -2084,11 +2174,30 @@ void l_scale_copy(int64_t n, double sc, const double *a, double *o, hipStream_t 
 { hipLaunchKernelGGL(k_scale_copy, dim3(nblk(n)), dim3(TPB), 0, s, n, sc, a, o); }
 void l_mr_scale(int64_t n, const MrState *st, const double *y, double *v, hipStream_t s)
 { hipLaunchKernelGGL(k_mr_scale, dim3(nblk(n)), dim3(TPB), 0, s, n, st, y, v); }
-void l_mr_axpy(int64_t n, const MrState *st, int which, const double *r, double *y, hipStream_t s)
-{ hipLaunchKernelGGL(k_mr_axpy, dim3(nblk(n)), dim3(TPB), 0, s, n, st, which, r, y); }
-void l_mr_step(MrState *st, hipStream_t s) { hipLaunchKernelGGL(k_mr_step, dim3(1), dim3(64), 0, s, st); }
-void l_mr_update(int64_t n, const MrState *st, const double *v, double *w, double *w1, double *w2, double *x, hipStream_t s)
-{ hipLaunchKernelGGL(k_mr_update, dim3(nblk(n)), dim3(TPB), 0, s, n, st, v, w, w1, w2, x); }
+static int dot_blocks(int64_t n) { return (int)std::min<int64_t>(1024, std::max<int64_t>(1, (n + TPB - 1) / TPB)); }
+void l_mr_mid(int64_t n, MrState *st, int first, const double *v, const double *r1, double *y, double *part, hipStream_t s)
+{ hipLaunchKernelGGL(k_mr_mid, dim3(dot_blocks(n)), dim3(TPB), 0, s, n, st, first, v, r1, y, part); }
+void l_mr_sub(int64_t n, const MrState *st, const double *r2, double *r1, double *y, int keep, hipStream_t s)
+{ hipLaunchKernelGGL(k_mr_sub, dim3(nblk(n)), dim3(TPB), 0, s, n, st, r2, r1, y, keep); }
+void l_mr_end(int64_t n, MrState *st, const double *r2, double *y, int w, int nb, const double *Cb, const double *t, double *part,
+              hipStream_t s)
+{
+#define MR_END(W) hipLaunchKernelGGL(k_mr_end<W>, dim3(dot_blocks(n)), dim3(TPB), 0, s, n, st, r2, y, nb, SPK_CH, Cb, t, part)
+    switch (w) {
+    case 0: MR_END(0); break;
+    case 1: MR_END(1); break;
+    case 2: MR_END(2); break;
+    case 3: MR_END(3); break;
+    case 4: MR_END(4); break;
+    case 5: MR_END(5); break;
+    case 6: MR_END(6); break;
+    case 7: MR_END(7); break;
+    default: MR_END(8); break;
+    }
+#undef MR_END
+}
+void l_mr_next(int64_t n, const MrState *st, const double *y, double *v, double *w, double *w2, double *x, hipStream_t s)
+{ hipLaunchKernelGGL(k_mr_next, dim3(nblk(n)), dim3(TPB), 0, s, n, st, y, v, w, w2, x); }
 void l_axpy_neg(int64_t n, double c, const double *r, double *y, hipStream_t s)
 { hipLaunchKernelGGL(k_axpy_neg, dim3(nblk(n)), dim3(TPB), 0, s, n, c, r, y); }
 void l_minres_update(int64_t n, const double *v, double *w, double *w1, double *w2, double *x, double oldeps, double delta,
@@ -2298,7 +2407,6 @@ void l_equslvs(int n, int m, const double *c, const int *india, const int *cb, c
 // Layout: row k (1-based) of the factor holds columns k-len+1..k at c[india(k)-k+j-1],
 // len = india(k)-india(k-1) (india(0)=0).
 // ---------------------------------------------------------------------------------------------
-#define SPK_CH 256
 #define SPK_WMAX 16
 
 __device__ __forceinline__ int spk_len(const int *india, int k) { return india[k - 1] - (k > 1 ? india[k - 2] : 0); }
@@ -2877,6 +2985,9 @@ static void spk_scan(int n, int w, int nch, const double *x, const double *A, in
     }
 #undef SPK_SCAN
 }
+
+void l_spk_scan(int n, int w, const double *x, const double *A, int nlev, double *t, int backward, hipStream_t s)
+{ spk_scan(n, w, (n + SPK_CH - 1) / SPK_CH, x, A, nlev, t, backward, s); }
 
 void l_equslvs_spike(int n, int m, int w, const double *c, const int *india, const double *Sf, const double *Sb,
                      double *tbuf, const int *cb, const int64_t *koff, const double *kmat, const double *h, const int *hind,

@@ -1794,11 +1794,9 @@ void op_dev(mpgpu_ctx *c, ElimWork &E, const double *x, double *y)
     if (!c->elim) { avprod_dev(c, x, y); return; }
     hipStream_t s = c->stream;
     const int32_t nv = c->nvar, nf = c->nfit;
-    l_ql_pad(nf, nv, x, E.e.p, s);
-    l_ql_apply(c->ql->dev, 0, E.e.p, s);
+    l_ql_op(c->ql->dev, 0, nf, x, E.e.p, nv, s);
     avprod_dev(c, E.e.p, E.f.p);
-    l_ql_apply(c->ql->dev, 1, E.f.p, s);
-    l_copy(nf, E.f.p, y, s);
+    l_ql_op(c->ql->dev, 1, nv, E.f.p, y, nf, s);
 }
 
 double dot_dev(mpgpu_ctx *c, int64_t n, const double *a, const double *b)
@@ -1814,10 +1812,16 @@ double dot_dev(mpgpu_ctx *c, int64_t n, const double *a, const double *b)
 struct Precond {
     int kind = 0; // 0 none, 1 diagonal (+constraints), 2 band (+constraints)
     DBuf<double> cu, sm, scratch, band, kmat, h, Sf, Sb, tbuf, dtmp, Af, Ab;   // Af/Ab: scan levels of the carry
+    DBuf<double> F, B, Tf, Tb, hinv;      // sub-chunk form (k_bandpc.hip); Sf, Sb: responses to a chunk's boundary
     DBuf<int> nrkd, india, hind, cb;
     DBuf<int64_t> koff;
     int n = 0, m = 0, w = 0, nlev = 0;
     bool spike = false;
+    bool sub = false;     // applied by l_bp_apply
+    BandPc bp() const
+    {
+        return BandPc{F.p, B.p, Tf.p, Tb.p, Sf.p, Sb.p, Af.p, Ab.p, hinv.p, kmat.p, cb.p, koff.p, tbuf.p, dtmp.p, nlev};
+    }
 };
 
 // With eliminated constraints the preconditioner is built from pede's band of Q^T A Q (qlpssq,
@@ -1940,9 +1944,19 @@ void setup_precond(mpgpu_ctx *c, Precond &P)
         P.Sb.alloc((size_t)P.n * P.w);
         P.tbuf.alloc((size_t)nch * P.w);
         P.dtmp.alloc(std::max(1, P.m));
-        DBuf<double> scr;
-        scr.alloc((size_t)nch * P.w * ch);
-        l_spk_build(P.n, P.w, P.band.p, P.india.p, P.Sf.p, P.Sb.p, scr.p, s);
+        P.sub = bp_usable(P.n, P.m, P.w);
+        if (P.sub) {
+            P.F.alloc((size_t)bp_sub_elems(P.n));
+            P.B.alloc((size_t)bp_sub_elems(P.n));
+            P.Tf.alloc((size_t)P.n * P.w);
+            P.Tb.alloc((size_t)P.n * P.w);
+            P.hinv.alloc((size_t)std::max(1, P.m * P.m));
+            l_bp_build(P.n, P.m, P.w, P.band.p, P.india.p, P.h.p, P.F.p, P.B.p, P.Tf.p, P.Tb.p, P.Sf.p, P.Sb.p, P.hinv.p, s);
+        } else {
+            DBuf<double> scr;
+            scr.alloc((size_t)nch * P.w * ch);
+            l_spk_build(P.n, P.w, P.band.p, P.india.p, P.Sf.p, P.Sb.p, scr.p, s);
+        }
         P.nlev = spk_scan_levels(P.n, P.w);
         if (P.nlev > 0) {
             const size_t lv = (size_t)nch * P.w * P.w * P.nlev;
@@ -1960,6 +1974,9 @@ void apply_precond(mpgpu_ctx *c, Precond &P, const double *x, double *y)
     hipStream_t s = c->stream;
     if (P.kind == 1) {
         l_presols(P.n, P.m, P.cu.p, c->d_cptr.p, c->d_cidx.p, c->d_cval.p, P.sm.p, x, y, s);
+    } else if (P.kind == 2 && P.sub) {
+        l_bp_apply(P.n, P.m, P.w, x, y, P.bp(), s);
+        l_bp_fix(P.n, P.w, y, P.bp(), s);
     } else if (P.kind == 2) {
         l_copy(P.n + P.m, x, y, s);
         if (P.spike)
@@ -1995,8 +2012,8 @@ void minres_dev(mpgpu_ctx *c, const double *b_dev, double *x_dev, mpgpu_solve_st
     if (c->elim) { E.e.alloc(c->nvar); E.f.alloc(c->nvar); }
     Precond &P = cached_precond(c);
     const bool precon = P.kind != 0;
-    DBuf<double> r1, r2, v, w, w1, w2, y;
-    r1.alloc(n); r2.alloc(n); v.alloc(n); w.alloc(n); w1.alloc(n); w2.alloc(n); y.alloc(n);
+    DBuf<double> r1, r2, v, w, w2, y;
+    r1.alloc(n); r2.alloc(n); v.alloc(n); w.alloc(n); w2.alloc(n); y.alloc(n);
     const double rtol = c->opt.mrestl;
     const int itnlim = c->opt.itnlim;
     int istop = 0, itn = 0;
@@ -2037,18 +2054,18 @@ void minres_dev(mpgpu_ctx *c, const double *b_dev, double *x_dev, mpgpu_solve_st
         w.zero(s);
         w2.zero(s);
         l_copy(n, r1.p, r2.p, s);
+        // v of the first iteration; each iteration ends with the next one's
+        l_mr_scale(n, d, y.p, v.p, s);
         auto iteration = [&](int k) {
-            l_mr_scale(n, d, y.p, v.p, s);
             op_dev(c, E, v.p, y.p);
-            if (k >= 2) l_mr_axpy(n, d, 0, r1.p, y.p, s);
-            l_dot(n, v.p, y.p, c->d_part.p, &d->alfa, s);
-            l_mr_axpy(n, d, 1, r2.p, y.p, s);
-            std::swap(r1.p, r2.p);          // r1 = r2 (old r2 buffer becomes r1)
-            l_copy(n, y.p, r2.p, s);        // r2 = y
-            if (precon) apply_precond(c, P, r2.p, y.p);
-            l_dot(n, r2.p, y.p, c->d_part.p, &d->bnew, s);
-            l_mr_step(d, s);
-            l_mr_update(n, d, v.p, w.p, w1.p, w2.p, x_dev, s);
+            l_mr_mid(n, d, k < 2, v.p, r1.p, y.p, c->d_part.p, s);
+            l_mr_sub(n, d, r2.p, r1.p, y.p, !precon, s);
+            std::swap(r1.p, r2.p);          // r1: the old r2, r2: the new one
+            const bool sub = P.kind == 2 && P.sub;
+            if (sub) l_bp_apply(P.n, P.m, P.w, r2.p, y.p, P.bp(), s);
+            else if (precon) apply_precond(c, P, r2.p, y.p);
+            l_mr_end(n, d, r2.p, y.p, sub ? P.w : 0, P.n, P.Sb.p, P.tbuf.p, c->d_part.p, s);
+            l_mr_next(n, d, y.p, v.p, w.p, w2.p, x_dev, s);
         };
         auto stopped = [&]() {
             dst.download(&h, 1, s);

@@ -144,9 +144,11 @@ int64_t packed_symv_scratch(int n);
 hipError_t noalloc_packed_symv(int device, int n, const double *a, const double *x, double *y, hipStream_t s);
 int noalloc_max_n();
 void l_mr_scale(int64_t n, const MrState *st, const double *y, double *v, hipStream_t s);
-void l_mr_axpy(int64_t n, const MrState *st, int which, const double *r, double *y, hipStream_t s);
-void l_mr_step(MrState *st, hipStream_t s);
-void l_mr_update(int64_t n, const MrState *st, const double *v, double *w, double *w1, double *w2, double *x, hipStream_t s);
+void l_mr_mid(int64_t n, MrState *st, int first, const double *v, const double *r1, double *y, double *part, hipStream_t s);
+void l_mr_sub(int64_t n, const MrState *st, const double *r2, double *r1, double *y, int keep, hipStream_t s);
+void l_mr_end(int64_t n, MrState *st, const double *r2, double *y, int w, int nb, const double *Cb, const double *t, double *part,
+              hipStream_t s);
+void l_mr_next(int64_t n, const MrState *st, const double *y, double *v, double *w, double *w2, double *x, hipStream_t s);
 void l_block_symv(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const int64_t *boff, const int32_t *gfirst,
                   const int64_t *ccol_ptr, const int64_t *cc_off, const int32_t *cc_fn, const double *a,
                   const double *x, double *y, int32_t nvar, int64_t nall, int32_t maxgrp, const int32_t *cc_blk,
@@ -191,6 +193,24 @@ void l_equslvs_spike(int n, int m, int w, const double *c, const int *india, con
 int spk_chunk_rows();   // rows per chunk of the chunk-parallel band solves
 int spk_scan_levels(int n, int w);
 void l_spk_scan_build(int n, int w, const double *Sf, const double *Sb, double *Af, double *Ab, int nlev, hipStream_t s);
+
+void l_spk_scan(int n, int w, const double *x, const double *A, int nlev, double *t, int backward, hipStream_t s);
+// application of the band preconditioner (k_bandpc.hip): sub-chunk inverses, responses of the rows
+// to the boundaries of their sub-chunk (S) and chunk (C), scan levels (A), carried boundary values
+// (t), inverse of the constraint block and its right-hand side
+struct BandPc {
+    const double *F, *B, *Sf, *Sb, *Cf, *Cb, *Af, *Ab, *hinv, *kmat;
+    const int *cb;
+    const int64_t *koff;
+    double *t, *d;
+    int nlev;
+};
+bool bp_usable(int n, int m, int w);
+int64_t bp_sub_elems(int n);
+void l_bp_build(int n, int m, int w, const double *c, const int *india, const double *h, double *F, double *B, double *Sf,
+                double *Sb, double *Cf, double *Cb, double *hinv, hipStream_t s);
+void l_bp_apply(int n, int m, int w, const double *x, double *y, const BandPc &P, hipStream_t s);
+void l_bp_fix(int n, int w, double *y, const BandPc &P, hipStream_t s);
 
 // dense LDL^T (k_chol.hip): full column-major n x n matrix (lda = n), lower triangle.  The
 // factor keeps the raw pivots on the diagonal, w_i = 1/d_i (d_i > 0) or d_i in w, and needs
@@ -403,6 +423,7 @@ struct QlElim {
     void wy();
 };
 void l_ql_apply(const QlDev &q, int trans, double *x, hipStream_t s);   // x <- Q x (0) or Q^T x (1)
+void l_ql_op(const QlDev &q, int trans, int32_t nx, const double *x, double *y, int32_t ny, hipStream_t s);
 void l_ql_pad(int32_t nfit, int32_t n, const double *x, double *e, hipStream_t s);
 void l_ql_vtx_cols(const QlDev &q, const double *x, int64_t ldx, int32_t ncols, double *w, int64_t ldw, hipStream_t s);
 void l_ql_vdense(const QlDev &q, double *Vd, hipStream_t s);
