@@ -887,6 +887,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 void k_rows_gather(int64_t nblock /* of this class */, const uint32_t *perm, const int64_t *boff, const int32_t *brg, const int32_t *bcol,
                    const int32_t *gfirst, const uint32_t *ptr, const uint2 *src, const char *unit, double *mat)
 {
+    // boff null: packed triangle
     constexpr int HM = GP / 2;
     const int lane = threadIdx.x & 63;
     const int64_t p = (xcd_run(blockIdx.x, gridDim.x, 64) * 256 + threadIdx.x) / (4 * SL);
@@ -933,7 +934,8 @@ void k_rows_gather(int64_t nblock /* of this class */, const uint32_t *perm, con
         i += SL;
     }
     const int nr = gfirst[ga + 1] - gfirst[ga], nc = gfirst[gb + 1] - gfirst[gb];
-    double *Bk = mat + (p < nblock ? boff[k] : 0);
+    const int64_t va = gfirst[ga], vb = gfirst[gb];
+    const int64_t m0 = p < nblock && boff ? boff[k] : 0;
 #pragma unroll
     for (int x = 0; x < HM; x++)
 #pragma unroll
@@ -948,7 +950,10 @@ void k_rows_gather(int64_t nblock /* of this class */, const uint32_t *perm, con
                 v += __shfl_xor(v, 32, WV);
             }
             const int rr = hi * HM + x, cc = lo * HM + y;
-            if (i1 > i0 && slot == ((x * HM + y) & (SL - 1)) && rr < nr && cc < nc) Bk[rr * nc + cc] -= v;
+            if (i1 > i0 && slot == ((x * HM + y) & (SL - 1)) && rr < nr && cc < nc) {
+                const int64_t i = va + rr;
+                mat[boff ? m0 + rr * nc + cc : (i * i - i) / 2 + vb - 1 + cc] -= v;
+            }
         }
 }
 
@@ -1030,7 +1035,8 @@ __global__ __launch_bounds__(256) void k_rows_gather_diag(int32_t ngroup, const 
     if (t < na * na) {
         const int r = t / na, q = t - r * na;
         const int e = r * GP + q;
-        if (q <= r) mat[boff[k] + t] += (s_m[0][e] + s_m[1][e]) + (s_m[2][e] + s_m[3][e]);
+        const int64_t v = gfirst[g], i = v + r;
+        if (q <= r) mat[boff ? boff[k] + t : (i * i - i) / 2 + v - 1 + q] += (s_m[0][e] + s_m[1][e]) + (s_m[2][e] + s_m[3][e]);
     } else if (t >= 128 && t < 128 + na) {
         const int e = t - 128;
         vec[gfirst[g] - 1 + e] += (s_v[0][e] + s_v[1][e]) + (s_v[2][e] + s_v[3][e]);

@@ -984,8 +984,11 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     PairMap pm;
     int32_t max_ngl_all = 1;
     for (int32_t x : ngl_rec) max_ngl_all = std::max(max_ngl_all, x);
-    st_record_stats(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, c->ngroup, max_ngl_all, sparse,
-                    pm, rst, cnt_r, d_rst, s);
+    // the pairs of groups that records couple: the blocks of group-block storage, and with full
+    // storage those that the records in row form are gathered by (a bitmap of up to 256 MB)
+    const bool try_rows = c->opt.monitor == 0 && nrec > 0 && (sparse || c->ngroup <= 65536);
+    st_record_stats(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, c->ngroup, max_ngl_all,
+                    sparse || try_rows, pm, rst, cnt_r, d_rst, s);
     const int32_t *st_nv = rst.data(), *st_nseg = rst.data() + nrec, *st_nalc = rst.data() + 2 * nrec,
                   *st_sup = rst.data() + 3 * nrec, *st_qe = rst.data() + 4 * nrec;
     phase("record stats and group pairs");
@@ -1154,7 +1157,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     if (c->nband > 0) c->d_band_info.upload(binfo, s);
     c->ngen = nrec;
     std::vector<int64_t> row_upd;      // update sizes of the records in row form, when a batch size is set
-    if (sparse && c->opt.monitor == 0) {
+    if (try_rows) {
         std::vector<int32_t> tg_of(ntot), tg_t0, tg_v0;
         std::vector<uint32_t> tg_mask;
         for (int32_t t = 0; t < ntot; t++) {
@@ -1200,8 +1203,20 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         for (int64_t q = 0; q < nrec; q++) (cls[order[q]] ? fast : gen).push_back(order[q]);
         if (std::getenv("MPGPU_UPDATE_BUFFER_GB"))
             for (int64_t r : fast) row_upd.push_back(cnt_r[r]);
-        for (int64_t r : fast) cnt_r[r] = 0;
         rows_build(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, Q, fast, c->rows, s);
+        if (!sparse && c->rows.nq > 0) {
+            // the lists of a dense matrix are long: without room for them the record kernel's
+            // atomic additions remain
+            size_t fr = 0, tot = 0;
+            const bool room = hipMemGetInfo(&fr, &tot) != hipSuccess || c->rows.list_bytes() < (int64_t)(fr / 2);
+            (void)hipGetLastError();
+            if (!room) {
+                c->rows.drop();
+                fast.clear();
+                gen = order;
+            }
+        }
+        for (int64_t r : fast) cnt_r[r] = 0;
         c->ngen = (int64_t)gen.size();
         c->d_order.upload(gen, s);
         HIPCHK(hipStreamSynchronize(s));     // the tables above end here
@@ -1294,6 +1309,18 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         c->d_cbuf.release();
         c->d_rec_pb.release();
         c->d_pair_blk.release();
+    }
+    if (!sparse && c->rows.nq > 0) {
+        st_blocks(pm, c->ngroup, c->d_gfirst.p, {}, blk, s);
+        c->rows.nblock = blk.nblock;
+        c->rows.brow.swap(blk.brow);
+        c->rows.brg.swap(blk.brg);
+        c->rows.bcol.swap(blk.bcol);
+        size_t fr = 0, tot = 0;
+        int64_t budget = (int64_t)1 << 33;
+        if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr > 0) budget = (int64_t)(0.45 * (double)fr) / 8;
+        else (void)hipGetLastError();
+        rows_incidence(c->rows, c->d_group_of.p, pm, blk.nblock, c->rows.brg.p, c->rows.bcol.p, budget, {}, s);
     }
     phase("two-phase index");
     // ---- remaining device state ----
@@ -1560,8 +1587,12 @@ extern "C" int mpgpu_loopn(mpgpu_ctx *c, int32_t icalcm, int32_t nloopn, float c
             if (!build) break;
             auto tg = timed(t_gat);
             HIPCHK(hipEventRecord(tg.first, s));
-            HIPCHK(launch_rows_gather(S, bt, c->ngroup, c->nblock, c->d_brow.p, c->d_boff.p, c->d_brg.p, c->d_bcol.p,
-                                      c->d_gfirst.p, c->d_mat.p, c->d_vec.p, c->d_cnt.p, s));
+            if (c->opt.matsto == MPGPU_SPARSE)
+                HIPCHK(launch_rows_gather(S, bt, c->ngroup, c->nblock, c->d_brow.p, c->d_boff.p, c->d_brg.p, c->d_bcol.p,
+                                          c->d_gfirst.p, c->d_mat.p, c->d_vec.p, c->d_cnt.p, s));
+            else
+                HIPCHK(launch_rows_gather(S, bt, c->ngroup, S.nblock, S.brow.p, nullptr, S.brg.p, S.bcol.p, c->d_gfirst.p,
+                                          c->d_mat.p, c->d_vec.p, c->d_cnt.p, s));
             HIPCHK(hipEventRecord(tg.second, s));
         }
     }

@@ -2,6 +2,7 @@
 #pragma once
 #include "mpgpu_device.h"
 #include "../../include/mpgpu.h"
+#include <algorithm>
 #include <string>
 #include <vector>
 #include <cstring>
@@ -370,6 +371,17 @@ struct RowStruct {
     DBuf<uint2> src;
     DBuf<uint8_t> unit;               // units and side array of the largest batch
     DBuf<double> side;
+    int64_t nblock = 0;               // full storage: the pairs of groups that some record couples
+    DBuf<int64_t> brow;
+    DBuf<int32_t> brg, bcol;
+    // device bytes of the incidence lists, with what their sort needs beside them
+    void drop()
+    {
+        nq = 0;
+        order.release(); c.release(); hdr.release(); rows.release(); eq_t0.release(); ptix.release(); eq_pos.release();
+        seq.release(); seg.release();
+    }
+    int64_t list_bytes() const { return 8 * npair + 24 * std::min<int64_t>(npair, (int64_t)1 << 30); }
 };
 void rows_classify(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix,
                    const int32_t *band, const RowGroups &Q, RowStruct &S, std::vector<uint8_t> &cls, hipStream_t s);

@@ -1,4 +1,4 @@
-"""Records in row form (group-block storage: equations that each touch one group of at most 8
+"""Records in row form (equations that each touch one group of at most 8
 parameters, at most 5 local parameters, 128 equations, 4 equations per group) against the oracle,
 at the edges of what has that form and just beyond, where the other record kernel takes over:
 equations per wavefront (64, 66, 128, 130), group sizes, local parameters, equations per group
@@ -55,13 +55,14 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("matsto", [mpgpu.SPARSE, mpgpu.FULL])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x) for x in c[:6]))
-def test_row_form_pass(orc, case):
+def test_row_form_pass(orc, case, matsto):
     nmod, gsize, nloc, nrec, hits, per_hit, dtype = case
     rp, ii, gg = _records(sum(case[:6]), nmod, gsize, nloc, nrec, hits, per_hit, dtype)
     # a parameter inside every third group is fixed at a start value
     fixed = [100 * (m + 1) + gsize // 2 + 1 for m in range(0, nmod, 3)] if gsize > 1 else []
-    P = mpgpu.Pede(matsto=mpgpu.SPARSE, metsol=mpgpu.MINRES, mreqenf=1, mcount=1, lhuber=3, lfitbb=0)
+    P = mpgpu.Pede(matsto=matsto, metsol=mpgpu.MINRES, mreqenf=1, mcount=1, lhuber=3, lfitbb=0)
     P.add_records(rp, ii, gg)
     if fixed:
         P.set_steering_parameters(fixed, 0.05 * np.ones(len(fixed)), -np.ones(len(fixed)))
