@@ -1011,7 +1011,7 @@ void st_record_stats(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<i
 }
 
 void st_blocks(PairMap &pm, int32_t ngroup, const int32_t *gfirst, const std::vector<int64_t> &extra_pairs, BlockDev &B,
-               hipStream_t s)
+               bool storage, hipStream_t s)
 {
     DBuf<uint8_t> tmp;
     const int64_t ng = ngroup;
@@ -1043,6 +1043,7 @@ void st_blocks(PairMap &pm, int32_t ngroup, const int32_t *gfirst, const std::ve
                        B.brow.p);
     hipLaunchKernelGGL(k_blocks, dim3(grid_for(pm.nw, 256)), dim3(256), 0, s, pm.nw, pm.bits.p, pm.wrank.p, gfirst,
                        B.brg.p, B.bcol.p, bsz.p, B.bcf.p);
+    if (!storage) return;               // only the pairs are wanted
     hipLaunchKernelGGL(k_tail_zero, dim3(1), dim3(1), 0, s, bsz.p + nb);
     scan_excl(bsz.p, B.boff.p, nb + 1, s, tmp);
     HIPCHK(hipMemcpyAsync(&B.nstored, B.boff.p + nb, sizeof(int64_t), hipMemcpyDeviceToHost, s));

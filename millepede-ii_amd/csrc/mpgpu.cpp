@@ -1,6 +1,7 @@
 // libmpgpu host side: context, record compilation, structure build (loop1/loop2
 // equivalents), data passes (loopn) and the global solve dispatch (xloopn's metsol switch).
 #include "mpgpu_internal.h"
+#include <mutex>
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -57,6 +58,7 @@ struct mpgpu_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = true;       // false: a stream the caller keeps (serving workers)
+    DevCache *cache = nullptr;    // outlives the buffers below (mpgpu_destroy)
     std::string err;
 
     // ---- input records: record pointers on the host; words and values go to the device as
@@ -169,13 +171,115 @@ struct mpgpu_ctx {
     std::vector<unsigned long long> last_cnt;
 };
 
+// ---- device memory (DevCache) ----
+namespace {
+constexpr size_t CACHE_BLOCK = (size_t)256 << 20, CACHE_CONTEXT = (size_t)2 << 30, CACHE_STORE = (size_t)4 << 30;
+struct DevStore {
+    std::mutex m;
+    std::unordered_map<size_t, std::vector<void *>> free;   // key: size class, device in the low byte
+    size_t held = 0;
+};
+DevStore &dev_store()
+{
+    static DevStore *st = new DevStore;      // never destroyed: contexts may end after static objects
+    return *st;
+}
+// sizes are rounded up to an eighth of their power of two (at least 256 bytes)
+size_t size_class(size_t b)
+{
+    size_t q = 256;
+    while (q * 16 <= b) q *= 2;
+    return (b + q - 1) / q * q;
+}
+void *store_take(size_t key)
+{
+    DevStore &S = dev_store();
+    std::lock_guard<std::mutex> g(S.m);
+    auto it = S.free.find(key);
+    if (it == S.free.end() || it->second.empty()) return nullptr;
+    void *p = it->second.back();
+    it->second.pop_back();
+    S.held -= key & ~(size_t)255;
+    return p;
+}
+} // namespace
+
+void DevCache::drop()
+{
+    for (auto &f : free_)
+        for (void *p : f.second) (void)hipFreeAsync(p, s);
+    free_.clear();
+    held = 0;
+}
+void *DevCache::get(size_t bytes)
+{
+    const size_t c = size_class(bytes);
+    if (c <= CACHE_BLOCK) {
+        auto it = free_.find(c);
+        if (it != free_.end() && !it->second.empty()) {
+            void *p = it->second.back();
+            it->second.pop_back();
+            held -= c;
+            return p;
+        }
+        if (void *p = store_take(c | (size_t)device)) return p;
+    }
+    void *p = nullptr;
+    hipError_t e = hipMallocAsync(&p, c, s);
+    if (e != hipSuccess) {
+        // give the free blocks back and try once more
+        (void)hipGetLastError();
+        drop();
+        std::vector<void *> blocks;
+        {
+            DevStore &S = dev_store();
+            std::lock_guard<std::mutex> g(S.m);
+            for (auto &f : S.free)
+                if ((int)(f.first & 255) == device) {
+                    blocks.insert(blocks.end(), f.second.begin(), f.second.end());
+                    S.held -= (f.first & ~(size_t)255) * f.second.size();
+                    f.second.clear();
+                }
+        }
+        for (void *q : blocks) (void)hipFreeAsync(q, s);
+        (void)hipStreamSynchronize(s);
+        HIPCHK(hipMallocAsync(&p, c, s));
+    }
+    return p;
+}
+void DevCache::put(void *p, size_t bytes)
+{
+    const size_t c = size_class(bytes);
+    if (c > CACHE_BLOCK || held + c > CACHE_CONTEXT) {
+        (void)hipFreeAsync(p, s);
+        return;
+    }
+    free_[c].push_back(p);
+    held += c;
+}
+DevCache::~DevCache()
+{
+    DevStore &S = dev_store();
+    std::vector<void *> over;
+    {
+        std::lock_guard<std::mutex> g(S.m);
+        for (auto &f : free_)
+            for (void *p : f.second) {
+                if (S.held + f.first > CACHE_STORE) { over.push_back(p); continue; }
+                S.free[f.first | (size_t)device].push_back(p);
+                S.held += f.first;
+            }
+    }
+    for (void *p : over) (void)hipFreeAsync(p, s);
+}
+
 static int fail(mpgpu_ctx *c, int code, const std::string &m)
 {
     if (c) c->err = m;
     return code;
 }
 
-#define API_TRY try { AllocScope alloc_scope_(c ? c->stream : nullptr);
+#define API_TRY try { AllocScope alloc_scope_(c ? c->cache : nullptr);
 #define API_CATCH(ctx)                                                                   \
     }                                                                                    \
     catch (const MpError &e) { return fail(ctx, e.code, e.msg); }                        \
@@ -259,6 +363,7 @@ int mpgpu::create_context(const mpgpu_options *opt, int32_t device, hipStream_t 
         }
         (void)hipGetLastError();
     }
+    c->cache = new DevCache(c->stream, device);
     *out = c;
     return 0;
     }
@@ -273,11 +378,13 @@ extern "C" int mpgpu_destroy(mpgpu_ctx *c)
     // the context's buffers are freed in the order of its stream: the stream goes last
     hipStream_t s = c->stream;
     const bool own = c->own_stream;
-    if (s) (void)hipStreamSynchronize(s);
+    DevCache *cache = c->cache;
     delete c;
-    if (s) {
+    if (s) (void)hipStreamSynchronize(s);
+    delete cache;
+    if (s && own) {
         (void)hipStreamSynchronize(s);
-        if (own) (void)hipStreamDestroy(s);
+        (void)hipStreamDestroy(s);
     }
     return 0;
 }
@@ -433,7 +540,7 @@ extern "C" int mpgpu_read_mille_file(mpgpu_ctx *c, const char *path, int32_t for
     const size_t rp_saved = c->rec_ptr.size();
     const int64_t total_saved = c->nwords + (c->stage ? c->stage->n : 0);
     try {
-        AllocScope alloc_scope_(c->stream);
+        AllocScope alloc_scope_(c->cache);
         HIPCHK(hipSetDevice(c->device));
         if (c->built) throw MpError(24, "records cannot be added after the structure was built");
         gzFile f = gzopen(path, "rb");
@@ -1070,7 +1177,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             for (int32_t l : b.labels) { int v = c->var_index[tix_of(l)]; if (v > 0) gs.push_back(c->group_of[v]); }
             for (int32_t a : gs) for (int32_t b2 : gs) if (a >= b2) xp.push_back((int64_t)a * (a + 1) / 2 + b2);
         }
-        st_blocks(pm, c->ngroup, c->d_gfirst.p, xp, blk, s);
+        st_blocks(pm, c->ngroup, c->d_gfirst.p, xp, blk, true, s);
         c->nblock = blk.nblock;
         c->nstored = blk.nstored;
         c->blocks_on_host = false;
@@ -1311,7 +1418,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         c->d_pair_blk.release();
     }
     if (!sparse && c->rows.nq > 0) {
-        st_blocks(pm, c->ngroup, c->d_gfirst.p, {}, blk, s);
+        st_blocks(pm, c->ngroup, c->d_gfirst.p, {}, blk, false, s);
         c->rows.nblock = blk.nblock;
         c->rows.brow.swap(blk.brow);
         c->rows.brg.swap(blk.brg);

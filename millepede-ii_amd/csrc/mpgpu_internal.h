@@ -4,6 +4,7 @@
 #include "../../include/mpgpu.h"
 #include <algorithm>
 #include <string>
+#include <unordered_map>
 #include <vector>
 #include <cstring>
 #include <utility>
@@ -23,28 +24,49 @@ struct MpError {
     MpError(int c, std::string m) : code(c), msg(std::move(m)) {}
 };
 
-// Stream of the library call in progress on this thread.  Device buffers made during a call are
-// stream-ordered on its context's stream (hipMallocAsync / hipFreeAsync): hipFree synchronizes
-// the whole device, which would make concurrent contexts (serving workers) wait for each other's
-// kernels at every freed buffer.
-inline hipStream_t &alloc_stream()
+// Device memory of a context.  Buffers made during a library call are ordered on the context's
+// stream, so a freed block can serve the next buffer of that context at once; when the context ends
+// (its stream has finished) its free blocks go to a store shared by the contexts of the device.
+// hipFreeAsync takes 8 us for a small block and over 100 us from 1 MB on, and a job of the serving
+// engine frees some two hundred.  Blocks above CACHE_BLOCK go straight to hipMallocAsync /
+// hipFreeAsync; a context keeps at most CACHE_CONTEXT bytes of free blocks and the store CACHE_STORE,
+// and both are given back when an allocation fails.
+class DevCache {
+  public:
+    DevCache(hipStream_t st, int dev) : s(st), device(dev) {}
+    ~DevCache();                             // the stream has finished
+    DevCache(const DevCache &) = delete;
+    DevCache &operator=(const DevCache &) = delete;
+    void *get(size_t bytes);
+    void put(void *p, size_t bytes);
+    hipStream_t stream() const { return s; }
+
+  private:
+    hipStream_t s;
+    int device;
+    size_t held = 0;
+    std::unordered_map<size_t, std::vector<void *>> free_;
+    void drop();
+};
+// memory of the library call in progress on this thread (none: hipMalloc / hipFree)
+inline DevCache *&alloc_cache()
 {
-    static thread_local hipStream_t s = nullptr;
-    return s;
+    static thread_local DevCache *c = nullptr;
+    return c;
 }
 struct AllocScope {
-    hipStream_t prev;
-    explicit AllocScope(hipStream_t s) : prev(alloc_stream()) { alloc_stream() = s; }
-    ~AllocScope() { alloc_stream() = prev; }
+    DevCache *prev;
+    explicit AllocScope(DevCache *c) : prev(alloc_cache()) { alloc_cache() = c; }
+    ~AllocScope() { alloc_cache() = prev; }
     AllocScope(const AllocScope &) = delete;
     AllocScope &operator=(const AllocScope &) = delete;
 };
 
-// owning device buffer; freed in the order of the stream it was made on (see alloc_stream)
+// owning device buffer; freed in the order of the stream it was made for (see DevCache)
 template <typename T> struct DBuf {
     T *p = nullptr;
     size_t n = 0;
-    hipStream_t as = nullptr;
+    DevCache *as = nullptr;
     DBuf() = default;
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
@@ -52,7 +74,7 @@ template <typename T> struct DBuf {
     void release()
     {
         if (p) {
-            if (as) (void)hipFreeAsync(p, as);
+            if (as) as->put(p, sizeof(T) * n);
             else (void)hipFree(p);
         }
         p = nullptr;
@@ -64,8 +86,8 @@ template <typename T> struct DBuf {
         if (count == n && p) return;
         release();
         if (count == 0) return;
-        as = alloc_stream();
-        if (as) HIPCHK(hipMallocAsync((void **)&p, sizeof(T) * count, as));
+        as = alloc_cache();
+        if (as) p = (T *)as->get(sizeof(T) * count);
         else HIPCHK(hipMalloc((void **)&p, sizeof(T) * count));
         n = count;
     }
@@ -338,8 +360,9 @@ void st_record_stats(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<i
                      const DBuf<int32_t> &gl_tix, const int32_t *var, const int32_t *group_of, int32_t ngroup,
                      int32_t max_ngl, bool sparse, PairMap &pm, std::vector<int32_t> &st, std::vector<int64_t> &cnt_r,
                      DBuf<int32_t> &d_st, hipStream_t s);
+// storage: with the blocks' offsets and column lists
 void st_blocks(PairMap &pm, int32_t ngroup, const int32_t *gfirst, const std::vector<int64_t> &extra_pairs, BlockDev &B,
-               hipStream_t s);
+               bool storage, hipStream_t s);
 void st_pair_blocks(const StructIn &in, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix, const int32_t *var,
                     const int32_t *group_of, int32_t max_nseg, const DBuf<int32_t> &d_st, const PairMap &pm,
                     DBuf<int64_t> &rec_pb, DBuf<int32_t> &pair_blk, hipStream_t s);
