@@ -183,123 +183,6 @@ __global__ void k_pass_stats(int64_t n, const double *chi2, const int32_t *ndf, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Gauss-Jordan inversion of the packed matrix, restating sqminl (src/mpnum.f90:230-355):
-// per pivot step one single-block kernel picks the pivot exactly as the sequential scan does
-// (first unused j with |v_jj| > max(|v_kk|, eps*|diag_j|), i.e. the largest |v_jj| above its
-// threshold, ties to the lowest index) and stages the scaled pivot column; a grid-wide kernel
-// then applies the rank-1 elimination with the reference's operand order.
-// state: used[n] (0 free / 1 used), info[0]=k, info[1]=nrank, info[2]=stop
-// ---------------------------------------------------------------------------------------------
-__global__ void k_gj_init(int n, const double *v, double *diag, int *used, int *info)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        diag[i] = fabs(v[pk64s(i + 1, i + 1)]);
-        used[i] = 0;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) { info[0] = 0; info[1] = 0; info[2] = 0; }
-}
-
-__global__ __launch_bounds__(1024) void k_gj_pivot(int n, double *v, const double *diag, int *used, int *info,
-                                                   double *vk, double *b, double eps)
-{
-    __shared__ double sv[1024];
-    __shared__ int si[1024];
-    if (info[2]) return;
-    double best = -1.0;
-    int bi = 0x7fffffff;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        if (used[j]) continue;
-        double a = fabs(v[pk64s(j + 1, j + 1)]);
-        if (a > eps * diag[j] && (a > best || (a == best && j < bi))) { best = a; bi = j; }
-    }
-    sv[threadIdx.x] = best;
-    si[threadIdx.x] = bi;
-    __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            double a = sv[threadIdx.x + o];
-            int ai = si[threadIdx.x + o];
-            if (a > sv[threadIdx.x] || (a == sv[threadIdx.x] && ai < si[threadIdx.x])) { sv[threadIdx.x] = a; si[threadIdx.x] = ai; }
-        }
-        __syncthreads();
-    }
-    int k = si[0];
-    if (sv[0] < 0.0 || k == 0x7fffffff) { // no pivot: stop; clearing happens in k_gj_clear
-        if (threadIdx.x == 0) { info[0] = 0; info[2] = 1; }
-        return;
-    }
-    const int K = k + 1;
-    const int64_t kk = pk64s(K, K);
-    const double vkk = 1.0 / v[kk];
-    // scaled column k: vk(j) = v(jk)*vkk, vk(k) = 0  (sqminl lines 299-311)
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        int J = j + 1;
-        if (J == K) vk[j] = 0.0;
-        else {
-            int64_t jk = J < K ? pk64s(K, J) : pk64s(J, K);
-            vk[j] = v[jk] * vkk;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        used[k] = 1;
-        info[0] = K;
-        info[1] += 1;
-        b[k] = b[k] * vkk;
-        vk[n] = vkk;
-    }
-}
-
-// elimination (sqminl lines 312-319): v(jl) -= vk(l) * (vk(j)/vkk) for j,l != k;
-// column k takes vk, v(kk) = -vkk; b(j) -= b(k)*(vk(j)/vkk)
-__global__ void k_gj_update(int n, double *v, const double *vk, double *b, const int *info)
-{
-    if (info[2]) return;
-    const int K = info[0];
-    const double vkk = vk[n];
-    const int64_t total = ((int64_t)n * (n + 1)) / 2;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        int64_t J = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5) + 1;
-        while ((J * J - J) / 2 > t) J--;
-        while ((J * J + J) / 2 <= t) J++;
-        int64_t L = t - (J * J - J) / 2 + 1;
-        if (J == K && L == K) v[t] = -vkk;
-        else if (J == K) v[t] = vk[L - 1];
-        else if (L == K) v[t] = vk[J - 1];
-        else {
-            double vjk = vk[J - 1] / vkk;
-            v[t] = v[t] - vk[L - 1] * vjk;
-        }
-    }
-    if (blockIdx.x == 0) {
-        const double bk = b[K - 1];
-        for (int j = threadIdx.x; j < n; j += blockDim.x) {
-            if (j + 1 == K) continue;
-            double vjk = vk[j] / vkk;
-            b[j] = b[j] - bk * vjk;
-        }
-    }
-}
-
-// rank defect: clear rows/columns of unused pivots (sqminl lines 320-331), then negate all
-__global__ void k_gj_finish(int n, double *v, double *b, const int *used, const int *info)
-{
-    const int64_t total = ((int64_t)n * (n + 1)) / 2;
-    const bool clear = info[2] != 0;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        int64_t J = (int64_t)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5) + 1;
-        while ((J * J - J) / 2 > t) J--;
-        while ((J * J + J) / 2 <= t) J++;
-        int64_t L = t - (J * J - J) / 2 + 1;
-        double x = v[t];
-        if (clear && !used[J - 1] && !used[L - 1]) x = 0.0;
-        v[t] = -x;
-    }
-    if (clear && blockIdx.x == 0)
-        for (int j = threadIdx.x; j < n; j += blockDim.x) if (!used[j]) b[j] = 0.0;
-}
-
-// ---------------------------------------------------------------------------------------------
 // y = A x for the packed full matrix (avprd0 full storage, src/pede.f90:5069-5232):
 // 64x64 tiles of the lower triangle; each stored element serves both halves.
 // ---------------------------------------------------------------------------------------------
@@ -2032,23 +1915,6 @@ void l_pass_stats(int64_t n, const double *chi2, const int32_t *ndf, const int8_
     hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(TPB), 0, s, g, part, chi_out);
 }
 
-void l_gj_init(int n, const double *v, double *diag, int *used, int *info, hipStream_t s)
-{ hipLaunchKernelGGL(k_gj_init, dim3(nblk(n)), dim3(TPB), 0, s, n, v, diag, used, info); }
-void l_gj_step(int n, double *v, const double *diag, int *used, int *info, double *vk, double *b, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(1024), 0, s, n, v, diag, used, info, vk, b, 1.0e-10);
-    int64_t tot = ((int64_t)n * (n + 1)) / 2;
-    int g = nblk(tot);
-    if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(k_gj_update, dim3(g), dim3(TPB), 0, s, n, v, vk, b, info);
-}
-void l_gj_finish(int n, double *v, double *b, const int *used, const int *info, hipStream_t s)
-{
-    int64_t tot = ((int64_t)n * (n + 1)) / 2;
-    int g = nblk(tot);
-    if (g > 8192) g = 8192;
-    hipLaunchKernelGGL(k_gj_finish, dim3(g), dim3(TPB), 0, s, n, v, b, used, info);
-}
 
 __global__ void k_zero(int64_t n, double *y);
 void l_packed_symv(int n, const double *a, const double *x, double *y, double *scratch, hipStream_t s)

@@ -2924,16 +2924,9 @@ extern "C" int mpgpu_solve(mpgpu_ctx *c, const double *rhs, double *x, mpgpu_sol
         DBuf<double> keep;
         keep.alloc(c->nstored);
         HIPCHK(hipMemcpyAsync(keep.p, c->d_mat.p, sizeof(double) * c->nstored, hipMemcpyDeviceToDevice, s));
-        DBuf<double> diag, vk;
-        DBuf<int> used, info;
-        diag.alloc(n);
-        vk.alloc(n + 1);
-        used.alloc(n);
+        DBuf<int> info;
         info.alloc(4);
-        HIPCHK(hipMemcpyAsync(xd.p, b.p, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-        l_gj_init((int)n, c->d_mat.p, diag.p, used.p, info.p, s);
-        for (int64_t step = 0; step < n; step++) l_gj_step((int)n, c->d_mat.p, diag.p, used.p, info.p, vk.p, xd.p, s);
-        l_gj_finish((int)n, c->d_mat.p, xd.p, used.p, info.p, s);
+        gauss_jordan((int)n, c->d_mat.p, b.p, xd.p, info.p, s);
         int hinfo[4];
         info.download(hinfo, 4, s);
         HIPCHK(hipStreamSynchronize(s));

@@ -156,9 +156,8 @@ void l_get_band(const DevModel &M, int32_t n, int32_t mbandw, const int32_t *ind
 void l_dot(int64_t n, const double *a, const double *b, double *part, double *out, hipStream_t s);
 void l_pass_stats(int64_t n, const double *chi2, const int32_t *ndf, const int8_t *st, double *part, long long *ndfsum,
                   unsigned long long *hist, double *chi_out, hipStream_t s);
-void l_gj_init(int n, const double *v, double *diag, int *used, int *info, hipStream_t s);
-void l_gj_step(int n, double *v, const double *diag, int *used, int *info, double *vk, double *b, hipStream_t s);
-void l_gj_finish(int n, double *v, double *b, const int *used, const int *info, hipStream_t s);
+// inversion of the packed matrix p in place and x = A^-1 b; info[1]: rank (k_inv.hip)
+void gauss_jordan(int n, double *p, const double *b, double *x, int *info, hipStream_t s);
 // y = A x for the packed symmetric matrix; scratch: packed_symv_scratch(n) doubles
 void l_packed_symv(int n, const double *a, const double *x, double *y, double *scratch, hipStream_t s);
 int64_t packed_symv_scratch(int n);
