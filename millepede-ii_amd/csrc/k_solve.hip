@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void k_bsymv_rows8(int32_t ngroup, const int64
     if (slot == 0 && t < nr) y[fa + t] = v;
 }
 // Rows pass for groups of at most 8 parameters with the matrix read once, fully coalesced.  A
-// wavefront takes one block row.  Per step it stages the row's next eight off-diagonal blocks
+// wavefront takes one part of a block row.  Per step it stages the part's next eight off-diagonal blocks
 // (one contiguous range of the matrix, consecutive lanes reading consecutive doubles) into LDS,
 // with the x values of their column groups beside them.  Lane (k, j) = (lane / 8, lane % 8) then
 // forms row j of block k times x_b (summed over the blocks of the row in the lane) and column j of
@@ -544,25 +544,25 @@ __global__ __launch_bounds__(256) void k_bsymv_rows8(int32_t ngroup, const int64
 // are then added over k.
 // (W: wavefronts per workgroup, chosen per matrix by the autotuner of the product)
 template <int W>
-__global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int32_t ngroup, const int64_t *brow, const int32_t *bcf,
+__global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int64_t npart, const RowPart *part, const int32_t *bcf,
                                                          const int64_t *boff, const int32_t *gfirst, const double *a,
-                                                         const double *x, double *y, double *tb, int tbw)
+                                                         const double *x, double *yp, double *tb, int tbw)
 {
     __shared__ double st[W][512];
     __shared__ double sx[W][64];
     __shared__ int sd[W][16];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int ga = blockIdx.x * W + w;
-    if (ga >= ngroup) return;                        // whole wavefronts; no workgroup barrier below
-    const int k = lane >> 3, j = lane & 7;
+    const int64_t pi = blockIdx.x * (int64_t)W + w;
+    if (pi >= npart) return;                         // whole wavefronts; no workgroup barrier below
+    const RowPart P = part[pi];
+    if (P.ga < 0) return;
+    const int ga = P.ga, k = lane >> 3, j = lane & 7;
     const int fa = gfirst[ga] - 1, nr = gfirst[ga + 1] - 1 - fa;
-    const int64_t b0 = brow[ga], b1 = brow[ga + 1];
-    int64_t be = b1;
+    const int64_t b0 = P.b0, be = b0 + P.n;
     double accy = 0.0;
-    if (b1 > b0 && bcf[2 * (b1 - 1)] == fa) {
-        be = b1 - 1;
+    if (P.diag) {
         const int tr = min(j, nr - 1), sr = min(k, nr - 1);
-        const double dv = a[boff[b1 - 1] + (tr >= sr ? tr * nr + sr : sr * nr + tr)];
+        const double dv = a[boff[be] + (tr >= sr ? tr * nr + sr : sr * nr + tr)];
         const double dx = x[fa + sr];
         if (j < nr && k < nr) accy = dv * dx;
     }
@@ -668,7 +668,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int32_t ngroup, const 
     accy += __shfl_xor(accy, 8, 64);
     accy += __shfl_xor(accy, 16, 64);
     accy += __shfl_xor(accy, 32, 64);
-    if (k == 0 && j < nr) y[fa + j] = accy;
+    if (k == 0 && j < nr) yp[8 * pi + j] = accy;
 }
 // Rows pass when every parameter group has the same size G <= 8 (blocks G x G; group g's first
 // index is g G).  As k_bsymv_rows_st, with the block layout known: the row's off-diagonal blocks
@@ -678,35 +678,35 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int32_t ngroup, const 
 // step t + 2, all unconditionally (clamped indices; the transposed products of lanes without a
 // block go to a spare slot past the end of tb), so that every wait is for the step it needs.
 template <int G, int W, bool V2>
-__global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int32_t ngroup, const int64_t *__restrict__ brow,
+__global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int64_t npart, const RowPart *__restrict__ part,
                                                                const int32_t *__restrict__ bcol,
-                                                               const int64_t *__restrict__ boff,
                                                                const double *__restrict__ a, const double *__restrict__ x,
-                                                               double *__restrict__ y, double *__restrict__ tb,
+                                                               double *__restrict__ yp, double *__restrict__ tb,
                                                                int64_t tb_spare)
 {
     constexpr int S = G * G;                   // values per block
     __shared__ __align__(16) double st[W][8 * S];
     __shared__ double sx[W][64];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int ga = blockIdx.x * W + w;
-    if (ga >= ngroup) return;                  // whole wavefronts; no workgroup barrier below
+    const int64_t pi = blockIdx.x * (int64_t)W + w;
+    if (pi >= npart) return;                   // whole wavefronts; no workgroup barrier below
+    const RowPart P = part[pi];
+    if (P.ga < 0) return;
     const int k = lane >> 3, j = lane & 7;
-    const int fa = ga * G;
-    const int64_t b0 = brow[ga], b1 = brow[ga + 1];
-    const int64_t be = b1 - 1;                 // the last block of a row is its diagonal block
+    const int fa = P.ga * G;
+    const int64_t b0 = P.b0, be = b0 + P.n;
+    const int64_t s_row = P.off;
     double accy = 0.0;
-    {
+    if (P.diag) {                              // the diagonal block follows the row's last part
         const int tr = min(j, G - 1), sr = min(k, G - 1);
-        const double dv = a[boff[be] + (tr >= sr ? tr * G + sr : sr * G + tr)];
+        const double dv = a[s_row + (int64_t)P.n * S + (tr >= sr ? tr * G + sr : sr * G + tr)];
         const double dx = x[fa + sr];
         if (j < G && k < G) accy = dv * dx;
     }
     double xa[G];
 #pragma unroll
     for (int r = 0; r < G; r++) xa[r] = x[fa + r];
-    const int64_t s_row = boff[b0];
-    const int64_t nsteps = (be - b0 + 7) / 8;
+    const int64_t nsteps = (P.n + 7) / 8;
     // matrix values per lane and step; with V2 (even block size, so every step starts on 16
     // bytes) they are loaded two at a time
     constexpr int NV2 = (4 * S + 63) / 64;
@@ -719,36 +719,37 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int32_t ngroup, const i
     auto ld_col = [&](int64_t t) -> int { return bcol[min(b0 + 8 * t + k, be - 1)]; };
     auto ld_x = [&](int64_t t, int col) -> double { return x[col * G + min(j, G - 1)]; };
     auto ld_v = [&](int64_t t, StepRegs &R) {
-        const int len = (int)(min((int64_t)8, be - (b0 + 8 * t)) * S);
-        const int64_t s0 = s_row + 8 * t * S;
+        // (a step past the last reads one value that was read before)
+        const int len = (int)(max(min((int64_t)8, be - (b0 + 8 * t)), (int64_t)0) * S);
+        const int64_t s0 = s_row + 8 * min(t, nsteps - 1) * S;
         if constexpr (V2) {
             const double2 *a2 = reinterpret_cast<const double2 *>(a + s0);
 #pragma unroll
             for (int i = 0; i < NV2; i++) {
-                const double2 u = a2[min(lane + 64 * i, len / 2 - 1)];
+                const double2 u = a2[min(lane + 64 * i, max(len / 2, 1) - 1)];
                 R.v[2 * i] = u.x;
                 R.v[2 * i + 1] = u.y;
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < NV; i++) R.v[i] = a[s0 + min(lane + 64 * i, len - 1)];
+            for (int i = 0; i < NV; i++) R.v[i] = a[s0 + min(lane + 64 * i, max(len, 1) - 1)];
         }
     };
-    if (nsteps == 0) {                          // a row with its diagonal block only
+    if (nsteps == 0) {                          // a row without off-diagonal blocks
         accy += __shfl_xor(accy, 8, 64);
         accy += __shfl_xor(accy, 16, 64);
         accy += __shfl_xor(accy, 32, 64);
-        if (k == 0 && j < G) y[fa + j] = accy;
+        if (k == 0 && j < G) yp[8 * pi + j] = accy;
         return;
     }
-    // steps past the last are loaded at the last step's indices and computed as empty steps
+    // steps past the last are computed as empty steps
     StepRegs RA, RB;
     RA.col = ld_col(0);
     RA.x = ld_x(0, RA.col);
     ld_v(0, RA);
     RB.col = ld_col(min((int64_t)1, nsteps - 1));
     RB.x = ld_x(1, RB.col);
-    ld_v(min((int64_t)1, nsteps - 1), RB);
+    ld_v(1, RB);
     int col2 = ld_col(min((int64_t)2, nsteps - 1)), col_next = 0;   // column groups of step t + 2
     auto step = [&](int64_t t, StepRegs &R) {
         const int64_t g0 = b0 + 8 * t;
@@ -775,7 +776,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int32_t ngroup, const i
             col_next = ld_col(t3);
             R.col = col2;
             R.x = ld_x(t2, col2);
-            ld_v(t2, R);
+            ld_v(t + 2, R);
             col2 = col_next;
         }
         const double *B = &st[w][max(min(k, kn - 1), 0) * S];
@@ -799,31 +800,46 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int32_t ngroup, const i
     accy += __shfl_xor(accy, 8, 64);
     accy += __shfl_xor(accy, 16, 64);
     accy += __shfl_xor(accy, 32, 64);
-    if (k == 0 && j < G) y[fa + j] = accy;
+    if (k == 0 && j < G) yp[8 * pi + j] = accy;
 }
-// Columns pass from the transposed block products of the rows pass: column group gb sums
-// tb[tbw * block + t] over its off-diagonal blocks in column-list order (slot s takes entries
-// s, s+8, ...; one read of the block's values), then over the slots.
-__global__ __launch_bounds__(256) void k_bsymv_colst(int32_t ngroup, const int64_t *ccol_ptr, const int32_t *cc_blk,
-                                                     const int32_t *gfirst, const double *tb, int tbw, double *y)
+// Columns pass from the sums of the row parts and the transposed block products of the rows pass:
+// group gb sums its parts, then tb[tbw * block + t] over its off-diagonal blocks in column-list
+// order (slot s takes entries s, s+8, ...; one read of the block's values), then over the slots.
+// A chain of dependent loads bounds it (list entry, then its value): the entries of 64 blocks come
+// with one load, one per lane, and the eight values of a slot are in flight together (673,083
+// blocks of 4,000 groups 25 -> 14.2 us, 1,000 groups 12.5 -> 6.5 us).
+__global__ __launch_bounds__(256) void k_bsymv_colst(int32_t ngroup, const int64_t *__restrict__ ccol_ptr,
+                                                     const int32_t *__restrict__ cc_blk,
+                                                     const int32_t *__restrict__ gfirst,
+                                                     const int64_t *__restrict__ part_ptr,
+                                                     const double *__restrict__ yp, const double *__restrict__ tb,
+                                                     int tbw, double *__restrict__ y)
 {
     const int gb = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, slot = lane >> 3, t = lane & 7;
     if (gb >= ngroup) return;
     const int fb = gfirst[gb] - 1, nc = gfirst[gb + 1] - 1 - fb;
     const int64_t q0 = ccol_ptr[gb], q1 = ccol_ptr[gb + 1];
-    if (q1 <= q0) return;
-    double a0 = 0.0, a1 = 0.0;
-    int64_t q = q0 + slot;
+    const int64_t p0 = part_ptr[gb], p1 = part_ptr[gb + 1];
     const int tt = min(t, nc - 1);
-    for (; q + 8 < q1; q += 16) {
-        const int64_t k0 = cc_blk[q], k1 = cc_blk[q + 8];
-        a0 += tb[tbw * k0 + tt];
-        a1 += tb[tbw * k1 + tt];
+    double pv = 0.0;
+    for (int64_t p = p0 + slot; p < p1; p += 8) pv += yp[8 * p + tt];
+    double a0 = 0.0, a1 = 0.0;
+    int blk = q1 > q0 ? cc_blk[min(q0 + lane, q1 - 1)] : 0;
+    for (int64_t q = q0; q < q1; q += 64) {
+        double v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = tb[tbw * (int64_t)__shfl(blk, 8 * i + slot, 64) + tt];
+        blk = cc_blk[min(q + 64 + lane, q1 - 1)];
+        const int m = (int)min(q1 - q, (int64_t)64);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            a0 += 8 * i + slot < m ? v[i] : 0.0;
+            a1 += 8 * i + 8 + slot < m ? v[i + 1] : 0.0;
+        }
     }
-    if (q < q1) a0 += tb[tbw * (int64_t)cc_blk[q] + tt];
-    const double acc = sum_slots(a0 + a1);
-    if (slot == 0 && t < nc) y[fb + t] += acc;
+    const double acc = sum_slots(pv) + sum_slots(a0 + a1);
+    if (slot == 0 && t < nc) y[fb + t] = acc;
 }
 // Columns pass for groups of at most 8 parameters: the off-diagonal blocks (row group a, column
 // group gb) of a column group, lane t of a slot taking column t of the slot's block and loading its
@@ -1946,52 +1962,51 @@ int block_symv_variants(int32_t ugrp, int32_t maxgrp, int *out)
     return n;
 }
 template <int G, int W, bool V2>
-static void launch_rows_u(int32_t ngroup, const int64_t *brow, const int32_t *bcol, const int64_t *boff, const double *a,
-                          const double *x, double *y, double *tb, int64_t spare, hipStream_t s)
+static void launch_rows_u(const BlockParts &P, const int32_t *bcol, const double *a, const double *x, double *tb,
+                          int64_t spare, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_bsymv_rows_u<G, W, V2>), dim3((unsigned)((ngroup + W - 1) / W)), dim3(64 * W), 0, s, ngroup,
-                       brow, bcol, boff, a, x, y, tb, spare);
+    hipLaunchKernelGGL((k_bsymv_rows_u<G, W, V2>), dim3((unsigned)((P.n + W - 1) / W)), dim3(64 * W), 0, s, P.n, P.part, bcol, a,
+                       x, P.yp, tb, spare);
 }
 template <int W>
-static void launch_rows_u_g(int32_t g, bool v2, int32_t ngroup, const int64_t *brow, const int32_t *bcol,
-                            const int64_t *boff, const double *a, const double *x, double *y, double *tb, int64_t spare,
-                            hipStream_t s)
+static void launch_rows_u_g(int32_t g, bool v2, const BlockParts &P, const int32_t *bcol, const double *a, const double *x,
+                            double *tb, int64_t spare, hipStream_t s)
 {
     switch (g) {
-    case 1: launch_rows_u<1, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s); break;
+    case 1: launch_rows_u<1, W, false>(P, bcol, a, x, tb, spare, s); break;
     case 2:
-        if (v2) launch_rows_u<2, W, true>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-        else launch_rows_u<2, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
+        if (v2) launch_rows_u<2, W, true>(P, bcol, a, x, tb, spare, s);
+        else launch_rows_u<2, W, false>(P, bcol, a, x, tb, spare, s);
         break;
-    case 3: launch_rows_u<3, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s); break;
+    case 3: launch_rows_u<3, W, false>(P, bcol, a, x, tb, spare, s); break;
     case 4:
-        if (v2) launch_rows_u<4, W, true>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-        else launch_rows_u<4, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
+        if (v2) launch_rows_u<4, W, true>(P, bcol, a, x, tb, spare, s);
+        else launch_rows_u<4, W, false>(P, bcol, a, x, tb, spare, s);
         break;
-    case 5: launch_rows_u<5, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s); break;
+    case 5: launch_rows_u<5, W, false>(P, bcol, a, x, tb, spare, s); break;
     case 6:
-        if (v2) launch_rows_u<6, W, true>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-        else launch_rows_u<6, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
+        if (v2) launch_rows_u<6, W, true>(P, bcol, a, x, tb, spare, s);
+        else launch_rows_u<6, W, false>(P, bcol, a, x, tb, spare, s);
         break;
-    case 7: launch_rows_u<7, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s); break;
+    case 7: launch_rows_u<7, W, false>(P, bcol, a, x, tb, spare, s); break;
     default:
-        if (v2) launch_rows_u<8, W, true>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-        else launch_rows_u<8, W, false>(ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
+        if (v2) launch_rows_u<8, W, true>(P, bcol, a, x, tb, spare, s);
+        else launch_rows_u<8, W, false>(P, bcol, a, x, tb, spare, s);
         break;
     }
 }
 template <int W>
-static void launch_rows_st(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const int64_t *boff,
-                           const int32_t *gfirst, const double *a, const double *x, double *y, double *tb, int tbw,
-                           hipStream_t s)
+static void launch_rows_st(const BlockParts &P, const int32_t *bcf, const int64_t *boff, const int32_t *gfirst,
+                           const double *a, const double *x, double *tb, int tbw, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_bsymv_rows_st<W>, dim3((unsigned)((ngroup + W - 1) / W)), dim3(64 * W), 0, s, ngroup, brow, bcf,
-                       boff, gfirst, a, x, y, tb, tbw);
+    hipLaunchKernelGGL(k_bsymv_rows_st<W>, dim3((unsigned)((P.n + W - 1) / W)), dim3(64 * W), 0, s, P.n, P.part, bcf, boff,
+                       gfirst, a, x, P.yp, tb, tbw);
 }
 void l_block_symv(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const int64_t *boff, const int32_t *gfirst,
                   const int64_t *ccol_ptr, const int64_t *cc_off, const int32_t *cc_fn, const double *a,
                   const double *x, double *y, int32_t nvar, int64_t nall, int32_t maxgrp, const int32_t *cc_blk,
-                  double *tb, int32_t ugrp, const int32_t *bcol, int64_t nblock, int variant, hipStream_t s)
+                  double *tb, int32_t ugrp, const int32_t *bcol, int64_t nblock, const BlockParts &parts, int variant,
+                  hipStream_t s)
 {
     // rows beyond the parameter groups (Lagrange multipliers) are written by k_cons_symv
     (void)nall;
@@ -2007,16 +2022,16 @@ void l_block_symv(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const
         if (kind != 1) {
             const int64_t spare = (int64_t)ugrp * nblock;
             const bool v2 = kind == 2;
-            if (w == 2) launch_rows_u_g<2>(ugrp, v2, ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-            else if (w == 8) launch_rows_u_g<8>(ugrp, v2, ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
-            else launch_rows_u_g<4>(ugrp, v2, ngroup, brow, bcol, boff, a, x, y, tb, spare, s);
+            if (w == 2) launch_rows_u_g<2>(ugrp, v2, parts, bcol, a, x, tb, spare, s);
+            else if (w == 8) launch_rows_u_g<8>(ugrp, v2, parts, bcol, a, x, tb, spare, s);
+            else launch_rows_u_g<4>(ugrp, v2, parts, bcol, a, x, tb, spare, s);
         } else {
-            if (w == 2) launch_rows_st<2>(ngroup, brow, bcf, boff, gfirst, a, x, y, tb, tbw, s);
-            else if (w == 8) launch_rows_st<8>(ngroup, brow, bcf, boff, gfirst, a, x, y, tb, tbw, s);
-            else launch_rows_st<4>(ngroup, brow, bcf, boff, gfirst, a, x, y, tb, tbw, s);
+            if (w == 2) launch_rows_st<2>(parts, bcf, boff, gfirst, a, x, tb, tbw, s);
+            else if (w == 8) launch_rows_st<8>(parts, bcf, boff, gfirst, a, x, tb, tbw, s);
+            else launch_rows_st<4>(parts, bcf, boff, gfirst, a, x, tb, tbw, s);
         }
         hipLaunchKernelGGL(k_bsymv_colst, dim3((unsigned)((ngroup + 3) / 4)), dim3(256), 0, s, ngroup, ccol_ptr, cc_blk,
-                           gfirst, tb, tbw, y);
+                           gfirst, parts.ptr, parts.yp, tb, tbw, y);
         return;
     }
     if (maxgrp <= 8)

@@ -1074,6 +1074,68 @@ void st_blocks(PairMap &pm, int32_t ngroup, const int32_t *gfirst, const std::ve
     HIPCHK(hipStreamSynchronize(s));
 }
 
+// Row parts of the block product: a row of m off-diagonal blocks is cut into ceil(m / C) parts of
+// equal length (a multiple of the product's eight-block step).
+__global__ void k_part_count(int32_t ngroup, const int64_t *brow, const int32_t *bcol, int64_t C, int64_t *cnt)
+{
+    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g <= ngroup; g += gridDim.x * blockDim.x) {
+        int64_t m = 0;
+        if (g < ngroup) {
+            m = brow[g + 1] - brow[g];
+            if (m > 0 && bcol[brow[g + 1] - 1] == g) m--;
+            m = max((m + C - 1) / C, (int64_t)1);
+        }
+        cnt[g] = m;
+    }
+}
+__global__ void k_part_fill(int32_t ngroup, int64_t npart, const int64_t *brow, const int32_t *bcol, const int64_t *boff,
+                            const int64_t *ptr, RowPart *part)
+{
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < npart; p += (int64_t)gridDim.x * blockDim.x) {
+        RowPart P = {-1, 0, 0, 0, 0};
+        if (p < ptr[ngroup]) {
+            int lo = 0, hi = ngroup;             // ptr[lo] <= p < ptr[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) / 2;
+                if (ptr[mid] <= p) lo = mid;
+                else hi = mid;
+            }
+            const int64_t b0 = brow[lo], b1 = brow[lo + 1], np = ptr[lo + 1] - ptr[lo], i = p - ptr[lo];
+            const int diag = b1 > b0 && bcol[b1 - 1] == lo;
+            const int64_t m = b1 - b0 - diag, len = ((m + np - 1) / np + 7) / 8 * 8;
+            const int64_t q = min(i * len, m), n = i + 1 < np ? min(len, m - q) : m - q;
+            P.ga = lo;
+            P.b0 = (int32_t)(b0 + q);
+            P.n = (int32_t)n;
+            P.diag = diag && i + 1 == np;
+            P.off = boff[b0 + q];
+        }
+        part[p] = P;
+    }
+}
+int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff,
+                     DBuf<RowPart> &part, DBuf<int64_t> &ptr, hipStream_t s)
+{
+    // A wavefront that takes a whole row is as slow as its row is long, and the rows of a small
+    // matrix do not fill the card: parts of 64 blocks (eight steps), longer ones where those would be
+    // more than 8,192 (8 wavefronts a SIMD), up to whole rows.  Measured per product: 4,000 groups of
+    // 6, 673,083 blocks (194 MB), rows pass 50 us by whole rows, 38 us (5.1 TB/s) in parts of 64, the
+    // same from 32 to 96 and 58 us in parts of 8; 1,000 groups 19.7 -> 9.9 us (16: 10.6, 96: 11.5).
+    const int64_t C = std::max<int64_t>(64, (nblock / 8192 + 7) / 8 * 8);
+    const int64_t npart = ngroup + nblock / C;
+    DBuf<int64_t> cnt;
+    DBuf<uint8_t> tmp;
+    cnt.alloc(ngroup + 1);
+    ptr.alloc(ngroup + 1);
+    part.alloc(std::max<int64_t>(npart, 1));
+    hipLaunchKernelGGL(k_part_count, dim3(grid_for(ngroup + 1, 256)), dim3(256), 0, s, ngroup, brow, bcol, C, cnt.p);
+    scan_excl(cnt.p, ptr.p, ngroup + 1, s, tmp);
+    hipLaunchKernelGGL(k_part_fill, dim3(grid_for(npart, 256)), dim3(256), 0, s, ngroup, npart, brow, bcol, boff, ptr.p,
+                       part.p);
+    HIPCHK(hipGetLastError());
+    return npart;
+}
+
 void st_pair_blocks(const StructIn &in, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix, const int32_t *var,
                     const int32_t *group_of, int32_t max_nseg, const DBuf<int32_t> &d_st, const PairMap &pm,
                     DBuf<int64_t> &rec_pb, DBuf<int32_t> &pair_blk, hipStream_t s)

@@ -123,6 +123,9 @@ struct mpgpu_ctx {
     DBuf<int32_t> d_bcf, d_cc_fn;   // per block / per column-list entry: first index and size of the other group
     DBuf<int32_t> d_cc_blk;         // per column-list entry: the block
     DBuf<double> d_tb;              // per block: its transposed product (max_grp values, groups <= 8)
+    DBuf<RowPart> d_bpart;          // parts of the block rows for the block product, and each row's first
+    DBuf<int64_t> d_part_ptr;
+    BlockParts parts;               // views of d_bpart, d_part_ptr and the end of d_tb
     DBuf<double> d_psymv;           // full storage: partial sums of the packed product (deterministic)
     DBuf<unsigned long long> d_cnt;
     DBuf<double> d_chi2;
@@ -731,7 +734,7 @@ static void tune_block_symv(mpgpu_ctx *c)
         auto run = [&]() {
             l_block_symv(c->ngroup, c->d_brow.p, c->d_bcf.p, c->d_boff.p, c->d_gfirst.p, c->d_ccol_ptr.p, c->d_cc_off.p,
                          c->d_cc_fn.p, c->d_mat.p, x.p, y.p, c->nvar, c->nall, c->plan.max_grp, c->d_cc_blk.p,
-                         c->d_tb.p, c->uniform_grp, c->d_bcol.p, c->nblock, cand[q], s);
+                         c->d_tb.p, c->uniform_grp, c->d_bcol.p, c->nblock, c->parts, cand[q], s);
         };
         run();
         float ms[3];
@@ -1403,10 +1406,19 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         if (c->plan.max_grp <= 8) {
             c->d_cc_blk.swap(blk.cc_blk);
             // transposed products of the blocks, and a spare slot per lane for the uniform kernel
-            c->d_tb.alloc((size_t)c->plan.max_grp * std::max<int64_t>(1, c->nblock) + 64);
+            // and the sums of the row parts
+            const int64_t ntb = c->plan.max_grp * std::max<int64_t>(1, c->nblock) + 64;
+            c->parts.n = st_row_parts(c->ngroup, c->nblock, c->d_brow.p, c->d_bcol.p, c->d_boff.p, c->d_bpart, c->d_part_ptr, s);
+            c->d_tb.alloc((size_t)(ntb + 8 * c->parts.n));
+            c->parts.part = c->d_bpart.p;
+            c->parts.ptr = c->d_part_ptr.p;
+            c->parts.yp = c->d_tb.p + ntb;
         } else {
             c->d_cc_blk.release();
             c->d_tb.release();
+            c->d_bpart.release();
+            c->d_part_ptr.release();
+            c->parts = BlockParts();
         }
     } else {
         c->d_rec_cb.release();
@@ -1915,7 +1927,7 @@ void avprod_dev(mpgpu_ctx *c, const double *x, double *y)
     if (c->opt.matsto == MPGPU_SPARSE) {
         l_block_symv(c->ngroup, c->d_brow.p, c->d_bcf.p, c->d_boff.p, c->d_gfirst.p, c->d_ccol_ptr.p, c->d_cc_off.p,
                      c->d_cc_fn.p, c->d_mat.p, x, y, c->nvar, c->nall, c->plan.max_grp, c->d_cc_blk.p, c->d_tb.p,
-                     c->uniform_grp, c->d_bcol.p, c->nblock, c->spmv_variant, s);
+                     c->uniform_grp, c->d_bcol.p, c->nblock, c->parts, c->spmv_variant, s);
         l_cons_symv(c->ncon, c->nvar, c->d_cptr.p, c->d_cidx.p, c->d_cval.p, x, y, s);
     } else {
         l_packed_symv(c->nall, c->d_mat.p, x, y, c->d_psymv.p, s);

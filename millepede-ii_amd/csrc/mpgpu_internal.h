@@ -171,10 +171,25 @@ void l_mr_sub(int64_t n, const MrState *st, const double *r2, double *r1, double
 void l_mr_end(int64_t n, MrState *st, const double *r2, double *y, int w, int nb, const double *Cb, const double *t, double *part,
               hipStream_t s);
 void l_mr_next(int64_t n, const MrState *st, const double *y, double *v, double *w, double *w2, double *x, hipStream_t s);
+// A part of a block row for the block product: n off-diagonal blocks from block b0 of the values at
+// a[off], and with diag the row's diagonal block behind them (ga < 0: no part).  The parts of a row
+// are summed by the columns pass, so the split is part of the sum's order and every variant of the
+// product uses the same one.
+struct RowPart {
+    int32_t ga, b0, n, diag;
+    int64_t off;
+};
+struct BlockParts {
+    int64_t n = 0;                  // entries of part (the last ones may be empty)
+    const RowPart *part = nullptr;
+    const int64_t *ptr = nullptr;   // per block row: its first part
+    double *yp = nullptr;           // 8 sums per part
+};
 void l_block_symv(int32_t ngroup, const int64_t *brow, const int32_t *bcf, const int64_t *boff, const int32_t *gfirst,
                   const int64_t *ccol_ptr, const int64_t *cc_off, const int32_t *cc_fn, const double *a,
                   const double *x, double *y, int32_t nvar, int64_t nall, int32_t maxgrp, const int32_t *cc_blk,
-                  double *tb, int32_t ugrp, const int32_t *bcol, int64_t nblock, int variant, hipStream_t s);
+                  double *tb, int32_t ugrp, const int32_t *bcol, int64_t nblock, const BlockParts &parts, int variant,
+                  hipStream_t s);
 // variants of the product with identical arithmetic (for the autotuner); returns their number
 int block_symv_variants(int32_t ugrp, int32_t maxgrp, int *out);
 void l_cons_symv(int32_t ncon, int32_t nvar, const int64_t *cptr, const int32_t *cidx, const double *cval, const double *x,
@@ -329,6 +344,9 @@ struct BlockDev {
     DBuf<int64_t> brow, boff, ccol_ptr, cc_off;
     DBuf<int32_t> brg, bcol, bcf, cc_fn, cc_blk;
 };
+// parts of the block rows for the block product (groups <= 8): returns the entries of part
+int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff,
+                     DBuf<RowPart> &part, DBuf<int64_t> &ptr, hipStream_t s);
 // equation tables of the records (decodeNextMeasurement): fills in.neq, in.rec_eq, in.eq_sl,
 // in.eq_n; error 20 names the first record that breaks the format
 int64_t st_decode(StructIn &in, DBuf<int64_t> &rec_eq, DBuf<int64_t> &eq_sl, DBuf<uint32_t> &eq_n, hipStream_t s);
