@@ -24,7 +24,6 @@ namespace mpgpu {
 
 #define BNT 256
 #define BWAVES (BNT / 64)
-#define NWM 4          // 64-bit words of a local-parameter support mask (nalc <= 256)
 #define QCH 16         // support entries of one class handled per register chunk
 
 __device__ __forceinline__ int64_t bpk64(int64_t i, int64_t j) { return (i * i - i) / 2 + j - 1; }
@@ -35,15 +34,8 @@ template <typename T> __device__ __forceinline__ double bval(const DevRecords &R
 template <> __device__ __forceinline__ double bval<float>(const DevRecords &R, int64_t w) { return (double)R.vf[w]; }
 template <> __device__ __forceinline__ double bval<double>(const DevRecords &R, int64_t w) { return R.vd[w]; }
 
-__device__ __forceinline__ int64_t band_block_addr(const DevModel &M, int32_t blk, int va, int vb, int ga, int gb)
-{
-    int fa = M.gfirst[ga], fb = M.gfirst[gb];
-    int nc = M.gfirst[gb + 1] - fb;
-    return M.boff[blk] + (int64_t)(va - fa) * nc + (vb - fb);
-}
-
 __device__ __forceinline__ void band_mat_add(const DevModel &M, int va, int vb, double v, const int32_t *seg_of,
-                                             const int32_t *seg_grp, const int32_t *pblk, int pos_a, int pos_b)
+                                             const int2 *seg_fn, const int32_t *pblk, int pos_a, int pos_b)
 {
     if (!M.sparse) {
         atomicAdd(&M.mat[bpk64(va, vb)], v);
@@ -51,7 +43,7 @@ __device__ __forceinline__ void band_mat_add(const DevModel &M, int va, int vb, 
         int sa = seg_of[pos_a], sb = seg_of[pos_b];
         int blk = pblk[(sa * sa + sa) / 2 + sb];
         if (blk < 0) return;
-        atomicAdd(&M.mat[band_block_addr(M, blk, va, vb, seg_grp[sa], seg_grp[sb])], v);
+        atomicAdd(&M.mat[M.boff[blk] + (int64_t)(va - seg_fn[sa].x) * seg_fn[sb].y + (vb - seg_fn[sb].x)], v);
     }
 }
 
@@ -133,9 +125,62 @@ __device__ void sqminv_small(double *v, double *b, int n, int *nrank, double *di
     for (int i = 1; i <= (n * n + n) / 2; i++) v[i] = -v[i];
 }
 
+// wavefront-wide order of LDS accesses (one wavefront's LDS operations complete in order)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ double readlane_d(double v, int l)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l), hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+    return __hiloint2double(hi, lo);
+}
+// Equations in order, 64 at a time, by one wavefront: lane q gets word q of the equation (its local
+// or total position and its value), the words of the next equations are in flight, and
+// f(i, words) does equation i.  Every equation has at most 64 words.
+template <typename T> struct EqWords { int nl, ng, wx; T v; };
+template <typename T> __device__ __forceinline__ T raw_val(const DevRecords &R, int64_t w);
+template <> __device__ __forceinline__ float raw_val<float>(const DevRecords &R, int64_t w) { return R.vf[w]; }
+template <> __device__ __forceinline__ double raw_val<double>(const DevRecords &R, int64_t w) { return R.vd[w]; }
+__device__ __forceinline__ double lane_val(float v, int l) { return (double)__shfl(v, l, 64); }
+__device__ __forceinline__ double lane_val(double v, int l) { return __shfl(v, l, 64); }
+template <typename T, class F>
+__device__ __forceinline__ void each_equation(const DevRecords &R, int64_t e0, int neq, int lane, F f)
+{
+    constexpr int D = 4;                                   // equations in flight
+    for (int base = 0; base < neq; base += 64) {
+        const int ne = min(64, neq - base);
+        const int64_t slv = R.eq_sl[e0 + base + min(lane, ne - 1)];
+        const uint32_t env = R.eq_n[e0 + base + min(lane, ne - 1)];
+        EqWords<T> W[D];
+        auto ld = [&](int i, EqWords<T> &E) {
+            const int q = min(i, ne - 1);
+            const int64_t sl = ((int64_t)__builtin_amdgcn_readlane((int)(slv >> 32), q) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane((int)slv, q);
+            const uint32_t en = (uint32_t)__builtin_amdgcn_readlane((int)env, q);
+            E.nl = en & 0xffff;
+            E.ng = en >> 16;
+            const int64_t w = sl + min(lane, E.nl + E.ng + 1);
+            E.wx = R.widx[w];
+            E.v = raw_val<T>(R, w);
+        };
+#pragma unroll
+        for (int u = 0; u < D; u++) ld(u, W[u]);
+        for (int i = 0; i < ne; i += D) {
+#pragma unroll
+            for (int u = 0; u < D; u++) {
+                if (i + u < ne) f(base + i + u, W[u]);
+                ld(i + u + D, W[u]);
+            }
+        }
+    }
+}
+
 // band solve with the root-free factor (dbcslv, src/Dbandmatrix.f90:521-560), one thread;
 // w column-major w(mp1, n) 1-based through W(r, c) = w[(c - 1) * mp1 + r]; x 1-based, in place
-__device__ void dbcslv_thread(const double *w, int mp1, int n, double *x)
+__device__ void dbcslv_any(const double *w, int mp1, int n, double *x)
 {
     for (int i = 1; i <= n; i++) {
         const double xi = x[i];
@@ -150,8 +195,52 @@ __device__ void dbcslv_thread(const double *w, int mp1, int n, double *x)
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, PassOpts o, RecOut out, BandPlan P,
+// the same for a half-width of at most MB: the last MB solutions in registers, so that the chain
+// from one row to the next has no LDS access (the loads run ahead of it); the terms of a row come
+// in the same order
+template <int MB>
+__device__ void dbcslv_win(const double *w, int mp1, int n, double *x)
+{
+    double xw[MB];
+#pragma unroll
+    for (int j = 0; j < MB; j++) xw[j] = 0.0;
+    for (int i = 1; i <= n; i++) {
+        double v = x[i];
+#pragma unroll
+        for (int j = MB; j >= 1; j--) {                    // sources i - MB .. i - 1
+            const bool ok = j < mp1 && j < i;
+            const double c = w[ok ? (i - j - 1) * mp1 + j + 1 : 1];
+            v = v - (ok ? c : 0.0) * xw[j - 1];
+        }
+#pragma unroll
+        for (int j = MB - 1; j >= 1; j--) xw[j] = xw[j - 1];
+        xw[0] = v;
+        x[i] = v;
+    }
+#pragma unroll
+    for (int j = 0; j < MB; j++) xw[j] = 0.0;
+    for (int i = n; i >= 1; i--) {
+        double v = x[i] * w[(i - 1) * mp1 + 1];
+#pragma unroll
+        for (int j = 1; j <= MB; j++) {
+            const bool ok = j < mp1 && i + j <= n;
+            const double c = w[ok ? (i - 1) * mp1 + j + 1 : 1];
+            v = v - (ok ? c : 0.0) * xw[j - 1];
+        }
+#pragma unroll
+        for (int j = MB - 1; j >= 1; j--) xw[j] = xw[j - 1];
+        xw[0] = v;
+        x[i] = v;
+    }
+}
+__device__ void dbcslv_thread(const double *w, int mp1, int n, double *x)
+{
+    if (mp1 <= 7) dbcslv_win<6>(w, mp1, n, x);
+    else dbcslv_any(w, mp1, n, x);
+}
+
+template <typename T, bool VL>
+__global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel M, PassOpts o, RecOut out, BandPlan P,
                                                       const int64_t *ids, int64_t nb, const int32_t *binfo,
                                                       double *scratch)
 {
@@ -177,8 +266,8 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
     double *ring = sdiag + P.nbdr_max + 1;         // [mp1_max * (NA + 1)]
     double *gval = ring + P.mp1_max * (NA + 1);    // [max_sup]
     double *red = gval + P.max_sup;                // [8]
-    unsigned long long *mask = (unsigned long long *)(red + 8); // [max_var * NWM]
-    int32_t *gv = (int32_t *)(mask + (size_t)P.max_var * NWM);  // [max_gl]
+    unsigned long long *mask = (unsigned long long *)(red + 8); // [max_var * nwm]
+    int32_t *gv = (int32_t *)(mask + (size_t)P.max_var * P.nwm);  // [max_gl]
     int32_t *gpos = gv + P.max_gl;                 // [max_gl]
     int32_t *gvl = gpos + P.max_gl;                // [max_var]
     int32_t *segof = gvl + P.max_var;              // [max_var]
@@ -193,7 +282,19 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
     int32_t *snext = pblk + P.max_pair;            // [nbdr_max + 1]
     int32_t *sh = snext + P.nbdr_max + 1;          // [32] scalars
 
-    double *vinv = scratch + (size_t)blockIdx.x * P.vinv_stride;   // packed inverse, 0-based bpk64
+    // packed inverse, 0-based bpk64
+    double *vinv;
+    if constexpr (VL) vinv = lds + P.vinv_lds;
+    else vinv = scratch + (size_t)blockIdx.x * P.vinv_stride;
+    const int nwm = P.nwm;
+    int2 *segfn = (int2 *)gp;                      // first variable and size of each segment's group (gp is done by then)
+    // pair (pj, pk), pj >= pk, of lane tid in the packed triangle
+    int pj = 1, pk = 1;
+    {
+        int rem = tid & 63;
+        while (rem >= pj) rem -= pj++;
+        pk = rem + 1;
+    }
 
     for (int64_t ri = blockIdx.x; ri < nb; ri += gridDim.x) {
         const int64_t r = ids[ri];
@@ -228,7 +329,7 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                 if (isv && pos < P.max_var) gvl[pos] = v;
                 nalg += __popcll(m);
             }
-            if (tid == 0) { sh[0] = nalg; sh[1] = 0; }
+            if (tid == 0) { sh[0] = nalg; sh[1] = 0; sh[7] = 0; }
         }
         __syncthreads();
         const int nalg = sh[0];
@@ -247,10 +348,19 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             int mx = 0;
             for (int j = 1; j <= nl; j++) mx = max(mx, R.widx[sl + j]);
             if (mx > 0) atomicMax(&sh[1], mx);
+            if (nl > 9 || nl + ng + 2 > 64) atomicOr(&sh[7], 1);
         }
         __syncthreads();
         const int nalc = sh[1];
         const int nmb = nalc - mbdr, mp1 = mbnd + 1;
+        // equations of at most 64 words and 9 locals, a band of at most 64 rows and 10 columns: one
+        // wavefront does the serial phases without workgroup barriers
+        const bool eq1 = sh[7] == 0, one = nmb <= 64 && mbnd <= 10;
+        const int tn = one ? 64 : BNT;
+        auto tsync = [&]() {
+            if (one) wave_sync();
+            else __syncthreads();
+        };
         if (nalg > P.max_var || nalc > NA || nalc <= 0 || nmb <= 0) {
             if (tid == 0) { out.status[r] = 9; out.chi2[r] = 0.0; out.ndf[r] = 0; }
             __syncthreads();
@@ -284,7 +394,31 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             if (tid == 0) sh[2] = 0;
             __syncthreads();
             // local normal equations into band / border storage, equations in order
-            for (int i = 0; i < neq; i++) {
+            auto put = [&](int ij, int ik, double val) {
+                const int J = max(ij, ik), K = min(ij, ik);
+                if (mside == 1) {
+                    if (K <= mbdr) vbdr[(K - 1) * nalc + J] += val;          // column K of the border
+                    else if (J - K <= mbnd) vbnd[(K - nb1) * mp1 + J - K + 1] += val;
+                    else sh[2] = 1;
+                } else {
+                    if (J > nmb) vbdr[(J - nb1) * nalc + K] += val;           // row J of the border
+                    else if (J - K <= mbnd) vbnd[(K - 1) * mp1 + J - K + 1] += val;
+                    else sh[2] = 1;
+                }
+            };
+            if (eq1 && tid < 64)
+                each_equation<T>(R, e0, neq, tid, [&](int i, const EqWords<T> &E) {
+                    const int npair = (E.nl * E.nl + E.nl) / 2;
+                    const bool rhs = tid >= 64 - E.nl;     // the last lanes: the right-hand side
+                    const int j = rhs ? 64 - tid : pj, k = pk;
+                    const int ij = __shfl(E.wx, j, 64), ik = __shfl(E.wx, k, 64);
+                    const double vj = lane_val(E.v, j), vk = lane_val(E.v, k);
+                    const double wght = lw[i];
+                    if (rhs) bl[ij] = bl[ij] + wght * rm[i] * vj;
+                    else if (tid < npair) put(ij, ik, wght * vj * vk);
+                    wave_sync();
+                });
+            for (int i = 0; i < (eq1 ? 0 : neq); i++) {
                 const int64_t sl = R.eq_sl[e0 + i];
                 const int nl = R.eq_n[e0 + i] & 0xffff;
                 const int npair = (nl * nl + nl) / 2;
@@ -302,45 +436,44 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                     int k = t - (j * j - j) / 2 + 1;
                     int ij = R.widx[sl + j], ik = R.widx[sl + k];
                     double val = wght * bval<T>(R, sl + j) * bval<T>(R, sl + k);
-                    int J = max(ij, ik), K = min(ij, ik);
-                    if (mside == 1) {
-                        if (K <= mbdr) vbdr[(K - 1) * nalc + J] += val;          // column K of the border
-                        else if (J - K <= mbnd) vbnd[(K - nb1) * mp1 + J - K + 1] += val;
-                        else sh[2] = 1;
-                    } else {
-                        if (J > nmb) vbdr[(J - nb1) * nalc + K] += val;           // row J of the border
-                        else if (J - K <= mbnd) vbnd[(K - 1) * mp1 + J - K + 1] += val;
-                        else sh[2] = 1;
-                    }
+                    put(ij, ik, val);
                 }
                 __syncthreads();
             }
+            __syncthreads();
             if (sh[2]) { status = 9; break; }   // element outside the detected structure
             // ---- sqmibb / sqmibb2: root-free band Cholesky (dbcdec) ----
             for (int i = tid; i < nmb; i += BNT) aux[i + 1] = 16.0 * vbnd[i * mp1 + 1];
             __syncthreads();
-            for (int i = 1; i <= nmb; i++) {
-                const int jm = min(mp1 - 1, nmb - i);
-                double piv = vbnd[(i - 1) * mp1 + 1];
-                piv = (piv + aux[i] != aux[i]) ? 1.0 / piv : 0.0;
-                // W(k, i+j) -= W(k+j, i) * rxw, rxw = W(j+1, i) * W(1, i); pairs (j, k) independent
-                const int nup = (jm * (jm + 1)) / 2;
-                double upd = 0.0;
-                int tgt = -1;
-                if (tid < nup) {
-                    int j = 1, rem = tid;
-                    while (rem >= jm + 1 - j) { rem -= jm + 1 - j; j++; }
-                    int k = rem + 1;
-                    double rxw = vbnd[(i - 1) * mp1 + j + 1] * piv;
-                    tgt = (i + j - 1) * mp1 + k;
-                    upd = vbnd[tgt] - vbnd[(i - 1) * mp1 + k + j] * rxw;
+            if (tid < tn) {
+                for (int i = 1; i <= nmb; i++) {
+                    const int jm = min(mp1 - 1, nmb - i);
+                    double piv = vbnd[(i - 1) * mp1 + 1];
+                    piv = (piv + aux[i] != aux[i]) ? 1.0 / piv : 0.0;
+                    // W(k, i+j) -= W(k+j, i) * rxw, rxw = W(j+1, i) * W(1, i); pairs (j, k) independent
+                    // (pair (pj, pk) of the triangle: j = pk, k + j = pj)
+                    int j = pk, kj = pj;
+                    if (!one) {
+                        kj = 1;
+                        int rem = tid;
+                        while (rem >= kj) rem -= kj++;
+                        j = rem + 1;
+                    }
+                    double upd = 0.0;
+                    int tgt = -1;
+                    if (kj <= jm) {
+                        const double rxw = vbnd[(i - 1) * mp1 + j + 1] * piv;
+                        tgt = (i + j - 1) * mp1 + kj - j + 1;
+                        upd = vbnd[tgt] - vbnd[(i - 1) * mp1 + kj + 1] * rxw;
+                    }
+                    tsync();
+                    if (tgt >= 0) vbnd[tgt] = upd;
+                    if (tid < jm) vbnd[(i - 1) * mp1 + tid + 2] = vbnd[(i - 1) * mp1 + tid + 2] * piv;
+                    if (tid == 0) vbnd[(i - 1) * mp1 + 1] = piv;
+                    tsync();
                 }
-                __syncthreads();
-                if (tgt >= 0) vbnd[tgt] = upd;
-                if (tid < jm) vbnd[(i - 1) * mp1 + tid + 2] = vbnd[(i - 1) * mp1 + tid + 2] * piv;
-                if (tid == 0) vbnd[(i - 1) * mp1 + 1] = piv;
-                __syncthreads();
             }
+            __syncthreads();
             // rank of the band part and its condition (inverted pivots, as sqmibb)
             if (tid == 0) {
                 int ok = 1;
@@ -534,7 +667,7 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                 bool st = (a < nalg) && (a == 0 || g != gprev);
                 unsigned long long m = __ballot(st);
                 int s = nseg + __popcll(m & ((2ull << tid) - 1ull)) - 1;
-                if (a < nalg) { segof[a] = s; if (st) seggr[s] = g; }
+                if (a < nalg) { segof[a] = s; if (st) { seggr[s] = g; segfn[s] = make_int2(M.gfirst[g], M.gfirst[g + 1] - M.gfirst[g]); } }
                 nseg += __popcll(m);
             }
             int npair = (nseg * nseg + nseg) / 2;
@@ -542,7 +675,7 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             for (int t = tid; t < npair; t += 64) pblk[t] = t < P.max_pair ? R.pair_blk[p0 + t] : -1;
         }
         if (o.icalcm == 1)
-            for (int t = tid; t < nalg * NWM; t += BNT) mask[t] = 0ull;
+            for (int t = tid; t < nalg * nwm; t += BNT) mask[t] = 0ull;
         __syncthreads();
         // ---- fourth loop: vector, counters, g g^T (4162-4201), support masks of G ----
         double s_chi = 0.0;
@@ -579,7 +712,7 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                         int aj = gpos[pj];
                         for (int l = 1; l <= nl; l++) {
                             int kk = R.widx[sl + l] - 1;
-                            atomicOr(&mask[aj * NWM + (kk >> 6)], 1ull << (kk & 63));
+                            atomicOr(&mask[aj * nwm + (kk >> 6)], 1ull << (kk & 63));
                         }
                         for (int k = 1; k <= j; k++) {
                             int pk_ = R.widx[sg + k];
@@ -587,8 +720,8 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                             if (vk > 0) {
                                 double val = dw1 * wght * gj * bval<T>(R, sg + k);
                                 int ak = gpos[pk_];
-                                if (vj >= vk) band_mat_add(M, vj, vk, val, segof, seggr, pblk, aj, ak);
-                                else band_mat_add(M, vk, vj, val, segof, seggr, pblk, ak, aj);
+                                if (vj >= vk) band_mat_add(M, vj, vk, val, segof, segfn, pblk, aj, ak);
+                                else band_mat_add(M, vk, vj, val, segof, segfn, pblk, ak, aj);
                             }
                         }
                     }
@@ -598,38 +731,51 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
         summ = block_sum(s_chi, red);
         if (o.icalcm == 1) {
             // ---- support classes: runs of globals with the same support of G ----
-            if (tid == 0) {
-                int ncls = 0, tot = 0, ok = 1;
-                for (int a = 0; a < nalg; a++) {
-                    bool same = a > 0;
-                    for (int w = 0; w < NWM && same; w++) same = mask[a * NWM + w] == mask[(a - 1) * NWM + w];
-                    if (!same) {
-                        int cnt = 0;
-                        for (int w = 0; w < NWM; w++) cnt += __popcll(mask[a * NWM + w]);
-                        cls0[ncls] = a;
-                        sptr[ncls] = tot;
-                        tot += cnt;
-                        ncls++;
+            // (one lane per global: sums over the earlier lanes give the offsets)
+            if (tid < 64) {
+                int ncls = 0, tot = 0, gt = 0, un = 0;
+                for (int base = 0; base < nalg; base += 64) {
+                    const int a = base + tid;
+                    bool start = a < nalg;
+                    int cnt = 0;
+                    if (a < nalg) {
+                        bool same = a > 0;
+                        for (int w = 0; w < nwm; w++) {
+                            const unsigned long long m = mask[a * nwm + w];
+                            cnt += __popcll(m);
+                            same = same && m == mask[(a - 1) * nwm + w];
+                        }
+                        start = !same;
                     }
-                    clsof[a] = ncls - 1;
+                    const unsigned long long m = __ballot(start);
+                    const int q = ncls + __popcll(m & ((2ull << tid) - 1ull)) - 1;
+                    int st = start ? cnt : 0, sg = cnt, su = start ? nalg - a : 0;
+                    for (int d = 1; d < 64; d <<= 1) {
+                        const int x = __shfl_up(st, d, 64), y = __shfl_up(sg, d, 64), z = __shfl_up(su, d, 64);
+                        if (tid >= d) { st += x; sg += y; su += z; }
+                    }
+                    if (a < nalg) {
+                        clsof[a] = q;
+                        gptr[a] = gt + sg - cnt;
+                        if (start) {
+                            cls0[q] = a;
+                            sptr[q] = tot + st - cnt;
+                            upre[q] = un + su - (nalg - a);
+                        }
+                    }
+                    ncls += __popcll(m);
+                    tot += __shfl(st, 63, 64);
+                    gt += __shfl(sg, 63, 64);
+                    un += __shfl(su, 63, 64);
                 }
-                cls0[ncls] = nalg;
-                sptr[ncls] = tot;
-                // G values: one row of |S| entries per global
-                int gt = 0;
-                for (int a = 0; a < nalg; a++) {
-                    gptr[a] = gt;
-                    int q = clsof[a];
-                    gt += sptr[q + 1] - sptr[q];
+                if (tid == 0) {
+                    cls0[ncls] = nalg;
+                    sptr[ncls] = tot;
+                    gptr[nalg] = gt;
+                    upre[ncls] = un;               // work units of the Schur update: (global a, class Q <= class(a))
+                    sh[5] = ncls;
+                    sh[6] = tot <= P.max_sup && gt <= P.max_sup;
                 }
-                gptr[nalg] = gt;
-                if (tot > P.max_sup || gt > P.max_sup) ok = 0;
-                // work units of the Schur update: (global a, class Q <= class(a))
-                int u = 0;
-                for (int q = 0; q < ncls; q++) { upre[q] = u; u += nalg - cls0[q]; }
-                upre[ncls] = u;
-                sh[5] = ncls;
-                sh[6] = ok;
             }
             __syncthreads();
             const int ncls = sh[5];
@@ -641,8 +787,8 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             // support lists (ascending local indices) and zeroed G rows
             for (int q = tid; q < ncls; q += BNT) {
                 int a = cls0[q], s = sptr[q];
-                for (int w = 0; w < NWM; w++) {
-                    unsigned long long m = mask[a * NWM + w];
+                for (int w = 0; w < nwm; w++) {
+                    unsigned long long m = mask[a * nwm + w];
                     while (m) {
                         int b = __ffsll((long long)m) - 1;
                         sidx[s++] = w * 64 + b + 1;
@@ -653,13 +799,19 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             for (int t = tid; t < gptr[nalg]; t += BNT) gval[t] = 0.0;
             __syncthreads();
             // G = sum over equations of sqrt(dw) w g l^T, equations in order (4206-4219)
-            for (int i = 0; i < neq; i++) {
+            auto slot_of = [&](int a, int kk) {
+                int pos = 0;
+                for (int w = 0; w < (kk >> 6); w++) pos += __popcll(mask[a * nwm + w]);
+                pos += __popcll(mask[a * nwm + (kk >> 6)] & ((1ull << (kk & 63)) - 1ull));
+                return &gval[gptr[a] + pos];
+            };
+            auto g_pairs = [&](int i, int t0, int nt) {
                 const int64_t sl = R.eq_sl[e0 + i];
                 const uint32_t en = R.eq_n[e0 + i];
                 const int nl = en & 0xffff, ng = en >> 16;
                 const int64_t sg = sl + nl + 1;
                 const double wght = lw[i];
-                for (int t = tid; t < ng * nl; t += BNT) {
+                for (int t = t0; t < ng * nl; t += nt) {
                     int j = t / nl + 1, k = t % nl + 1;
                     const int pj = R.widx[sg + j];
                     int a = gpos[pj];
@@ -675,11 +827,7 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                         if (x != k && R.widx[sl + x] == ik) { rep = true; own = own && x > k; }
                     // zero derivatives add nothing and are not part of the support masks
                     if (!own || (!rep && bval<T>(R, sg + j) == 0.0)) continue;
-                    const int kk = ik - 1;
-                    int pos = 0;
-                    for (int w = 0; w < (kk >> 6); w++) pos += __popcll(mask[a * NWM + w]);
-                    pos += __popcll(mask[a * NWM + (kk >> 6)] & ((1ull << (kk & 63)) - 1ull));
-                    double *ge = &gval[gptr[a] + pos];
+                    double *ge = slot_of(a, ik - 1);
                     if (!rep) {
                         *ge = *ge + dw2 * wght * bval<T>(R, sg + j) * bval<T>(R, sl + k);
                         continue;
@@ -697,6 +845,37 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                     }
                     if (any) *ge = v;
                 }
+            };
+            if (eq1 && tid < 64)
+                each_equation<T>(R, e0, neq, tid, [&](int i, const EqWords<T> &E) {
+                    if (E.ng == 0 || E.nl == 0) return;
+                    // a label or local index that comes twice in the equation: the general form
+                    bool dup = false;
+                    for (int x = 1; x < E.nl; x++)
+                        dup = dup || (tid > x && tid <= E.nl && E.wx == __builtin_amdgcn_readlane(E.wx, x));
+                    for (int x = E.nl + 2; x < E.nl + 1 + E.ng; x++)
+                        dup = dup || (tid > x && tid <= E.nl + 1 + E.ng && E.wx == __builtin_amdgcn_readlane(E.wx, x));
+                    if (__any(dup)) {
+                        g_pairs(i, tid, 64);
+                    } else {
+                        const double wght = lw[i];
+                        const int div = 65536 / E.nl + 1;
+                        for (int t = 0; t < E.ng * E.nl; t += 64) {
+                            const int tt = min(t + tid, E.ng * E.nl - 1);
+                            const int j = (tt * div) >> 16, k = tt - j * E.nl;
+                            const int pg = __shfl(E.wx, E.nl + 2 + j, 64), ik = __shfl(E.wx, 1 + k, 64);
+                            const double vj = lane_val(E.v, E.nl + 2 + j), vk = lane_val(E.v, 1 + k);
+                            const int a = gpos[pg];
+                            if (t + tid < E.ng * E.nl && a >= 0 && vj != 0.0) {
+                                double *ge = slot_of(a, ik - 1);
+                                *ge = *ge + dw2 * wght * vj * vk;
+                            }
+                        }
+                    }
+                    wave_sync();
+                });
+            for (int i = 0; i < (eq1 ? 0 : neq); i++) {
+                g_pairs(i, tid, BNT);
                 __syncthreads();
             }
             // ---- complete inverse of the local matrix (inv = 2) into vinv ----
@@ -705,41 +884,48 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
             // the mbnd columns to the right of j live in the LDS ring (slot = column mod mp1)
             const int n = nalc;
             const int nq = (mbdr * mbdr + mbdr) / 2;
-            for (int j = nmb; j >= 1; j--) {
-                double *colj = &ring[(j % mp1) * (NA + 1)];
-                const int kmax = min(nmb, j + mp1 - 1);
-                // off-diagonal entries of column j (rows i > j) from the columns to the right
-                for (int i = j + 1 + tid; i <= nmb; i += BNT) {
-                    double rxw = 0.0;
-                    for (int k = j + 1; k <= kmax; k++) {
-                        double vik = (k <= i) ? ring[(k % mp1) * (NA + 1) + i] : ring[(i % mp1) * (NA + 1) + k];
-                        rxw = rxw - vik * vbnd[(j - 1) * mp1 + 1 + k - j];
+            if (tid < tn) {
+                for (int j = nmb; j >= 1; j--) {
+                    double *colj = &ring[(j % mp1) * (NA + 1)];
+                    const int kmax = min(nmb, j + mp1 - 1);
+                    // off-diagonal entries of column j (rows i > j) from the columns to the right
+                    for (int i = j + 1 + tid; i <= nmb; i += tn) {
+                        double rxw = 0.0;
+                        for (int k = j + 1; k <= kmax; k++) {
+                            double vik = (k <= i) ? ring[(k % mp1) * (NA + 1) + i] : ring[(i % mp1) * (NA + 1) + k];
+                            rxw = rxw - vik * vbnd[(j - 1) * mp1 + 1 + k - j];
+                        }
+                        colj[i] = rxw;
+                        vinv[bpk64(bo + i, bo + j)] = rxw;
                     }
-                    colj[i] = rxw;
-                }
-                __syncthreads();
-                if (tid == 0) {
-                    double rxw = vbnd[(j - 1) * mp1 + 1];
-                    for (int k = j + 1; k <= kmax; k++) rxw = rxw - colj[k] * vbnd[(j - 1) * mp1 + 1 + k - j];
-                    colj[j] = rxw;
-                }
-                __syncthreads();
-                // store with the border correction sum_{ib,jb} VBK(ib,jb) AUX_ib(i) AUX_jb(j)
-                for (int i = j + tid; i <= nmb; i += BNT) {
-                    double v = colj[i];
-                    if (mbdr > 0) {
-                        for (int ib = 1; ib <= mbdr; ib++)
-                            for (int jb = 1; jb <= mbdr; jb++) {
-                                int ij = ib > jb ? ib : jb;
-                                ij = (ij * ij - ij) / 2 + (ib < jb ? ib : jb);
-                                const double ai = mside == 1 ? aux[nb1 + (ib - 1) * n + i - 1] : aux[(ib - 1) * n + i];
-                                const double aj = mside == 1 ? aux[nb1 + (jb - 1) * n + j - 1] : aux[(jb - 1) * n + j];
-                                v = v + vbk[ij] * ai * aj;
-                            }
+                    tsync();
+                    if (tid == 0) {
+                        double rxw = vbnd[(j - 1) * mp1 + 1];
+                        for (int k = j + 1; k <= kmax; k++) rxw = rxw - colj[k] * vbnd[(j - 1) * mp1 + 1 + k - j];
+                        colj[j] = rxw;
+                        vinv[bpk64(bo + j, bo + j)] = rxw;
                     }
-                    vinv[bpk64(bo + i, bo + j)] = v;
+                    tsync();
                 }
-                __syncthreads();
+            }
+            __threadfence_block();
+            __syncthreads();
+            // the border correction sum_{ib,jb} VBK(ib,jb) AUX_ib(i) AUX_jb(j)
+            for (int t = tid; mbdr > 0 && t < (nmb * nmb + nmb) / 2; t += BNT) {
+                int i = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f) + 1;
+                while ((i * i - i) / 2 > t) i--;
+                while ((i * i + i) / 2 <= t) i++;
+                const int j = t - (i * i - i) / 2 + 1;
+                double v = vinv[bpk64(bo + i, bo + j)];
+                for (int ib = 1; ib <= mbdr; ib++)
+                    for (int jb = 1; jb <= mbdr; jb++) {
+                        int ij = ib > jb ? ib : jb;
+                        ij = (ij * ij - ij) / 2 + (ib < jb ? ib : jb);
+                        const double ai = mside == 1 ? aux[nb1 + (ib - 1) * n + i - 1] : aux[(ib - 1) * n + i];
+                        const double aj = mside == 1 ? aux[nb1 + (jb - 1) * n + j - 1] : aux[(jb - 1) * n + j];
+                        v = v + vbk[ij] * ai * aj;
+                    }
+                vinv[bpk64(bo + i, bo + j)] = v;
             }
             // border rows: -sum_jb VBK(ib,jb) AUX_jb(i) against the band, VBK within the border
             for (int t = tid; t < mbdr * nmb; t += BNT) {
@@ -785,15 +971,19 @@ __global__ __launch_bounds__(BNT) void k_records_band(DevRecords R, DevModel M, 
                         const int k = sidx[sa0 + s];
                         const double gak = gval[gptr[a] + s];
 #pragma unroll
-                        for (int l = 0; l < QCH; l++)
-                            if (l0 + l < nq_) m[l] = m[l] + gak * vinv[bsym(k, sidx[sq0 + l0 + l])];
+                        for (int g = 0; g < QCH; g += 4)
+                            if (l0 + g < nq_) {            // four at a time (past the support: values that are not used)
+#pragma unroll
+                                for (int l = g; l < g + 4; l++)
+                                    m[l] = m[l] + gak * vinv[bsym(k, sidx[sq0 + min(l0 + l, nq_ - 1)])];
+                            }
                     }
                     for (int b = cls0[Q]; b <= bend; b++) {
                         double c = 0.0;
 #pragma unroll
                         for (int l = 0; l < QCH; l++)
                             if (l0 + l < nq_) c = c + m[l] * gval[gptr[b] + l0 + l];
-                        band_mat_add(M, gvl[a], gvl[b], -c, segof, seggr, pblk, a, b);
+                        band_mat_add(M, gvl[a], gvl[b], -c, segof, segfn, pblk, a, b);
                     }
                 }
             }
@@ -808,20 +998,16 @@ hipError_t launch_records_band(const DevRecords &R, const DevModel &M, const Pas
                                double *scratch, int grid, hipStream_t s)
 {
     if (nb <= 0) return hipSuccess;
-    if (P.bytes > 65536) {
-        hipError_t e = R.vf ? hipFuncSetAttribute((const void *)k_records_band<float>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, P.bytes)
-                            : hipFuncSetAttribute((const void *)k_records_band<double>,
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, P.bytes);
-        if (e != hipSuccess) return e;
-    }
-    if (R.vf)
-        hipLaunchKernelGGL(k_records_band<float>, dim3(grid), dim3(BNT), P.bytes, s, R, M, o, out, P, ids, nb, binfo,
-                           scratch);
-    else
-        hipLaunchKernelGGL(k_records_band<double>, dim3(grid), dim3(BNT), P.bytes, s, R, M, o, out, P, ids, nb, binfo,
-                           scratch);
-    return hipGetLastError();
+    auto run = [&](auto kernel) {
+        if (P.bytes > 65536) {
+            hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, P.bytes);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(BNT), P.bytes, s, R, M, o, out, P, ids, nb, binfo, scratch);
+        return hipGetLastError();
+    };
+    if (P.vinv_lds) return R.vf ? run(k_records_band<float, true>) : run(k_records_band<double, true>);
+    return R.vf ? run(k_records_band<float, false>) : run(k_records_band<double, false>);
 }
 
 int band_lds_bytes(BandPlan &P)
@@ -830,10 +1016,18 @@ int band_lds_bytes(BandPlan &P)
     size_t d = (size_t)P.max_gl + 4 * (size_t)P.max_eq + NA * P.mp1_max + 1 + (size_t)P.nbdr_max * NA + 1 +
                ((size_t)P.nbdr_max + 1) * NA + 1 + 2 * (NA + 1) + ((size_t)P.nbdr_max * P.nbdr_max + P.nbdr_max) / 2 + 1 +
                2 * ((size_t)P.nbdr_max + 1) + (size_t)P.mp1_max * (NA + 1) + P.max_sup + 8;
-    size_t u64 = (size_t)P.max_var * NWM;
+    P.nwm = (P.nalc_max + 63) / 64;
+    size_t u64 = (size_t)P.max_var * P.nwm;
     size_t i32 = 2 * (size_t)P.max_gl + 4 * (size_t)P.max_var + 4 * ((size_t)P.max_var + 1) + P.max_sup + P.max_pair +
                  P.nbdr_max + 1 + 32;
     size_t b = d * 8 + u64 * 8 + i32 * 4;
+    // the local inverse in LDS behind the rest where four workgroups still fit a CU, else in memory
+    P.vinv_lds = 0;
+    const size_t at = (b + 7) / 8;
+    if ((at + (size_t)P.vinv_stride) * 8 <= 40 * 1024) {
+        P.vinv_lds = (int32_t)at;
+        b = (at + (size_t)P.vinv_stride) * 8;
+    }
     P.bytes = (int)b;
     return P.bytes;
 }

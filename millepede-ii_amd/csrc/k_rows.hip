@@ -347,13 +347,18 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_incidence(int64_t q0, int64
     }
 }
 
-// first position of every key (sorted), keys 0 .. nk
+// first position of every key (sorted), keys 0 .. nk: a search per key, since a thread that filled a
+// gap between two keys took as long as the gap (few records in row form, 200,000 blocks: 45 ms)
 __global__ void k_rows_ptr(int64_t n, const uint32_t *key, int64_t nk, uint32_t *ptr)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t lo = i == 0 ? -1 : (int64_t)key[i - 1];
-        const int64_t hi = i == n ? nk : (int64_t)key[i];
-        for (int64_t k = lo + 1; k <= hi; k++) ptr[k] = (uint32_t)i;
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k <= nk; k += (int64_t)gridDim.x * blockDim.x) {
+        int64_t lo = 0, hi = n;                  // keys below lo are < k, from hi on >= k
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if ((int64_t)key[mid] < k) lo = mid + 1;
+            else hi = mid;
+        }
+        ptr[k] = (uint32_t)lo;
     }
 }
 
@@ -1198,7 +1203,7 @@ void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, in
         if (B.npair > 0)
             HIPCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, bytes, k0.p, k1.p, v0.p, S.src.p + B.inc0, (int)B.npair, 0, bits,
                                                       s));
-        hipLaunchKernelGGL(k_rows_ptr, dim3(rows_grid(B.npair + 1, 256)), dim3(256), 0, s, B.npair, k1.p, nblock,
+        hipLaunchKernelGGL(k_rows_ptr, dim3(rows_grid(nblock + 1, 256)), dim3(256), 0, s, B.npair, k1.p, nblock,
                            S.ptr.p + b * (nblock + 1));
         HIPCHK(hipGetLastError());
     }

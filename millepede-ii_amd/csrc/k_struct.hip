@@ -571,13 +571,18 @@ __global__ void k_ccol_fill(int64_t n, const int32_t *blk, const int64_t *boff, 
         ccfn[2 * q + 1] = gfirst[g + 1] - gfirst[g];
     }
 }
-// pointers of sorted keys: ptr[k] = first position with key >= k, k = 0 .. nk
+// pointers of sorted keys: ptr[k] = first position with key >= k, k = 0 .. nk (a search per key: filling
+// the gaps between the keys takes one thread as long as its gap)
 __global__ void k_key_ptr(int64_t n, const uint32_t *key, int64_t nk, int64_t *ptr)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t lo = i == 0 ? -1 : (int64_t)key[i - 1];
-        const int64_t hi = i == n ? nk : (int64_t)key[i];
-        for (int64_t k = lo + 1; k <= hi; k++) ptr[k] = i;
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k <= nk; k += (int64_t)gridDim.x * blockDim.x) {
+        int64_t lo = 0, hi = n;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if ((int64_t)key[mid] < k) lo = mid + 1;
+            else hi = mid;
+        }
+        ptr[k] = lo;
     }
 }
 __global__ void k_npair(int64_t nrec, const int32_t *nseg, int64_t *np)
@@ -1061,7 +1066,7 @@ void st_blocks(PairMap &pm, int32_t ngroup, const int32_t *gfirst, const std::ve
         sort_pairs(k0.p, k1.p, v0.p, v1.p, nb, key_bits(ng), s, tmp);
     }
     B.ccol_ptr.alloc(ng + 1);
-    hipLaunchKernelGGL(k_key_ptr, dim3(grid_for(noff + 1, 256)), dim3(256), 0, s, noff, k1.p, ng, B.ccol_ptr.p);
+    hipLaunchKernelGGL(k_key_ptr, dim3(grid_for(ng + 1, 256)), dim3(256), 0, s, noff, k1.p, ng, B.ccol_ptr.p);
     B.ncc = noff;
     B.cc_off.alloc(std::max<int64_t>(noff, 1));
     B.cc_fn.alloc(std::max<int64_t>(2 * noff, 1));
@@ -1211,7 +1216,7 @@ void st_incidence(const StructIn &in, const DBuf<int64_t> &rec_gl, const DBuf<in
                            gl_tix.p, var, group_of, rec_pb.p, pair_blk.p, rec_cb.p, pos.p, k0.p, v0.p);
     HIPCHK(hipGetLastError());
     if (n > 0) sort_pairs(k0.p, k1.p, v0.p, src, n, key_bits(nblock), s, tmp);
-    hipLaunchKernelGGL(k_key_ptr, dim3(grid_for(n + 1, 256)), dim3(256), 0, s, n, k1.p, nblock, ptr);
+    hipLaunchKernelGGL(k_key_ptr, dim3(grid_for(nblock + 1, 256)), dim3(256), 0, s, n, k1.p, nblock, ptr);
     HIPCHK(hipStreamSynchronize(s));
 }
 

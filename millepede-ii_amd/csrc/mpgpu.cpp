@@ -1250,7 +1250,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         band_lds_bytes(B);
         if (B.bytes > 160 * 1024)
             throw MpError(30, "record too large for the bordered-band kernel (LDS " + std::to_string(B.bytes) + " bytes)");
-        const int per_cu = std::max(1, std::min(8, (160 * 1024) / B.bytes));
+        const int per_cu = std::max(1, std::min(4, (160 * 1024) / B.bytes));
         c->band_grid = (int)std::min<int64_t>(c->nband, 256 * per_cu);
     }
 

@@ -121,6 +121,8 @@ struct LdsPlan {
 struct BandPlan {
     int32_t max_gl, max_eq, nalc_max, max_var, max_pair, mp1_max, nbdr_max, max_sup;
     int64_t vinv_stride;     // doubles of global scratch per workgroup (packed local inverse)
+    int32_t nwm;             // 64-bit words of a local-parameter support mask (nalc_max <= 256)
+    int32_t vinv_lds;        // offset of the packed local inverse in LDS (doubles; 0: it is in scratch)
     int32_t bytes;
 };
 
