@@ -33,27 +33,30 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def workload_bytes(rp):
-    """Algorithmic bytes of one pass: per record the Mille record itself (4 + 8 nw bytes for
-    FP32 payload) plus one FP64 read-modify-write (16 B) per updated matrix element of the
-    record's nalg(nalg+1)/2 triangle and per updated vector element.  With this generator
-    every hit adds 18 words (two measurements of 9 words) and 6 globals."""
+def workload_bytes(rp, stored):
+    """Bytes that the two kernels of a pass have to move, and the mean number of variable parameters
+    per record.  With this generator every hit adds 18 words (two measurements of 9 words), 6 globals
+    and one unit (the pair of measurements of one module: 128 B and 32 B of vector values).
+    k_rows_pass: the Mille record (4 + 8 nw bytes for FP32 payload) read, its units written;
+    k_rows_gather: the units and the lists (8 B per pair of a record's units) read once, every stored
+    matrix word read and written."""
     nw = np.diff(rp)
     hits = (nw - 1) // 18
-    nalg = 6 * hits
-    return float(np.sum(4 + 8 * nw + 16 * (nalg * (nalg + 1) // 2 + nalg))), float(np.mean(nalg))
+    rec = float(np.sum(4 + 8 * nw + 160 * hits))
+    gather = float(np.sum(160 * hits + 8 * (hits * (hits + 1) // 2))) + 16.0 * stored
+    return rec, gather, float(np.mean(6 * hits))
 
 
 def committed_traffic():
-    """HBM bytes per k_records launch from the committed rocprofv3 counter summary (FETCH_SIZE and
+    """HBM bytes per launch of the dominant kernel (k_rows_gather) from the committed rocprofv3 counter summary (FETCH_SIZE and
     WRITE_SIZE per dispatch, each scaled by the same counter's reading for a copy of known size);
     None when no summary is present."""
-    path = os.path.join(ROOT, "profiles", "k_records_pixel2M_traffic.txt")
+    path = os.path.join(ROOT, "profiles", "records_pixel2M_traffic.txt")
     if not os.path.exists(path):
         return None
     for line in open(path):
         if line.startswith("traffic_bytes_per_launch:"):
-            return {"bytes_per_launch": float(line.split(":", 1)[1]), "source": "profiles/k_records_pixel2M_traffic.txt"}
+            return {"bytes_per_launch": float(line.split(":", 1)[1]), "source": "profiles/records_pixel2M_traffic.txt"}
     return None
 
 
@@ -283,7 +286,7 @@ def main():
         gath_ms.append(st["ms_gather"])
         gath_launches.append(st["n_gather"])
         log(f"step {k}: {times[-1] * 1e3:.2f} ms wall, record loop {st['ms_kernel']:.2f} ms "
-            f"(k_records {st['ms_records']:.2f} ms in {st['n_records']}, gather {st['ms_gather']:.2f} ms)")
+            f"(records {st['ms_records']:.2f} ms in {st['n_records']}, gather {st['ms_gather']:.2f} ms)")
     tot = sum(times)
     nrec = len(rp) - 1
     value = nrec * args.steps / tot
@@ -298,21 +301,22 @@ def main():
                       "records": nrec, "ntot": ntot, "nvar": nvar, "ncon": ncon,
                       "stored_matrix_words": info["stored"], "structure_s": t_struct}}
 
-    # roofline of the dominant kernel (k_records): algorithmic bytes per launch over its average
-    # launch duration, both from the timed steps (HIP events around every launch, on the
-    # library's stream)
-    abytes, mean_nalg = workload_bytes(rp)
-    nl = sum(recs_launches)
-    kavg = sum(recs_ms) / max(nl, 1) / 1e3
-    per_launch = abytes * args.steps / max(nl, 1)
-    achieved = per_launch / kavg / 1e9
+    # roofline of the dominant kernel (k_rows_gather, the launches of one gather together) and of the
+    # record kernel: the bytes they have to move over their average durations, from the timed steps
+    # (HIP events around the launches, on the library's stream)
+    rec_bytes, gather_bytes, mean_nalg = workload_bytes(rp, info["stored"])
+    nl, ngl = max(sum(recs_launches), 1), max(sum(gath_launches), 1)
+    kavg, gavg = sum(recs_ms) / nl / 1e3, sum(gath_ms) / ngl / 1e3
+    per_launch = gather_bytes * args.steps / ngl
+    achieved = per_launch / max(gavg, 1e-9) / 1e9
     traffic = committed_traffic()
     out["roofline"] = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                        "frac": achieved / HBM_PEAK_GBS,
                        "traffic": traffic["bytes_per_launch"] if traffic else None,
-                       "kernel": "k_records<float>", "kernel_ms": kavg * 1e3, "launches_per_step": nl / args.steps,
+                       "kernel": "k_rows_gather<float>", "kernel_ms": gavg * 1e3, "launches_per_step": ngl / args.steps,
                        "algorithmic_bytes_per_launch": per_launch, "mean_nalg": mean_nalg,
-                       "gather_ms_per_launch": sum(gath_ms) / max(sum(gath_launches), 1),
+                       "record_kernel": "k_rows_pass<float>", "record_kernel_ms": kavg * 1e3,
+                       "record_kernel_achieved": rec_bytes * args.steps / nl / max(kavg, 1e-9) / 1e9,
                        "traffic_source": traffic["source"] if traffic else None}
     out["spmv_autotuner"] = P.tuning()
     lab, var, cnt, gsl = P.labels()

@@ -1,7 +1,8 @@
 // Record-loop kernel: one workgroup of RT threads (RW wavefronts) per Mille record.
 //
 // Restates loopbf (src/pede.f90:3387-4442) for records whose local fit takes the full
-// (non-banded) path; records with bordered-band structure go to k_records_band.  Residuals
+// (non-banded) path and that have no row form; records in row form go to k_rows_pass, records with
+// bordered-band structure to k_records_band.  Residuals
 // after the current global parameters, local normal equations,
 // symmetric Gauss-Jordan inversion with diagonal pivoting (sqminv, src/mpnum.f90:97-213),
 // chi^2 / down-weighting / reject logic, then the "Millepede" update of the global system:
