@@ -13,10 +13,18 @@
 //    operation order of sqmibb, so rank and condition decisions are pede's;
 //  * the complete inverse (inv = 2) is formed column by column from the right with the dbcinv
 //    recursion (the entries of a column need only the mbnd columns to its right, held in an
-//    LDS ring), plus the border corrections, into a per-workgroup global scratch area;
+//    LDS ring), plus the border corrections, into LDS where it fits beside the rest, else into a
+//    per-workgroup global scratch area;
 //  * G Gamma^-1 G^T (dbavats order, src/mpnum.f90:1470-1528) uses support classes: runs of
 //    record globals whose rows of G have the same local-parameter support share the same
 //    block of Gamma^-1, so each matrix element costs |S| FMAs and one FP64 atomic.
+//
+// Chains of dependent steps bound it (equation after equation, column after column), so one
+// wavefront walks the short ones with LDS order instead of workgroup barriers and with the words of
+// the next four equations in flight, and as many records as possible are in flight beside each
+// other: 128 registers for four workgroups a CU, though some values spill (three without spills: 8.4
+// against 5.4 ms), and a grid of what is resident.  20,000 broken-lines tracks of up to 44 local
+// parameters: pass 14.8 -> 5.4 ms, without the matrix 4.2 -> 2.1 ms.
 #include "mpgpu_device.h"
 #include <float.h>
 
@@ -1022,6 +1030,7 @@ int band_lds_bytes(BandPlan &P)
                  P.nbdr_max + 1 + 32;
     size_t b = d * 8 + u64 * 8 + i32 * 4;
     // the local inverse in LDS behind the rest where four workgroups still fit a CU, else in memory
+    // (fewer workgroups cost more than its latency)
     P.vinv_lds = 0;
     const size_t at = (b + 7) / 8;
     if ((at + (size_t)P.vinv_stride) * 8 <= 40 * 1024) {
