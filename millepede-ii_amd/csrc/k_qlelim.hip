@@ -115,25 +115,29 @@ __global__ void k_ql_band(int32_t nfit, int32_t mb, const int32_t *india, const 
     band[india[i] - nb + j] += corr;
 }
 
-// w_k = v_k . x for every reflector, x zero from index nx on
+// k_ql_vtx for one column that is zero from index nx on, every sum in k_ql_vtx's order
 __global__ __launch_bounds__(QTPB) void k_ql_vtx_n(int32_t m, int32_t nx, const int64_t *rf_ptr, const int32_t *rf_lo,
                                                    const int32_t *rf_kn, const double *rf_val, const double *rf_vk,
                                                    const double *x, double *w)
 {
-    __shared__ double red[QTPB / 64];
-    const int k = blockIdx.x;
+    __shared__ double red[QTPB];
+    const int k = blockIdx.x, t = threadIdx.x;
     const int64_t p0 = rf_ptr[k];
     const int32_t lo = rf_lo[k], len = min((int32_t)(rf_ptr[k + 1] - p0), nx - lo), kn = rf_kn[k];
     double s = 0.0;
-    for (int32_t q = threadIdx.x; q < len; q += QTPB) s += rf_val[p0 + q] * x[lo + q];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    for (int32_t q = t; q < len; q += QTPB) s += rf_val[p0 + q] * x[lo + q];
+    red[t] = s;
     __syncthreads();
-    if (threadIdx.x == 0)
-        w[k] = (((red[0] + red[1]) + (red[2] + red[3]))) + (kn < nx ? rf_vk[k] * x[kn] : 0.0);
+    if (t < 128) red[t] += red[t + 128];
+    __syncthreads();
+    if (t >= 64) return;
+    s = red[t] + red[t + 64];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (t == 0) w[k] = fma(rf_vk[k], kn < nx ? x[kn] : 0.0, s);
 }
-// y_p = x_p - sum_k v_k[p] u_k for p < ny, with u = T w or T^T w (trans) formed by every workgroup:
-// m^2/2 products each, so for few constraints only (l_ql_op); four threads share a u_i
+// k_ql_tmul and k_ql_xmvu in one launch, sums in their order: y_p = x_p - sum_k v_k[p] u_k for
+// p < ny, x zero from index nx on; every workgroup forms u by itself (m^2/2 products), so for few
+// constraints only (op_dev)
 __global__ __launch_bounds__(QTPB) void k_ql_out(int32_t m, int32_t nx, int32_t ny, const double *T, int trans, const double *w,
                                                  const int64_t *tr_ptr, const int32_t *tr_k, const double *tr_v, const double *x,
                                                  double *y)
@@ -142,18 +146,13 @@ __global__ __launch_bounds__(QTPB) void k_ql_out(int32_t m, int32_t nx, int32_t 
     const int t = threadIdx.x;
     if (t < m) sw[t] = w[t];
     __syncthreads();
-    for (int i0 = 0; i0 < m; i0 += QTPB / 4) {
-        const int i = i0 + (t >> 2);
+    if (t < m) {
         double s = 0.0;
-        if (i < m) {
-            if (trans)
-                for (int j = i + (t & 3); j < m; j += 4) s += T[(int64_t)i * m + j] * sw[j];
-            else
-                for (int j = t & 3; j <= i; j += 4) s += T[(int64_t)j * m + i] * sw[j];
-        }
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        if (i < m && (t & 3) == 0) su[i] = s;
+        if (trans)
+            for (int j = t; j < m; j++) s += T[(int64_t)t * m + j] * sw[j];
+        else
+            for (int j = 0; j <= t; j++) s += T[(int64_t)j * m + t] * sw[j];
+        su[t] = s;
     }
     __syncthreads();
     const int p = blockIdx.x * QTPB + t;
@@ -162,12 +161,6 @@ __global__ __launch_bounds__(QTPB) void k_ql_out(int32_t m, int32_t nx, int32_t 
     for (int64_t q = tr_ptr[p]; q < tr_ptr[p + 1]; q++) s += tr_v[q] * su[tr_k[q]];
     y[p] = (p < nx ? x[p] : 0.0) - s;
 }
-__global__ void k_ql_copy(int32_t n, const double *x, double *y)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < n) y[p] = x[p];
-}
-
 static inline unsigned qblk(int64_t n) { return (unsigned)((n + QTPB - 1) / QTPB < 1 ? 1 : (n + QTPB - 1) / QTPB); }
 
 void l_ql_apply(const QlDev &q, int trans, double *x, hipStream_t s)
@@ -177,23 +170,14 @@ void l_ql_apply(const QlDev &q, int trans, double *x, hipStream_t s)
     hipLaunchKernelGGL(k_ql_tmul, dim3(qblk(q.m)), dim3(QTPB), 0, s, q.m, q.T, trans, q.w, q.u);
     hipLaunchKernelGGL(k_ql_xmvu, dim3(qblk(q.n)), dim3(QTPB), 0, s, q.n, q.tr_ptr, q.tr_k, q.tr_v, q.u, x);
 }
-// y (first ny values) = Q x (trans 0) or Q^T x (1), x zero from index nx on, in two launches while
-// the constraints are few; y must not be x
+bool ql_few(const QlDev &q) { return q.m <= QL_FEW; }
+// y (first ny values) = Q x (trans 0) or Q^T x (1), x zero from index nx on, in two launches and bit
+// for bit as l_ql_apply; ql_few only, y must not be x.  An iteration of MINRES for 60 constraints and
+// 5,280 parameters with two of them: 140 us with l_ql_pad, l_ql_apply and a copy, 130 with these.
 void l_ql_op(const QlDev &q, int trans, int32_t nx, const double *x, double *y, int32_t ny, hipStream_t s)
 {
-    if (q.m <= QL_FEW) {
-        hipLaunchKernelGGL(k_ql_vtx_n, dim3(q.m), dim3(QTPB), 0, s, q.m, nx, q.rf_ptr, q.rf_lo, q.rf_kn, q.rf_val, q.rf_vk, x, q.w);
-        hipLaunchKernelGGL(k_ql_out, dim3(qblk(ny)), dim3(QTPB), 0, s, q.m, nx, ny, q.T, trans, q.w, q.tr_ptr, q.tr_k, q.tr_v, x, y);
-        return;
-    }
-    if (ny == q.n) {
-        l_ql_pad(nx, q.n, x, y, s);
-        l_ql_apply(q, trans, y, s);
-    } else {
-        // x is the caller's work vector of n values
-        l_ql_apply(q, trans, const_cast<double *>(x), s);
-        hipLaunchKernelGGL(k_ql_copy, dim3(qblk(ny)), dim3(QTPB), 0, s, ny, x, y);
-    }
+    hipLaunchKernelGGL(k_ql_vtx_n, dim3(q.m), dim3(QTPB), 0, s, q.m, nx, q.rf_ptr, q.rf_lo, q.rf_kn, q.rf_val, q.rf_vk, x, q.w);
+    hipLaunchKernelGGL(k_ql_out, dim3(qblk(ny)), dim3(QTPB), 0, s, q.m, nx, ny, q.T, trans, q.w, q.tr_ptr, q.tr_k, q.tr_v, x, y);
 }
 void l_ql_pad(int32_t nfit, int32_t n, const double *x, double *e, hipStream_t s)
 {

@@ -1118,7 +1118,7 @@ __global__ void k_part_fill(int32_t ngroup, int64_t npart, const int64_t *brow, 
         part[p] = P;
     }
 }
-int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff,
+int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff, bool whole,
                      DBuf<RowPart> &part, DBuf<int64_t> &ptr, hipStream_t s)
 {
     // A wavefront that takes a whole row is as slow as its row is long, and the rows of a small
@@ -1126,7 +1126,7 @@ int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const 
     // more than 8,192 (8 wavefronts a SIMD), up to whole rows.  Measured per product: 4,000 groups of
     // 6, 673,083 blocks (194 MB), rows pass 50 us by whole rows, 38 us (5.1 TB/s) in parts of 64, the
     // same from 32 to 96 and 58 us in parts of 8; 1,000 groups 19.7 -> 9.9 us (16: 10.6, 96: 11.5).
-    const int64_t C = std::max<int64_t>(64, (nblock / 8192 + 7) / 8 * 8);
+    const int64_t C = whole ? (int64_t)1 << 40 : std::max<int64_t>(64, (nblock / 8192 + 7) / 8 * 8);
     const int64_t npart = ngroup + nblock / C;
     DBuf<int64_t> cnt;
     DBuf<uint8_t> tmp;

@@ -97,7 +97,13 @@ struct mpgpu_ctx {
     std::vector<double> crhs;
     std::vector<std::vector<std::pair<int32_t, double>>> con_tot; // (total index, factor) per constraint
     // constraint elimination (the MINRES methods without 'withmultipliers'): QL decomposition of
-    // the constraint matrix; the solve works on the first nfit components of Q^T x
+    // the constraint matrix; the solve works on the first nfit components of Q^T x.
+    // These solves converge slowly (2,000 to 2,700 iterations for 20 layers of 40 to 50 modules) and
+    // may end at the iteration limit.  What an unfinished iteration returns depends on the order of
+    // every sum: another order of the pass's, the product's or the preconditioner's alone moves the
+    // solution at the limit by up to 3e-3, finished solves by 1e-5 or less.  So with group blocks all of
+    // them have one fixed order: every record by the record kernel, whole block rows in the product,
+    // band solves by substitution, reflections summed as l_ql_apply's.
     bool elim = false;
     int32_t nfit = 0;
     std::unique_ptr<QlElim> ql;
@@ -1096,7 +1102,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     for (int32_t x : ngl_rec) max_ngl_all = std::max(max_ngl_all, x);
     // the pairs of groups that records couple: the blocks of group-block storage, and with full
     // storage those that the records in row form are gathered by (a bitmap of up to 256 MB)
-    const bool try_rows = c->opt.monitor == 0 && nrec > 0 && (sparse || c->ngroup <= 65536);
+    const bool try_rows = c->opt.monitor == 0 && nrec > 0 && (sparse ? !c->elim : c->ngroup <= 65536);
     st_record_stats(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, c->ngroup, max_ngl_all,
                     sparse || try_rows, pm, rst, cnt_r, d_rst, s);
     const int32_t *st_nv = rst.data(), *st_nseg = rst.data() + nrec, *st_nalc = rst.data() + 2 * nrec,
@@ -1408,7 +1414,8 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
             // transposed products of the blocks, and a spare slot per lane for the uniform kernel
             // and the sums of the row parts
             const int64_t ntb = c->plan.max_grp * std::max<int64_t>(1, c->nblock) + 64;
-            c->parts.n = st_row_parts(c->ngroup, c->nblock, c->d_brow.p, c->d_bcol.p, c->d_boff.p, c->d_bpart, c->d_part_ptr, s);
+            c->parts.n = st_row_parts(c->ngroup, c->nblock, c->d_brow.p, c->d_bcol.p, c->d_boff.p, c->elim, c->d_bpart,
+                                      c->d_part_ptr, s);
             c->d_tb.alloc((size_t)(ntb + 8 * c->parts.n));
             c->parts.part = c->d_bpart.p;
             c->parts.ptr = c->d_part_ptr.p;
@@ -1944,9 +1951,17 @@ void op_dev(mpgpu_ctx *c, ElimWork &E, const double *x, double *y)
     if (!c->elim) { avprod_dev(c, x, y); return; }
     hipStream_t s = c->stream;
     const int32_t nv = c->nvar, nf = c->nfit;
-    l_ql_op(c->ql->dev, 0, nf, x, E.e.p, nv, s);
+    if (ql_few(c->ql->dev)) {
+        l_ql_op(c->ql->dev, 0, nf, x, E.e.p, nv, s);
+        avprod_dev(c, E.e.p, E.f.p);
+        l_ql_op(c->ql->dev, 1, nv, E.f.p, y, nf, s);
+        return;
+    }
+    l_ql_pad(nf, nv, x, E.e.p, s);
+    l_ql_apply(c->ql->dev, 0, E.e.p, s);
     avprod_dev(c, E.e.p, E.f.p);
-    l_ql_op(c->ql->dev, 1, nv, E.f.p, y, nf, s);
+    l_ql_apply(c->ql->dev, 1, E.f.p, s);
+    l_copy(nf, E.f.p, y, s);
 }
 
 double dot_dev(mpgpu_ctx *c, int64_t n, const double *a, const double *b)
@@ -2094,7 +2109,7 @@ void setup_precond(mpgpu_ctx *c, Precond &P)
         P.Sb.alloc((size_t)P.n * P.w);
         P.tbuf.alloc((size_t)nch * P.w);
         P.dtmp.alloc(std::max(1, P.m));
-        P.sub = bp_usable(P.n, P.m, P.w);
+        P.sub = !c->elim && bp_usable(P.n, P.m, P.w);      // (mpgpu_ctx::elim)
         if (P.sub) {
             P.F.alloc((size_t)bp_sub_elems(P.n));
             P.B.alloc((size_t)bp_sub_elems(P.n));

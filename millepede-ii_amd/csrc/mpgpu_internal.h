@@ -344,8 +344,9 @@ struct BlockDev {
     DBuf<int64_t> brow, boff, ccol_ptr, cc_off;
     DBuf<int32_t> brg, bcol, bcf, cc_fn, cc_blk;
 };
-// parts of the block rows for the block product (groups <= 8): returns the entries of part
-int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff,
+// parts of the block rows for the block product (groups <= 8; whole: one part a row): returns the
+// entries of part
+int64_t st_row_parts(int32_t ngroup, int64_t nblock, const int64_t *brow, const int32_t *bcol, const int64_t *boff, bool whole,
                      DBuf<RowPart> &part, DBuf<int64_t> &ptr, hipStream_t s);
 // equation tables of the records (decodeNextMeasurement): fills in.neq, in.rec_eq, in.eq_sl,
 // in.eq_n; error 20 names the first record that breaks the format
@@ -475,6 +476,7 @@ struct QlElim {
     void wy();
 };
 void l_ql_apply(const QlDev &q, int trans, double *x, hipStream_t s);   // x <- Q x (0) or Q^T x (1)
+bool ql_few(const QlDev &q);                 // few enough constraints for l_ql_op
 void l_ql_op(const QlDev &q, int trans, int32_t nx, const double *x, double *y, int32_t ny, hipStream_t s);
 void l_ql_pad(int32_t nfit, int32_t n, const double *x, double *e, hipStream_t s);
 void l_ql_vtx_cols(const QlDev &q, const double *x, int64_t ldx, int32_t ncols, double *w, int64_t ldw, hipStream_t s);
