@@ -347,9 +347,10 @@ void l_bp_build(int n, int m, int w, const double *c, const int *india, const do
 #undef BP_F
     if (m > 0) {
         const int lds = (m * m + m) / 2 * 8;
-        if (lds > 65536) (void)hipFuncSetAttribute((const void *)k_bp_hinv, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (lds > 65536) HIPCHK(hipFuncSetAttribute((const void *)k_bp_hinv, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         hipLaunchKernelGGL(k_bp_hinv, dim3(m), dim3(64), lds, s, m, h, hinv);
     }
+    HIPCHK(hipGetLastError());
 }
 
 // y = M^-1 x up to the backward correction (t: the carried boundary values), which the caller's next
