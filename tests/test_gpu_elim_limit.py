@@ -9,6 +9,8 @@ import numpy as np
 import pytest
 
 import mpgpu
+from helpers import packed_to_dense
+from test_gpu_parity import _dense_constraints, _pede
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "minres_elim_limit.txt")
@@ -38,4 +40,31 @@ def test_solution_at_the_iteration_limit():
     assert np.linalg.norm(x[at] - gold) <= 1e-10 * np.linalg.norm(gold)
     y, _ = P.solve()
     assert np.array_equal(x, y)
+    P.close()
+
+
+@pytest.mark.parametrize("ncon", [127, 128, 129, 132])
+def test_many_eliminated_constraints(ncon):
+    """Around 128 constraints, where the reflections go from two launches each to four: against the
+    dense KKT solve of the same matrix, the bars of test_minres_elimination."""
+    nl, nx, ny = 44, 2, 1
+    rp, ii, gg, _ = mpgpu.pixel_records(47, nl, nx, ny, 3000, 20, nl + 2, wx=10.0, wy=20.0)
+    weak = mpgpu.pixel_weak_labels(nl, nx, ny)
+    cons = mpgpu.pixel_constraints(nl, nx, ny)[:ncon]
+    cons = [(2e-3 * (j % 7), s, l, f) for j, (_, s, l, f) in enumerate(cons)]
+    P = _pede(rp, ii, gg, weak, mpgpu.pixel_presigma(weak), cons, matsto=mpgpu.SPARSE, metsol=mpgpu.MINRES, mreqenf=5,
+              mcount=1, mbandw=6, mrestl=1e-12, itnlim=5000, withmultipliers=0)
+    assert P.ncon == 0 and P.nall == P.nvar
+    P.loopn()
+    x, st = P.solve()
+    A = packed_to_dense(P.matrix_packed(), P.nvar)
+    b, _ = P.vector()
+    C, d = _dense_constraints(P, cons)
+    assert C.shape[0] == ncon
+    K = np.block([[A, C.T], [C, np.zeros((ncon, ncon))]])
+    xr = np.linalg.solve(K, np.concatenate([b, d]))[:P.nvar]
+    sig = np.sqrt(np.abs(np.diag(np.linalg.inv(K))[:P.nvar]))
+    assert st["istop"] in (1, 2)
+    assert np.abs(C @ x - d).max() < 1e-10 * max(1.0, np.abs(C).max() * np.abs(x).max())
+    assert np.max(np.abs(x - xr) / sig) < 1e-4
     P.close()
