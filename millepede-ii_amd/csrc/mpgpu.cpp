@@ -193,12 +193,14 @@ DevStore &dev_store()
     static DevStore *st = new DevStore;      // never destroyed: contexts may end after static objects
     return *st;
 }
-// sizes are rounded up to an eighth of their power of two (at least 256 bytes)
-size_t size_class(size_t b)
+// sizes of blocks that may be kept are rounded up to an eighth of their power of two (at least 256
+// bytes), the others to 256 bytes
+size_t block_bytes(size_t b)
 {
     size_t q = 256;
     while (q * 16 <= b) q *= 2;
-    return (b + q - 1) / q * q;
+    const size_t c = (b + q - 1) / q * q;
+    return c <= CACHE_BLOCK ? c : (b + 255) / 256 * 256;
 }
 void *store_take(size_t key)
 {
@@ -213,6 +215,17 @@ void *store_take(size_t key)
 }
 } // namespace
 
+size_t mpgpu::dev_store_kept()
+{
+    DevStore &S = dev_store();
+    std::lock_guard<std::mutex> g(S.m);
+    return S.held;
+}
+
+DevCache::DevCache(hipStream_t st, int dev) : s(st), device(dev)
+{
+    if (const char *e = std::getenv("MPGPU_MEMORY_LIMIT_MB")) limit = (size_t)std::max(0.0, std::atof(e) * (1 << 20));
+}
 void DevCache::drop()
 {
     for (auto &f : free_)
@@ -220,22 +233,26 @@ void DevCache::drop()
     free_.clear();
     held = 0;
 }
+hipError_t DevCache::fresh(void **p, size_t c)
+{
+    if (limit && live_ + held + c > limit) return hipErrorOutOfMemory;
+    return hipMallocAsync(p, c, s);
+}
 void *DevCache::get(size_t bytes)
 {
-    const size_t c = size_class(bytes);
-    if (c <= CACHE_BLOCK) {
+    const size_t c = block_bytes(bytes);
+    void *p = nullptr;
+    if (c <= CACHE_BLOCK && (!limit || live_ + c <= limit)) {
         auto it = free_.find(c);
         if (it != free_.end() && !it->second.empty()) {
-            void *p = it->second.back();
+            p = it->second.back();
             it->second.pop_back();
             held -= c;
-            return p;
+        } else if (!limit || live_ + held + c <= limit) {
+            p = store_take(c | (size_t)device);
         }
-        if (void *p = store_take(c | (size_t)device)) return p;
     }
-    void *p = nullptr;
-    hipError_t e = hipMallocAsync(&p, c, s);
-    if (e != hipSuccess) {
+    if (!p && fresh(&p, c) != hipSuccess) {
         // give the free blocks back and try once more
         (void)hipGetLastError();
         drop();
@@ -252,34 +269,56 @@ void *DevCache::get(size_t bytes)
         }
         for (void *q : blocks) (void)hipFreeAsync(q, s);
         (void)hipStreamSynchronize(s);
-        HIPCHK(hipMallocAsync(&p, c, s));
+        const hipError_t e = fresh(&p, c);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            throw MemError(30, "no device memory for " + std::to_string(bytes) + " bytes beside " + std::to_string(live_) +
+                                   " in use (" + hipGetErrorString(e) + ")");
+        }
     }
+    live_ += c;
+    peak_ = std::max(peak_, live_);
     return p;
 }
-void DevCache::put(void *p, size_t bytes)
+void DevCache::put(void *p, size_t bytes) noexcept
 {
-    const size_t c = size_class(bytes);
-    if (c > CACHE_BLOCK || held + c > CACHE_CONTEXT) {
-        (void)hipFreeAsync(p, s);
-        return;
+    const size_t c = block_bytes(bytes);
+    live_ -= c;
+    if (c <= CACHE_BLOCK && held + c <= CACHE_CONTEXT) {
+        try {
+            free_[c].push_back(p);
+            held += c;
+            return;
+        } catch (...) {      // no host memory for the list: the block is not kept
+        }
     }
-    free_[c].push_back(p);
-    held += c;
+    (void)hipFreeAsync(p, s);
 }
 DevCache::~DevCache()
 {
     DevStore &S = dev_store();
-    std::vector<void *> over;
-    {
-        std::lock_guard<std::mutex> g(S.m);
-        for (auto &f : free_)
-            for (void *p : f.second) {
-                if (S.held + f.first > CACHE_STORE) { over.push_back(p); continue; }
-                S.free[f.first | (size_t)device].push_back(p);
-                S.held += f.first;
+    std::lock_guard<std::mutex> g(S.m);
+    for (auto &f : free_)
+        for (void *p : f.second) {
+            bool kept = false;
+            if (S.held + f.first <= CACHE_STORE) {
+                try {
+                    S.free[f.first | (size_t)device].push_back(p);
+                    S.held += f.first;
+                    kept = true;
+                } catch (...) {
+                }
             }
-    }
-    for (void *p : over) (void)hipFreeAsync(p, s);
+            if (!kept) (void)hipFreeAsync(p, s);
+        }
+}
+
+// MPGPU_VERBOSE: device memory of the context on stderr
+static void memory_line(mpgpu_ctx *c, const char *where)
+{
+    if (std::getenv("MPGPU_VERBOSE"))
+        std::fprintf(stderr, "device memory after %s: %zu bytes in use, %zu at most, %zu kept, %zu of ended contexts\n", where,
+                     c->cache->live(), c->cache->peak(), c->cache->kept(), mpgpu::dev_store_kept());
 }
 
 static int fail(mpgpu_ctx *c, int code, const std::string &m)
@@ -1498,6 +1537,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     c->built = true;
     c->pc.reset();
     c->dfac.reset();
+    memory_line(c, "the structure build");
     if (ntot_out) *ntot_out = c->ntot;
     if (nvar_out) *nvar_out = c->nvar;
     if (ncon_out) *ncon_out = c->ncon;
@@ -2987,6 +3027,7 @@ extern "C" int mpgpu_solve(mpgpu_ctx *c, const double *rhs, double *x, mpgpu_sol
     xd.download(x, n, s);
     HIPCHK(hipStreamSynchronize(s));
     loc.ms = now_ms() - t0;
+    memory_line(c, "the solve");
     if (st) *st = loc;
     return 0;
     API_CATCH(c)

@@ -23,31 +23,41 @@ struct MpError {
     std::string msg;
     MpError(int c, std::string m) : code(c), msg(std::move(m)) {}
 };
+// no device memory (DevCache::get)
+struct MemError : MpError {
+    using MpError::MpError;
+};
 
 // Device memory of a context.  Buffers made during a library call are ordered on the context's
 // stream, so a freed block can serve the next buffer of that context at once; when the context ends
 // (its stream has finished) its free blocks go to a store shared by the contexts of the device.
 // hipFreeAsync takes 8 us for a small block and over 100 us from 1 MB on, and a job of the serving
 // engine frees some two hundred.  Blocks above CACHE_BLOCK go straight to hipMallocAsync /
-// hipFreeAsync; a context keeps at most CACHE_CONTEXT bytes of free blocks and the store CACHE_STORE,
-// and both are given back when an allocation fails.
+// hipFreeAsync, in their own size; a context keeps at most CACHE_CONTEXT bytes of free blocks and the
+// store CACHE_STORE, and both are given back when an allocation fails.
 class DevCache {
   public:
-    DevCache(hipStream_t st, int dev) : s(st), device(dev) {}
+    DevCache(hipStream_t st, int dev);
     ~DevCache();                             // the stream has finished
     DevCache(const DevCache &) = delete;
     DevCache &operator=(const DevCache &) = delete;
     void *get(size_t bytes);
-    void put(void *p, size_t bytes);
+    void put(void *p, size_t bytes) noexcept;
     hipStream_t stream() const { return s; }
+    size_t live() const { return live_; }    // bytes in use, their maximum, and bytes of free blocks
+    size_t peak() const { return peak_; }
+    size_t kept() const { return held; }
 
   private:
     hipStream_t s;
     int device;
-    size_t held = 0;
+    size_t held = 0, live_ = 0, peak_ = 0;
+    size_t limit = 0;                        // most bytes in use (MPGPU_MEMORY_LIMIT_MB; 0: the device's)
     std::unordered_map<size_t, std::vector<void *>> free_;
     void drop();
+    hipError_t fresh(void **p, size_t c);
 };
+size_t dev_store_kept();                     // bytes of free blocks of ended contexts
 // memory of the library call in progress on this thread (none: hipMalloc / hipFree)
 inline DevCache *&alloc_cache()
 {
