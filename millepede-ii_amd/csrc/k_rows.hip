@@ -1233,8 +1233,9 @@ void rows_incidence(RowStruct &S, const int32_t *group_of, const PairMap &pm, in
         for (size_t b = 0; b < S.batches.size(); b++)
             for (int x = 0; x < 3; x++) S.batches[b].ncls[x] = (int64_t)h[3 * b + x];
     }
-    S.unit.alloc((size_t)mu * ubytes);
-    S.side.alloc((size_t)mu * 4);
+    S.unit_bytes = (size_t)mu * ubytes;
+    S.side_len = (size_t)mu * 4;
+    S.alloc_units();
     S.c.release();
 }
 

@@ -222,9 +222,11 @@ size_t mpgpu::dev_store_kept()
     return S.held;
 }
 
-DevCache::DevCache(hipStream_t st, int dev) : s(st), device(dev)
+DevCache::DevCache(hipStream_t st, int dev) : s(st), device(dev) { read_limit(); }
+void DevCache::read_limit()
 {
-    if (const char *e = std::getenv("MPGPU_MEMORY_LIMIT_MB")) limit = (size_t)std::max(0.0, std::atof(e) * (1 << 20));
+    const char *e = std::getenv("MPGPU_MEMORY_LIMIT_MB");
+    limit = e ? (size_t)std::max(0.0, std::atof(e) * (1 << 20)) : 0;
 }
 void DevCache::drop()
 {
@@ -232,6 +234,15 @@ void DevCache::drop()
         for (void *p : f.second) (void)hipFreeAsync(p, s);
     free_.clear();
     held = 0;
+}
+int64_t DevCache::room() const
+{
+    size_t fr = 0, tot = 0;
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
+        (void)hipGetLastError();
+        fr = (size_t)128 << 30;
+    }
+    return (int64_t)(limit ? std::min(fr, limit > live_ ? limit - live_ : 0) : fr);
 }
 hipError_t DevCache::fresh(void **p, size_t c)
 {
@@ -253,8 +264,9 @@ void *DevCache::get(size_t bytes)
         }
     }
     if (!p && fresh(&p, c) != hipSuccess) {
-        // give the free blocks back and try once more
+        // give back what the context can do without and the free blocks, and try once more
         (void)hipGetLastError();
+        if (reclaim) reclaim();
         drop();
         std::vector<void *> blocks;
         {
@@ -312,6 +324,10 @@ DevCache::~DevCache()
             if (!kept) (void)hipFreeAsync(p, s);
         }
 }
+
+// device bytes of a packed matrix of n rows with what the solves allocate beside it (at most: copy and
+// square matrix of the inversion, or FP32 and FP64 factors), and of vectors and factor workspaces
+static int64_t full_storage_bytes(int64_t n) { return 4 * (8 * n * (n + 1) / 2) + 4096 * n; }
 
 // MPGPU_VERBOSE: device memory of the context on stderr
 static void memory_line(mpgpu_ctx *c, const char *where)
@@ -412,6 +428,7 @@ int mpgpu::create_context(const mpgpu_options *opt, int32_t device, hipStream_t 
         (void)hipGetLastError();
     }
     c->cache = new DevCache(c->stream, device);
+    c->cache->reclaim = [c] { if (!c->rows.in_pass) c->rows.free_units(); };
     *out = c;
     return 0;
     }
@@ -427,6 +444,7 @@ extern "C" int mpgpu_destroy(mpgpu_ctx *c)
     hipStream_t s = c->stream;
     const bool own = c->own_stream;
     DevCache *cache = c->cache;
+    cache->reclaim = nullptr;
     delete c;
     if (s) (void)hipStreamSynchronize(s);
     delete cache;
@@ -462,6 +480,7 @@ extern "C" int mpgpu_set_options(mpgpu_ctx *c, const mpgpu_options *o)
             return fail(c, 30, std::string("option ") + which + " is fixed once the structure is built (rebuild the context to change it)");
     }
     c->opt = *o;
+    c->cache->read_limit();
     return 0;
 }
 
@@ -1140,8 +1159,11 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     int32_t max_ngl_all = 1;
     for (int32_t x : ngl_rec) max_ngl_all = std::max(max_ngl_all, x);
     // the pairs of groups that records couple: the blocks of group-block storage, and with full
-    // storage those that the records in row form are gathered by (a bitmap of up to 256 MB)
-    const bool try_rows = c->opt.monitor == 0 && nrec > 0 && (sparse ? !c->elim : c->ngroup <= 65536);
+    // storage those that the records in row form are gathered by (a bitmap of up to 256 MB; the pairs of
+    // up to 65,535 groups are below 2^31, as st_blocks needs them)
+    constexpr int32_t FULL_ROW_GROUPS = 65535;
+    static_assert((int64_t)FULL_ROW_GROUPS * (FULL_ROW_GROUPS + 1) / 2 < ((int64_t)1 << 31), "pairs of groups");
+    const bool try_rows = c->opt.monitor == 0 && nrec > 0 && (sparse ? !c->elim : c->ngroup <= FULL_ROW_GROUPS);
     st_record_stats(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->d_var.p, c->d_group_of.p, c->ngroup, max_ngl_all,
                     sparse || try_rows, pm, rst, cnt_r, d_rst, s);
     const int32_t *st_nv = rst.data(), *st_nseg = rst.data() + nrec, *st_nalc = rst.data() + 2 * nrec,
@@ -1312,6 +1334,14 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     if (c->nband > 0) c->d_band_info.upload(binfo, s);
     c->ngen = nrec;
     std::vector<int64_t> row_upd;      // update sizes of the records in row form, when a batch size is set
+    // what the passes' update buffers and units may take: MPGPU_UPDATE_BUFFER_GB, else 45 % of the
+    // memory that the rest leaves, up to 128 GB (a whole pass of the large workloads in one batch: the
+    // matrix is read and written once per pass)
+    const char *buffer_gb = std::getenv("MPGPU_UPDATE_BUFFER_GB");
+    auto buffer_doubles = [&](int64_t left) {
+        const double gb = buffer_gb ? std::atof(buffer_gb) : std::min(128.0, 0.45 * (double)std::max<int64_t>(left, 0) / (1ull << 30));
+        return std::max<int64_t>(1 << 20, (int64_t)(gb * (1ull << 30) / 8.0));
+    };
     if (try_rows) {
         std::vector<int32_t> tg_of(ntot), tg_t0, tg_v0;
         std::vector<uint32_t> tg_mask;
@@ -1352,20 +1382,43 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         d_mask.upload(tg_mask, s);
         const RowGroups Q{d_of.p, d_t0.p, c->d_var.p, d_col.p, d_mask.p, d_v0.p};
         std::vector<uint8_t> cls;
-        rows_classify(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->nband > 0 ? c->d_band_info.p : nullptr, Q, c->rows, cls, s);
         std::vector<int64_t> fast, gen;
-        fast.reserve(nrec);
-        for (int64_t q = 0; q < nrec; q++) (cls[order[q]] ? fast : gen).push_back(order[q]);
-        if (std::getenv("MPGPU_UPDATE_BUFFER_GB"))
-            for (int64_t r : fast) row_upd.push_back(cnt_r[r]);
-        rows_build(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, Q, fast, c->rows, s);
-        if (!sparse && c->rows.nq > 0) {
-            // the lists of a dense matrix are long: without room for them the record kernel's
-            // atomic additions remain
-            size_t fr = 0, tot = 0;
-            const bool room = hipMemGetInfo(&fr, &tot) != hipSuccess || c->rows.list_bytes() < (int64_t)(fr / 2);
-            (void)hipGetLastError();
-            if (!room) {
+        auto form = [&]() {
+            rows_classify(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, c->nband > 0 ? c->d_band_info.p : nullptr, Q, c->rows, cls, s);
+            fast.reserve(nrec);
+            for (int64_t q = 0; q < nrec; q++) (cls[order[q]] ? fast : gen).push_back(order[q]);
+            if (buffer_gb)
+                for (int64_t r : fast) row_upd.push_back(cnt_r[r]);
+            rows_build(sin, c->d_widx, c->d_rec_gl, c->d_gl_tix, Q, fast, c->rows, s);
+        };
+        if (sparse) {
+            form();
+        } else {
+            // with full storage the record kernel's atomic additions do without lists and units: it
+            // keeps the records when the lists (long ones, of a dense matrix) would take more than
+            // half of what the matrix and the solve leave, or an allocation fails
+            bool ok = true;
+            try {
+                form();
+                if (c->rows.nq > 0) {
+                    const int64_t pairs = (int64_t)c->ngroup * (c->ngroup + 1) / 2;
+                    const int64_t left = c->cache->room() - full_storage_bytes(c->nall);
+                    const int64_t lists = c->rows.list_bytes(std::min(pairs, c->rows.npair)) + 32 * std::min(pairs, c->rows.npair);
+                    ok = lists < left / 2;
+                    if (ok) {
+                        st_blocks(pm, c->ngroup, c->d_gfirst.p, {}, blk, false, s);
+                        c->rows.nblock = blk.nblock;
+                        c->rows.brow.swap(blk.brow);
+                        c->rows.brg.swap(blk.brg);
+                        c->rows.bcol.swap(blk.bcol);
+                        rows_incidence(c->rows, c->d_group_of.p, pm, blk.nblock, c->rows.brg.p, c->rows.bcol.p,
+                                       buffer_doubles(left - lists), row_upd, s);
+                    }
+                }
+            } catch (const MemError &) {
+                ok = false;
+            }
+            if (!ok) {
                 c->rows.drop();
                 fast.clear();
                 gen = order;
@@ -1389,19 +1442,17 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         std::vector<int32_t> rec_cn(nrec, 0);
         for (int64_t r = 0; r < nrec; r++)
             if (binfo[r]) cnt_r[r] = 0;             // bordered-band records update the matrix directly
-        // update-buffer cap: MPGPU_UPDATE_BUFFER_GB, else 45 % of the free device memory up to
-        // 128 GB (a whole pass of the large workloads in one batch: the matrix is read and
-        // written once per pass, one record-kernel launch)
-        const char *env = std::getenv("MPGPU_UPDATE_BUFFER_GB");
-        double gb = 64.0;
-        if (env) gb = std::atof(env);
-        else {
-            size_t fr = 0, tot = 0;
-            if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr > 0) gb = std::min(128.0, 0.45 * (double)fr / (1ull << 30));
-            else (void)hipGetLastError();
-        }
-        const int64_t budget = std::max<int64_t>(1 << 20, (int64_t)(gb * (1ull << 30) / 8.0));
+        // one budget for the units of the records in row form and the updates of the others, out of
+        // what the matrix, the product's values, the lists of both and the vectors leave
+        int64_t gen_pairs = 0;
+        for (int64_t q = 0; q < c->ngen; q++)
+            if (cnt_r[order[q]] > 0) gen_pairs += (int64_t)st_nseg[order[q]] * (st_nseg[order[q]] + 1) / 2;
+        const int64_t left = c->cache->room() - 8 * c->nstored - 8 * (int64_t)c->plan.max_grp * c->nblock - 512 * (int64_t)c->nall -
+                             (c->rows.nq > 0 ? c->rows.list_bytes(c->nblock) : 0) - 40 * gen_pairs;
+        int64_t budget = buffer_doubles(left);
         rows_incidence(c->rows, c->d_group_of.p, pm, c->nblock, c->d_brg.p, c->d_bcol.p, budget, row_upd, s);
+        if (!buffer_gb && c->rows.nq > 0)
+            budget = std::max<int64_t>(1 << 20, budget - (int64_t)(c->rows.unit_bytes / 8 + c->rows.side_len));
         phase("row incidence lists");
         // the other records: per record the block id of each segment pair
         if (c->ngen > 0)
@@ -1475,18 +1526,6 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
         c->d_rec_pb.release();
         c->d_pair_blk.release();
     }
-    if (!sparse && c->rows.nq > 0) {
-        st_blocks(pm, c->ngroup, c->d_gfirst.p, {}, blk, false, s);
-        c->rows.nblock = blk.nblock;
-        c->rows.brow.swap(blk.brow);
-        c->rows.brg.swap(blk.brg);
-        c->rows.bcol.swap(blk.bcol);
-        size_t fr = 0, tot = 0;
-        int64_t budget = (int64_t)1 << 33;
-        if (hipMemGetInfo(&fr, &tot) == hipSuccess && fr > 0) budget = (int64_t)(0.45 * (double)fr) / 8;
-        else (void)hipGetLastError();
-        rows_incidence(c->rows, c->d_group_of.p, pm, blk.nblock, c->rows.brg.p, c->rows.bcol.p, budget, {}, s);
-    }
     phase("two-phase index");
     // ---- remaining device state ----
     if (c->nband > 0) {
@@ -1537,6 +1576,9 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
     c->built = true;
     c->pc.reset();
     c->dfac.reset();
+    if (verbose)
+        std::fprintf(stderr, "records in row form: %lld in %zu batches, by the record kernel: %lld in %zu\n", (long long)c->rows.nq,
+                     c->rows.batches.size(), (long long)c->ngen, sparse ? c->batches.size() : (size_t)(c->ngen > 0));
     memory_line(c, "the structure build");
     if (ntot_out) *ntot_out = c->ntot;
     if (nvar_out) *nvar_out = c->nvar;
@@ -1740,10 +1782,35 @@ extern "C" int mpgpu_loopn(mpgpu_ctx *c, int32_t icalcm, int32_t nloopn, float c
     HIPCHK(hipEventRecord(e1, s));
     if (c->rows.nq > 0) {
         // records in row form
-        const RowStruct &S = c->rows;
+        RowStruct &S = c->rows;
+        struct InPass {
+            bool &f;
+            explicit InPass(bool &b) : f(b) { f = true; }
+            ~InPass() { f = false; }
+        } in_pass(S.in_pass);
+        bool units = true;
+        if (icalcm == 1) {
+            try {
+                S.alloc_units();
+            } catch (const MemError &) {
+                // no room for the units beside what was allocated since the structure build: with full
+                // storage the record kernel adds these records
+                if (c->opt.matsto == MPGPU_SPARSE) throw;
+                S.free_units();
+                units = false;
+            }
+        }
+        if (!units) {
+            DevRecords Q = R;
+            Q.order = S.order.p;
+            auto tr = timed(t_rec);
+            HIPCHK(hipEventRecord(tr.first, s));
+            HIPCHK(launch_records(Q, M, o, out, c->plan, 0, S.nq, (int)std::min<int64_t>(S.nq, 256 * 40), s, mon));
+            HIPCHK(hipEventRecord(tr.second, s));
+        }
         RowDev D{S.hdr.p, S.rows.p, S.eq_t0.p, S.eq_pos.p, S.seq.p, S.seg.p, S.ptix.p, c->ntot, 0, S.unit.p, S.side.p};
         const bool build = icalcm == 1;
-        for (size_t bt = 0; bt < (build ? S.batches.size() : 1); bt++) {
+        for (size_t bt = 0; units && bt < (build ? S.batches.size() : 1); bt++) {
             const int64_t q0 = build ? S.batches[bt].q0 : 0, q1 = build ? S.batches[bt].q1 : S.nq;
             if (build) D.ub = S.batches[bt].unit0;
             auto tr = timed(t_rec);

@@ -3,6 +3,7 @@
 #include "mpgpu_device.h"
 #include "../../include/mpgpu.h"
 #include <algorithm>
+#include <functional>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -47,12 +48,15 @@ class DevCache {
     size_t live() const { return live_; }    // bytes in use, their maximum, and bytes of free blocks
     size_t peak() const { return peak_; }
     size_t kept() const { return held; }
+    int64_t room() const;                    // bytes new buffers may take: free on the device, within the limit
+    void read_limit();                       // MPGPU_MEMORY_LIMIT_MB
+    std::function<void()> reclaim;           // gives back what the context can do without, when an allocation fails
 
   private:
     hipStream_t s;
     int device;
     size_t held = 0, live_ = 0, peak_ = 0;
-    size_t limit = 0;                        // most bytes in use (MPGPU_MEMORY_LIMIT_MB; 0: the device's)
+    size_t limit = 0;                        // most bytes in use (0: the device's)
     std::unordered_map<size_t, std::vector<void *>> free_;
     void drop();
     hipError_t fresh(void **p, size_t c);
@@ -420,19 +424,35 @@ struct RowStruct {
     std::vector<Batch> batches;       // matrix build: batches of records and their incidence lists
     DBuf<uint32_t> ptr, perm;         // perm: order of the blocks in the gather
     DBuf<uint2> src;
-    DBuf<uint8_t> unit;               // units and side array of the largest batch
+    // units and side array of the largest batch: contents live only within a pass, so that an
+    // allocation that fails between passes can have their memory (alloc_units)
+    DBuf<uint8_t> unit;
     DBuf<double> side;
+    size_t unit_bytes = 0, side_len = 0;
+    bool in_pass = false;
     int64_t nblock = 0;               // full storage: the pairs of groups that some record couples
     DBuf<int64_t> brow;
     DBuf<int32_t> brg, bcol;
-    // device bytes of the incidence lists, with what their sort needs beside them
+    void alloc_units()
+    {
+        unit.alloc(unit_bytes);
+        side.alloc(side_len);
+    }
+    void free_units()
+    {
+        unit.release(); side.release();
+    }
     void drop()
     {
         nq = 0;
-        order.release(); c.release(); hdr.release(); rows.release(); eq_t0.release(); ptix.release(); eq_pos.release();
-        seq.release(); seg.release();
+        order.release(); c.release(); n.release(); hdr.release(); rows.release(); eq_t0.release(); ptix.release();
+        eq_pos.release(); seq.release(); seg.release(); ptr.release(); perm.release(); src.release(); brow.release();
+        brg.release(); bcol.release();
+        free_units();
+        batches.clear();
     }
-    int64_t list_bytes() const { return 8 * npair + 24 * std::min<int64_t>(npair, (int64_t)1 << 30); }
+    // device bytes of the incidence lists and the block order for nb blocks, with what their sorts need
+    int64_t list_bytes(int64_t nb) const { return 8 * npair + 24 * std::min<int64_t>(npair, (int64_t)1 << 30) + 48 * nb; }
 };
 void rows_classify(const StructIn &in, const DBuf<int32_t> &widx, const DBuf<int64_t> &rec_gl, const DBuf<int32_t> &gl_tix,
                    const int32_t *band, const RowGroups &Q, RowStruct &S, std::vector<uint8_t> &cls, hipStream_t s);

@@ -5,6 +5,8 @@ equations per wavefront (64, 66, 128, 130), group sizes, local parameters, equat
 (an odd one leaves half a unit empty), fixed parameters inside a group, FP64 payloads, rejected
 records, and lists of a matrix block short and long (few modules, many records).  The bar is that
 of the other parity tests: FP64 arithmetic, only the order of sums differs, 1e-10 relative."""
+import re
+
 import numpy as np
 import pytest
 
@@ -53,6 +55,86 @@ CASES = [
     (12, 6, 6, 100, 8, 2, np.float32),      # six local parameters: not in row form
     (5, 6, 4, 1500, 4, 2, np.float32),      # lists of 900 pairs per block
 ]
+
+
+# which records of the cases have row form
+IN_ROW_FORM = [True] * 6 + [False] + [True] * 2 + [False] * 3 + [True]
+
+
+def paths(err):
+    """(records in row form, batches, records of the record kernel, batches) from the build's MPGPU_VERBOSE line"""
+    m = re.findall(r"records in row form: (\d+) in (\d+) batches, by the record kernel: (\d+) in (\d+)", err)
+    return tuple(map(int, m[-1]))
+
+
+@pytest.mark.parametrize("matsto", [mpgpu.SPARSE, mpgpu.FULL])
+@pytest.mark.parametrize("k", range(len(CASES)))
+def test_which_records_have_row_form(monkeypatch, capfd, k, matsto):
+    nmod, gsize, nloc, nrec, hits, per_hit, dtype = CASES[k]
+    rp, ii, gg = _records(sum(CASES[k][:6]), nmod, gsize, nloc, nrec, hits, per_hit, dtype)
+    monkeypatch.setenv("MPGPU_VERBOSE", "1")
+    P = mpgpu.Pede(matsto=matsto, metsol=mpgpu.MINRES, mreqenf=1, mcount=1, lfitbb=0)
+    P.add_records(rp, ii, gg)
+    P.build_structure()
+    P.close()
+    row, _, gen, _ = paths(capfd.readouterr().err)
+    assert (row, gen) == ((nrec, 0) if IN_ROW_FORM[k] else (0, nrec))
+
+
+def _mixed(seed, nmod=24, nrec=600):
+    """records of both forms on the same modules: two thirds with 4 local parameters, the others with 6"""
+    a = _records(seed, nmod, 6, 4, nrec * 2 // 3, 8, 2, np.float32)
+    b = _records(seed + 1, nmod, 6, 6, nrec - nrec * 2 // 3, 8, 2, np.float32)
+    cut = lambda r: [(r[1][x:y], r[2][x:y]) for x, y in zip(r[0][:-1], r[0][1:])]
+    recs = cut(a) + cut(b)
+    np.random.default_rng(seed + 2).shuffle(order := np.arange(len(recs)))
+    rp = np.concatenate([[0], np.cumsum([len(recs[k][0]) for k in order])]).astype(np.int64)
+    return rp, np.concatenate([recs[k][0] for k in order]), np.concatenate([recs[k][1] for k in order])
+
+
+@pytest.mark.parametrize("matsto", [mpgpu.SPARSE, mpgpu.FULL])
+@pytest.mark.parametrize("batches", [False, True])
+def test_records_of_both_forms(orc, monkeypatch, capfd, matsto, batches):
+    """Both gathers (or the gather and the atomic additions) add to the same blocks, vector and counters, in one
+    batch and with a buffer so small that each takes several."""
+    rp, ii, gg = _mixed(11, nrec=3600 if batches else 600)
+    n = len(rp) - 1
+    monkeypatch.setenv("MPGPU_VERBOSE", "1")
+    if batches:
+        monkeypatch.setenv("MPGPU_UPDATE_BUFFER_GB", "0.001")       # 2^20 doubles, the least that is taken
+    P = mpgpu.Pede(matsto=matsto, metsol=mpgpu.MINRES, mreqenf=1, mcount=1, lhuber=3, lfitbb=0)
+    P.add_records(rp, ii, gg)
+    P.build_structure()
+    row, nb, gen, nb2 = paths(capfd.readouterr().err)
+    assert (row, gen) == (n * 2 // 3, n - n * 2 // 3)
+    assert (nb > 1) == batches and (nb2 > 1) == (batches and matsto == mpgpu.SPARSE)
+    lab, var = P.labels()[:2]
+    par = P.parameters()
+    par[var > 0] = 1e-3 * np.arange(P.nvar)
+    P.set_parameters(par)
+    _compare_pass(P, orc, rp, ii, gg, lab, var, chicut=0.0)
+    _compare_pass(P, orc, rp, ii, gg, lab, var, nloopn=2, lhuber=3, chicut=1.2)
+    _compare_pass(P, orc, rp, ii, gg, lab, var, nloopn=2, lhuber=3, icalcm=0)
+    P.close()
+
+
+@pytest.mark.parametrize("matsto", [mpgpu.SPARSE, mpgpu.FULL])
+@pytest.mark.parametrize("nloc", [4, 6])
+def test_small_buffer(monkeypatch, capfd, orc, matsto, nloc):
+    """Several batches of records of one form (6 local parameters: the record kernel and the gather of its
+    updates, in full storage one launch of atomic additions)."""
+    rp, ii, gg = _records(5 + nloc, 24, 6, nloc, 2500, 8, 2, np.float32)
+    monkeypatch.setenv("MPGPU_VERBOSE", "1")
+    monkeypatch.setenv("MPGPU_UPDATE_BUFFER_GB", "0.001")
+    P = mpgpu.Pede(matsto=matsto, metsol=mpgpu.MINRES, mreqenf=1, mcount=1, lfitbb=0)
+    P.add_records(rp, ii, gg)
+    P.build_structure()
+    row, nb, gen, nb2 = paths(capfd.readouterr().err)
+    assert (row, gen) == ((2500, 0) if nloc == 4 else (0, 2500))
+    assert nb > 1 if nloc == 4 else nb2 > 1 or matsto == mpgpu.FULL
+    lab, var = P.labels()[:2]
+    _compare_pass(P, orc, rp, ii, gg, lab, var)
+    P.close()
 
 
 @pytest.mark.parametrize("matsto", [mpgpu.SPARSE, mpgpu.FULL])
