@@ -23,8 +23,8 @@ def memory(monkeypatch, capfd):
     return lambda: [(m[0], *map(int, m[1:])) for m in re.findall(LINE, capfd.readouterr().err)]
 
 
-def _context(matsto, metsol, seed=3, modules=40, tracks=400, **opt):
-    rp, ii, gg = _records(seed, modules, 6, 4, tracks, 8, 2, np.float32)
+def _context(matsto, metsol, seed=3, modules=40, tracks=400, nloc=4, **opt):
+    rp, ii, gg = _records(seed, modules, 6, nloc, tracks, 8, 2, np.float32)
     P = mpgpu.Pede(matsto=matsto, metsol=metsol, mreqenf=1, mcount=1, **opt)
     P.add_records(rp, ii, gg)
     labels = np.array([100 * (m + 1) + k + 1 for m in range(modules) for k in range(6)], np.int32)
@@ -139,9 +139,9 @@ def test_pass_without_room_for_units(memory, monkeypatch):
     v, A = _pass_of(P)
     monkeypatch.setenv("MPGPU_MEMORY_LIMIT_MB", repr((use - 4000 * 8 * 64) / (1 << 20)))
     P.set_options()
-    with pytest.raises(mpgpu.MpgpuError):
-        P.solve()
+    P.solve()                           # takes the units' memory
     w, B = _pass_of(P)
+    assert not np.array_equal(A, B)     # (atomic additions)
     assert np.abs(v - w).max() <= 1e-10 * np.abs(v).max() and np.abs(A - B).max() <= 1e-10 * np.abs(A).max()
     monkeypatch.delenv("MPGPU_MEMORY_LIMIT_MB")
     P.set_options()
@@ -166,3 +166,41 @@ def test_full_storage_without_room_for_lists(monkeypatch, capfd):
     assert "records in row form: 0 in 0 batches, by the record kernel: 4000 in 1" in capfd.readouterr().err
     assert np.abs(v - w).max() <= 1e-10 * np.abs(v).max() and np.abs(A - B).max() <= 1e-10 * np.abs(A).max()
     P.close()
+
+
+@pytest.mark.parametrize("modules,defect", [(22, False), (22, True), (150, False)])
+def test_inversion_without_room_for_the_square_matrix(memory, monkeypatch, modules, defect):
+    """The square copy of the matrix (16 n^2 / 2 bytes) does not fit beside the packed one and its copy: one
+    pivot at a time in the packed matrix, with the same pivots, so the same rank, and the same solution and
+    inverse but for rounding.  (defect: parameters that nothing determines.)"""
+    def context():
+        # (6 local parameters: no units whose memory could be had instead)
+        P = _context(mpgpu.FULL, mpgpu.INVERSION, modules=modules, tracks=1000, nloc=6)
+        P.loopn()
+        if defect:
+            # the last module's rows and columns away
+            A = P.matrix_packed()
+            n = P.nall
+            i = np.arange(n - 6, n)
+            rows = np.concatenate([np.full(k + 1, k) for k in i])
+            cols = np.concatenate([np.arange(k + 1) for k in i])
+            P.mupdat(rows + 1, cols + 1, -A[rows * (rows + 1) // 2 + cols])
+        return P
+
+    P = context()
+    x, st = P.solve()
+    err, gcor = P.errors()
+    P.close()
+    use = memory()[1][1]
+    n, packed = P.nall, 4 * P.nall * (P.nall + 1)
+    Q = context()
+    assert Q.nall == n > 128
+    monkeypatch.setenv("MPGPU_MEMORY_LIMIT_MB", repr((use + packed + 4 * n * n) / (1 << 20)))
+    Q.set_options()
+    y, st2 = Q.solve()
+    e2, g2 = Q.errors()
+    Q.close()
+    assert st["nrank"] == st2["nrank"] == n - (6 if defect else 0)
+    # REAL(4) errors; the condition of these systems is below 1e4
+    assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max()
+    assert np.allclose(err, e2, rtol=1e-6) and np.allclose(gcor, g2, rtol=1e-5, atol=1e-6)
