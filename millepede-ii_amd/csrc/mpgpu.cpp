@@ -222,6 +222,18 @@ size_t mpgpu::dev_store_kept()
     return S.held;
 }
 
+void mpgpu::dev_store_trim(int device, size_t most, hipStream_t st)
+{
+    DevStore &S = dev_store();
+    std::lock_guard<std::mutex> g(S.m);
+    for (auto &f : S.free)
+        while (S.held > most && (int)(f.first & 255) == device && !f.second.empty()) {
+            (void)hipFreeAsync(f.second.back(), st);
+            f.second.pop_back();
+            S.held -= f.first & ~(size_t)255;
+        }
+}
+
 DevCache::DevCache(hipStream_t st, int dev) : s(st), device(dev) { read_limit(); }
 void DevCache::read_limit()
 {
@@ -296,7 +308,7 @@ void DevCache::put(void *p, size_t bytes) noexcept
 {
     const size_t c = block_bytes(bytes);
     live_ -= c;
-    if (c <= CACHE_BLOCK && held + c <= CACHE_CONTEXT) {
+    if (c <= CACHE_BLOCK && held + c <= CACHE_CONTEXT && live_ + held + c <= share) {
         try {
             free_[c].push_back(p);
             held += c;
@@ -325,9 +337,7 @@ DevCache::~DevCache()
         }
 }
 
-// device bytes of a packed matrix of n rows with what the solves allocate beside it (at most: copy and
-// square matrix of the inversion, or FP32 and FP64 factors), and of vectors and factor workspaces
-static int64_t full_storage_bytes(int64_t n) { return 4 * (8 * n * (n + 1) / 2) + 4096 * n; }
+DevCache &mpgpu::context_memory(mpgpu_ctx *c) { return *c->cache; }
 
 // MPGPU_VERBOSE: device memory of the context on stderr
 static void memory_line(mpgpu_ctx *c, const char *where)
@@ -1402,7 +1412,7 @@ extern "C" int mpgpu_build_structure(mpgpu_ctx *c, int32_t *ntot_out, int32_t *n
                 form();
                 if (c->rows.nq > 0) {
                     const int64_t pairs = (int64_t)c->ngroup * (c->ngroup + 1) / 2;
-                    const int64_t left = c->cache->room() - full_storage_bytes(c->nall);
+                    const int64_t left = c->cache->room() - full_storage_bytes(MPGPU_CHOLESKY_FP32_IR, c->nall);   // the largest
                     const int64_t lists = c->rows.list_bytes(std::min(pairs, c->rows.npair)) + 32 * std::min(pairs, c->rows.npair);
                     ok = lists < left / 2;
                     if (ok) {

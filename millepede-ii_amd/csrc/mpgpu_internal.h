@@ -50,6 +50,7 @@ class DevCache {
     size_t kept() const { return held; }
     int64_t room() const;                    // bytes new buffers may take: free on the device, within the limit
     void read_limit();                       // MPGPU_MEMORY_LIMIT_MB
+    void set_share(size_t b) { share = b; }  // no more free blocks than fit below b bytes with those in use
     std::function<void()> reclaim;           // gives back what the context can do without, when an allocation fails
 
   private:
@@ -57,11 +58,13 @@ class DevCache {
     int device;
     size_t held = 0, live_ = 0, peak_ = 0;
     size_t limit = 0;                        // most bytes in use (0: the device's)
+    size_t share = SIZE_MAX;
     std::unordered_map<size_t, std::vector<void *>> free_;
     void drop();
     hipError_t fresh(void **p, size_t c);
 };
 size_t dev_store_kept();                     // bytes of free blocks of ended contexts
+void dev_store_trim(int device, size_t most, hipStream_t st);   // frees blocks of a device until at most that many are kept
 // memory of the library call in progress on this thread (none: hipMalloc / hipFree)
 inline DevCache *&alloc_cache()
 {
@@ -381,6 +384,21 @@ void st_record_lists(const StructIn &in, const LabelMap &map, int32_t ntot, bool
 // a context on a stream the caller keeps (serving workers reuse one stream per worker), or on
 // a stream of its own when stream is null
 int create_context(const mpgpu_options *opt, int32_t device, hipStream_t stream, mpgpu_ctx **out);
+DevCache &context_memory(mpgpu_ctx *c);
+// device bytes of a packed matrix of n rows and what a solve allocates beside it: the inversion a
+// copy and a square matrix (1 + 2 packed), the FP64 factor a full matrix (2), the FP32 factor a full
+// FP32 one (1) and, when the refinement does not converge, the FP64 factor as well; workspaces
+inline int64_t full_storage_bytes(int metsol, int64_t n)
+{
+    int64_t mult = 2;
+    switch (metsol) {
+    case MPGPU_INVERSION: mult = n > 128 ? 4 : 2; break;
+    case MPGPU_DECOMPOSITION: case MPGPU_LAPACK_PACKED: case MPGPU_LAPACK_UNPACKED: mult = 3; break;
+    case MPGPU_CHOLESKY_FP32_IR: mult = 4; break;
+    default: break;
+    }
+    return mult * (8 * n * (n + 1) / 2) + 4096 * n;
+}
 // FP32 values widened to FP64 (device to device)
 void st_widen(const float *src, double *dst, int64_t n, hipStream_t s);
 // residual monitoring: label of the first global word (0: none) and error of every equation

@@ -38,7 +38,10 @@ struct Job {
     const int64_t *cptr = nullptr;
     const int32_t *clab = nullptr;
     const double *cfac = nullptr, *crhs = nullptr;
-    int64_t footprint = -1;   // device bytes, sized by the worker that takes the job
+    // device bytes, sized by the worker that takes the job: what it is charged, and what it cannot do
+    // without (the rest makes passes faster or is there only while the structure is built)
+    int64_t footprint = -1, least = -1;
+    size_t peak = 0;          // most bytes its context had in use
     double size_ms = 0;       // time of the sizing
     clk::time_point t_arrival, t_start, t_end;
     // results
@@ -52,11 +55,13 @@ struct Job {
     bool done = false;
 };
 
-// device bytes a job needs: records (8 B/word + compiled tables), the matrix (full packed or
-// an upper estimate of the group-block storage), the update buffer of the two-phase build
-// (group-block storage: at most the lower triangle of each record's global words, 8 B each),
-// vectors and solver work space
-int64_t estimate_footprint(const Job &j)
+// Device bytes of a job.  Least: records (8 B/word + compiled tables), the matrix (full packed or an
+// upper estimate of the group-block storage) and what the solve puts beside it, the update buffer of
+// the two-phase build (group-block storage: at most the lower triangle of each record's global
+// words, 8 B each), vectors.  Charged: also the records in row form with their units (k_rows.hip; at
+// most 192 + 32 bytes for two equations of a group), the lists of group pairs of either form (8 to
+// 12 B a pair, and 28 while they are sorted) and the square matrix of the inversion.
+void size_job(Job &j)
 {
     const int64_t nrec = j.nrec;
     const int64_t nw = nrec > 0 ? j.rec_ptr[nrec] - j.rec_ptr[0] : 0;
@@ -66,25 +71,44 @@ int64_t estimate_footprint(const Job &j)
     // (the worker's OpenMP threads): their global words and label range, then a bitmap
     const int64_t *rp = j.rec_ptr;
     const int32_t *I = j.inder;
-    int64_t upd = 0;
+    const bool full = j.opt.matsto == MPGPU_FULL;
+    int64_t upd = 0, scratch = 0, rows = 0;
     int32_t lmin = INT32_MAX, lmax = INT32_MIN;
-#pragma omp parallel for schedule(static, 256) reduction(+ : upd) reduction(min : lmin) reduction(max : lmax)
+#pragma omp parallel for schedule(static, 256) reduction(+ : upd, scratch, rows) reduction(min : lmin) reduction(max : lmax)
     for (int64_t r = 0; r < nrec; r++) {
+        // equations with the same first label are of one group; runs of them bound the record's
+        // groups and units from above (a group that comes in several runs is counted in each)
         int zeros = 0;
-        int64_t g = 0;
+        int64_t g = 0, runs = 0, units = 0, len = 0;
+        int32_t first = 0;
+        bool start = false;
         for (int64_t w = rp[r] + 1; w < rp[r + 1]; w++) {
             const int32_t l = I[w];
-            if (l == 0) { zeros++; continue; }
+            if (l == 0) { zeros++; start = true; continue; }
             if (zeros > 0 && zeros % 2 == 0) {
                 g++;
+                if (start) {
+                    if (len == 0 || l != first) {
+                        units += (len + 1) / 2;
+                        runs++;
+                        len = 0;
+                        first = l;
+                    }
+                    len++;
+                    start = false;
+                }
                 lmin = std::min(lmin, l);
                 lmax = std::max(lmax, l);
             }
         }
-        upd += 8 * g * (g + 1) / 2;
+        units += (len + 1) / 2;
+        const int64_t u = full ? 0 : 8 * g * (g + 1) / 2, pairs = std::max(runs, units);
+        upd += u;
+        scratch += std::max(u, 224 * units);
+        rows += 72 * (zeros / 2) + 32 * runs + 160 + 40 * pairs * (pairs + 1) / 2;
     }
-    if (j.opt.matsto == MPGPU_FULL) upd = 0;
     upd = std::min<int64_t>(upd, (int64_t)128 << 30);
+    scratch = std::min<int64_t>(scratch, (int64_t)128 << 30);
     int64_t nlab = 0;
     if (lmax >= lmin) {
         const int64_t span = (int64_t)lmax - lmin + 1;
@@ -106,26 +130,22 @@ int64_t estimate_footprint(const Job &j)
         for (uint64_t b : bits) nlab += __builtin_popcountll(b);
     }
     int64_t nall = nlab + (int64_t)j.ncon;
-    int64_t mat;
-    if (j.opt.matsto == MPGPU_FULL) {
-        // packed matrix, plus what the solve allocates beside it: the inversion keeps a copy
-        // (1x packed); the FP64 factor is a full n x n FP64 matrix (2x packed); the FP32 factor
-        // a full FP32 one (1x) and, when the refinement does not converge, the FP64 factor
-        // as well (2x); the error diagonal of the LAPACK methods 512 unit columns
-        const int64_t packed = 8 * nall * (nall + 1) / 2;
-        int64_t mult = 2;
-        switch (j.opt.metsol) {
-        case MPGPU_DECOMPOSITION: case MPGPU_LAPACK_PACKED: case MPGPU_LAPACK_UNPACKED: mult = 3; break;
-        case MPGPU_CHOLESKY_FP32_IR: mult = 4; break;
-        default: mult = 2;
+    int64_t mat, more = 0;
+    if (full) {
+        mat = mpgpu::full_storage_bytes(j.opt.metsol, nall) - 4096 * nall;
+        // (without room for the square matrix the inversion works in the packed one)
+        if (j.opt.metsol == MPGPU_INVERSION) {
+            more = mat;
+            mat = 2 * (8 * nall * (nall + 1) / 2);
+            more -= mat;
         }
-        mat = packed * mult;
         if (j.opt.lapack_errors && (j.opt.metsol == MPGPU_LAPACK_PACKED || j.opt.metsol == MPGPU_LAPACK_UNPACKED))
             mat += 8 * nall * 512;
     } else {
         mat = std::min<int64_t>(8 * nall * (nall + 1) / 2, 8 * nw * 24);
     }
-    return rec + mat + upd + 200 * nall + (64 << 20);
+    j.least = rec + mat + upd + 200 * nall + (64 << 20);
+    j.footprint = rec + mat + more + scratch + rows + 4096 * nall + (64 << 20);
 }
 
 } // namespace
@@ -145,8 +165,8 @@ struct mpgpu_server {
     void run_job(Job &j, hipStream_t wstream)
     {
         j.t_start = clk::now();
-        // MPGPU_VERBOSE: time of each step of the job on stderr
-        static const bool verbose = std::getenv("MPGPU_VERBOSE") != nullptr;
+        // MPGPU_VERBOSE: time of each step and memory of the job on stderr
+        const bool verbose = std::getenv("MPGPU_VERBOSE") != nullptr;
         clk::time_point tp = j.t_start;
         double ms[6] = {0, 0, 0, 0, 0, 0};
         auto lap = [&](int k) {
@@ -157,6 +177,7 @@ struct mpgpu_server {
         int rc = 0;
         mpgpu_ctx *c = nullptr;
         rc = mpgpu::create_context(&j.opt, device, wstream, &c);
+        if (!rc) mpgpu::context_memory(c).set_share((size_t)j.footprint);
         if (!rc) rc = mpgpu_add_records(c, j.nrec, j.rec_ptr, j.inder, j.glder, nullptr);
         if (!rc && j.npar > 0) rc = mpgpu_set_steering_parameters(c, j.npar, j.plab, j.pval, j.psig);
         if (!rc && j.ncon > 0) {
@@ -173,10 +194,12 @@ struct mpgpu_server {
         std::vector<double> x((size_t)nvar + ncon);
         if (!rc) rc = mpgpu_solve(c, nullptr, x.data(), &j.sst);
         lap(3);
+        if (c) j.peak = mpgpu::context_memory(c).peak();
         if (verbose)
-            std::fprintf(stderr, "job %lld: nvar %d nrec %lld: size %.1f create+copy %.1f structure %.1f pass %.1f solve %.1f ms "
+            std::fprintf(stderr, "job %lld: device memory charged %lld bytes (least %lld), in use at most %zu\n"
+                                 "job %lld: nvar %d nrec %lld: size %.1f create+copy %.1f structure %.1f pass %.1f solve %.1f ms "
                                  "(method %d, itn %d)\n",
-                         (long long)j.id, nvar, (long long)j.nrec, j.size_ms, ms[0], ms[1], ms[2], ms[3],
+                         (long long)j.id, (long long)j.footprint, (long long)j.least, j.peak, (long long)j.id, nvar, (long long)j.nrec, j.size_ms, ms[0], ms[1], ms[2], ms[3],
                          j.sst.method, j.sst.itn);
         if (!rc) {
             std::vector<int32_t> lab(ntot), var(ntot), grp(ntot);
@@ -217,18 +240,20 @@ struct mpgpu_server {
                 j = queue.front();
                 queue.pop_front();
             }
-            // size the job (a scan of its words), then wait until it fits the budget; a job
-            // alone may use more than the budget's remainder when nothing else runs
+            // size the job (a scan of its words), then wait until it fits the budget beside the
+            // running ones and the free blocks that are kept; a job whose least part fits the budget
+            // runs at least alone
             const clk::time_point t_size = clk::now();
-            j->footprint = estimate_footprint(*j);
+            size_job(*j);
             j->size_ms = std::chrono::duration<double, std::milli>(clk::now() - t_size).count();
             bool admitted = false;
             {
                 std::unique_lock<std::mutex> lk(mu);
-                if (j->footprint <= budget) {
+                if (j->least <= budget) {
                     cv_budget.wait(lk, [&] { return in_use + j->footprint <= budget || in_use == 0; });
                     in_use += j->footprint;
                     admitted = true;
+                    mpgpu::dev_store_trim(device, (size_t)std::max<int64_t>(0, budget - in_use), wstream);
                 }
             }
             if (admitted) {

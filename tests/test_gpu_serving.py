@@ -83,3 +83,58 @@ def test_budget_rejects_oversized_job():
     rc, st, lab, x = S.wait(j, capacity=10000)
     assert rc == 0 and st["nvar"] == len(lab) > 0
     S.close()
+
+
+def _sized_jobs():
+    """jobs of every method and storage, and records with and without row form"""
+    from test_gpu_rows import _records
+    rec, par, cons = _job(5, 6, 4, 3, 4000)
+    no_rows = _records(9, 30, 6, 6, 2000, 8, 2, np.float32)
+    single = _records(10, 400, 1, 3, 4000, 20, 1, np.float32)
+    dense, dpar, dcons = _job(6, 8, 6, 4, 2000)
+    full = dict(matsto=mpgpu.FULL, mreqenf=5, mcount=1)
+    block = dict(matsto=mpgpu.SPARSE, metsol=mpgpu.MINRES, mreqenf=5, mcount=1, mbandw=6, mrestl=1e-10)
+    out = []
+    for m in (mpgpu.INVERSION, mpgpu.DECOMPOSITION, mpgpu.CHOLESKY_FP32_IR, mpgpu.LAPACK_PACKED, mpgpu.MINRES):
+        out.append((rec, par, cons, dict(full, metsol=m)))
+        out.append((dense, dpar, dcons, dict(full, metsol=m)))
+    out.append((dense, dpar, dcons, dict(full, metsol=mpgpu.CHOLESKY_FP32_IR, fp32_min_n=100)))
+    for r in (no_rows, single):
+        out.append((r, None, None, dict(full, metsol=mpgpu.INVERSION, default_presigma=1.0)))
+        out.append((r, None, None, dict(block, default_presigma=1.0)))
+    for w in (0, 1):
+        out.append((rec, par, cons, dict(block, withmultipliers=w)))
+        out.append((dense, dpar, dcons, dict(block, withmultipliers=w)))
+    return out
+
+
+def test_memory_charged_to_a_job_covers_what_it_uses(monkeypatch, capfd):
+    import re
+    monkeypatch.setenv("MPGPU_VERBOSE", "1")
+    S = mpgpu.Server(nworkers=1, budget_bytes=60 << 30)
+    capfd.readouterr()
+    for rec, par, cons, opt in _sized_jobs():
+        rc, st, _, _ = S.wait(S.submit(rec, par, cons, **opt))
+        assert rc == 0, (rc, opt)
+    S.close()
+    lines = re.findall(r"charged (\d+) bytes \(least (\d+)\), in use at most (\d+)", capfd.readouterr().err)
+    assert len(lines) == len(_sized_jobs())
+    # (64 MB of every estimate are for what does not grow with the job: not for these to hide in)
+    for line, (_, _, _, opt) in zip(lines, _sized_jobs()):
+        charged, least, peak = map(int, line)
+        assert peak <= charged - (64 << 20), opt
+
+
+def test_job_whose_least_part_fits_the_budget_runs():
+    """More memory than the budget would only make the job faster: it is accepted as long as what it cannot do
+    without fits, and refused below that."""
+    rec, par, cons = _job(5, 8, 8, 6, 20000)
+    opt = dict(matsto=mpgpu.FULL, metsol=mpgpu.INVERSION, mreqenf=5, mcount=1)
+    n = 6 * 8 * 8 * 6 + 3 * 8
+    words = len(rec[1])
+    least = 12 * words + 64 * 20000 + 8 * n * (n + 1) + 200 * n + (64 << 20)
+    for budget, want in ((int(1.001 * least), 0), (int(0.9 * least), 30)):
+        S = mpgpu.Server(nworkers=2, budget_bytes=budget)
+        rc, st, _, _ = S.wait(S.submit(rec, par, cons, **opt))
+        assert rc == want
+        S.close()
