@@ -155,12 +155,6 @@ __global__ __launch_bounds__(64) void k_bp_hinv(int m, const double *h, double *
     }
 }
 
-__device__ __forceinline__ double bp_lane(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
 
 // Solution of a chunk with a zero boundary, one thread per row (b: its right-hand side): the
 // sub-chunk's inverse (M), then the boundary values carried over the sub-chunks by the first
@@ -197,7 +191,7 @@ __device__ __forceinline__ double bp_solve(double b, bool live, const double *M,
             if (r < W) sS[w * W + r] = s;
             double t = sv[w * SUB + (DIR == 0 ? SUB - W + l : l)];
 #pragma unroll
-            for (int q = 0; q < W; q++) t += sB[(w * W + l) * W + q] * bp_lane(s, q);
+            for (int q = 0; q < W; q++) t += sB[(w * W + l) * W + q] * wave_lane(s, q);
             s = t;
         }
     }

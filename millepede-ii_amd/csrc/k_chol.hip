@@ -134,11 +134,6 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
     typedef typename Mfma<T>::acc_t acc_t;
     const int nb = min(LB, n - k0);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
-    auto wfence = []() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
     // load: rows and columns past the end as those of a unit matrix
     for (int e = t; e < 36 * 256; e += DG_THREADS) {
         const int tl = e >> 8, c = (e >> 4) & 15, r = e & 15;
@@ -158,7 +153,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
         T *xi = Xs + dg_tile(p, p);
         T lt[4];
         dg_factor16<T>(dg, dg, dv + 16 * p, wv + 16 * p, Xs + dg_tile(7, 6), xi);
-        wfence();
+        wave_order();
 #pragma unroll
         for (int m = 0; m < 4; m++) lt[m] = dg[(4 * lk + m) * 16 + lr];
 #pragma unroll
@@ -166,10 +161,10 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
             const int c = 16 * p + 4 * lk + m, r = 16 * p + lr;
             if (r < nb && c <= r) a[(int64_t)(k0 + c) * lda + k0 + r] = c < r ? lt[m] : dv[c];
         }
-        wfence();
+        wave_order();
 #pragma unroll
         for (int m = 0; m < 4; m++) dg[(4 * lk + m) * 16 + lr] = (Xs + dg_tile(7, 6))[(4 * lk + m) * 16 + lr];
-        wfence();
+        wave_order();
     };
     if (wave == 0) factor(0);
     __syncthreads();
@@ -184,7 +179,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
                 const int k = 4 * s + lk;
                 acc = Mfma<T>::op(li[k * 16 + lr], tile[k * 16 + lr], acc);
             }
-            wfence();
+            wave_order();
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int c = Mfma<T>::row(lk, e), o = c * 16 + lr;
@@ -212,7 +207,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
         const int m = 7 - p;                          // trailing row tiles
         if (wave == 0) {
             update(p + 1, p + 1);
-            wfence();
+            wave_order();
             factor(p + 1);
         } else {
             for (int q = wave; q < m * (m + 1) / 2; q += 7) {
@@ -248,7 +243,7 @@ __global__ __launch_bounds__(DG_THREADS) void k_ldl_diag(int n, T *a, int lda, i
                 const int r = Mfma<T>::row(lk, e);
                 x[r * 16 + (lr ^ r)] = -y[e];
             }
-            wfence();
+            wave_order();
         }
     }
     __syncthreads();

@@ -30,16 +30,6 @@ namespace mpgpu {
 typedef double d4 __attribute__((ext_vector_type(4)));
 #define RT 256                  // threads per record workgroup
 #define RW (RT / WAVE)          // wavefronts per record workgroup
-// Lanes of one wavefront exchanging data through LDS: a wavefront executes its LDS operations
-// in order, so a wavefront-scope barrier (no wait for the wave's outstanding global stores,
-// unlike a workgroup barrier) orders them.
-#define WSYNC()                                                    \
-    do {                                                           \
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");     \
-        __builtin_amdgcn_wave_barrier();                           \
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");     \
-    } while (0)
-
 __device__ __forceinline__ double wave_sum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
@@ -174,13 +164,6 @@ __device__ __forceinline__ int gj_regs(double *cl, double *bl, int lane)
     return nrank;
 }
 
-// Value of a lane-held double at a uniform lane
-__device__ __forceinline__ double rdlane(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
 
 // sqminv (src/mpnum.f90:97-213) for a packed symmetric n x n matrix held one element per lane
 // (lane t < npk = n(n+1)/2) with the right-hand side in lanes npk .. npk+n-1 (npk + n <= 64):
@@ -210,8 +193,8 @@ __device__ int gj_lanes(double acc, int npk, int n, int lane, double *cl, double
         for (int j = 1; j <= n; j++) {
             if (!((rem >> (j - 1)) & 1ull)) continue;
             const int d = pk(j, j);
-            const double vjj = rdlane(cv, d);
-            const double m = fmax(fabs(vkk), eps * fabs(rdlane(cv0, d)));
+            const double vjj = wave_lane(cv, d);
+            const double m = fmax(fabs(vkk), eps * fabs(wave_lane(cv0, d)));
             if (fabs(vjj) > m) { vkk = vjj; k = j; }
         }
         if (k == 0) {
@@ -222,11 +205,11 @@ __device__ int gj_lanes(double acc, int npk, int n, int lane, double *cl, double
         }
         rem &= ~(1ull << (k - 1));
         nrank++;
-        const double vinv = 1.0 / rdlane(cv, pk(k, k));
+        const double vinv = 1.0 / wave_lane(cv, pk(k, k));
         const double coJ = __shfl(cv, J >= k ? pk(J, k) : pk(k, J), WAVE);
         const double coK = __shfl(cv, K >= k ? pk(K, k) : pk(k, K), WAVE);
         const double coL = __shfl(cv, L1 >= k ? pk(L1, k) : pk(k, L1), WAVE);
-        const double bk = rdlane(bv, k - 1) * vinv;
+        const double bk = wave_lane(bv, k - 1) * vinv;
         double nv;
         if (J == k && K == k) nv = -vinv;
         else if (J == k) nv = vinv * coK;
@@ -480,7 +463,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                     }
                     lw[i] = wght;
                 }
-                WSYNC();
+                wave_order();
                 // local normal equations, element-parallel, equations in order (3781-3836); systems
                 // of up to 9 parameters keep the elements in registers for the inversion
                 const bool regs5 = nalc <= 5;
@@ -544,7 +527,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                     else cl[t] = acc;
                 }
                 if (regs5) {
-                    WSYNC();
+                    wave_order();
                     switch (nalc) {
                     case 1: nrank = gj_regs<1>(cl, bl, lane); break;
                     case 2: nrank = gj_regs<2>(cl, bl, lane); break;
@@ -552,21 +535,21 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                     case 4: nrank = gj_regs<4>(cl, bl, lane); break;
                     default: nrank = gj_regs<5>(cl, bl, lane); break;
                     }
-                    WSYNC();
+                    wave_order();
                 } else if (regfit) {
                     nrank = gj_lanes(acc_r, npk, nalc, lane, cl, bl);
-                    WSYNC();
+                    wave_order();
                 } else {
-                    WSYNC();
+                    wave_order();
                     // ---- sqminv (src/mpnum.f90:97-213), element-parallel Gauss-Jordan ----
                     const double eps = 16.0 * DBL_EPSILON;
                     for (int i = lane; i < nalc; i += WAVE) {
                         dg[i] = fabs(cl[pk(i + 1, i + 1)]);
                         nxt[i + 1] = i + 2;
                     }
-                    WSYNC();
+                    wave_order();
                     if (lane == 0) { nxt[nalc] = -1; sh[1] = 1; /* next0 */ sh[2] = 0; /* nrank */ }
-                    WSYNC();
+                    wave_order();
                     for (int step = 1; step <= nalc; step++) {
                         if (lane == 0) {
                             int k = 0, l = 0, last = 0;
@@ -586,7 +569,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                             }
                             sh[3] = k;
                         }
-                        WSYNC();
+                        wave_order();
                         const int k = sh[3];
                         if (k == 0) {
                             for (int t = lane; t < npk; t += WAVE) {
@@ -597,7 +580,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                                 if (nxt[J] != 0 && nxt[K] != 0) cl[t] = 0.0;
                             }
                             for (int i = lane; i < nalc; i += WAVE) if (nxt[i + 1] != 0) bl[i] = 0.0;
-                            WSYNC();
+                            wave_order();
                             break;
                         }
                         const int kk = pk(k, k);
@@ -609,7 +592,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                                 cs[j - 1] = vkk * v;
                             }
                         }
-                        WSYNC();
+                        wave_order();
                         const double bk = bl[k - 1] * vkk;
                         for (int t = lane; t < npk; t += WAVE) {
                             int J = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5) + 1;
@@ -625,11 +608,11 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                             if (j == k) bl[j - 1] = bk;
                             else bl[j - 1] = bl[j - 1] - bk * co[j - 1];
                         }
-                        WSYNC();
+                        wave_order();
                     }
                     for (int t = lane; t < npk; t += WAVE) cl[t] = -cl[t];
                     nrank = sh[2];
-                    WSYNC();
+                    wave_order();
                 }
                 // NaN check (3903-3906)
                 int nan = 0;
@@ -702,7 +685,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 }
                 summ = wave_sum(s_chi);
                 double suwt = wave_sum(s_wt);
-                WSYNC();
+                wave_order();
                 ndf = neq - nrank;
                 resing = ((float)neq - (float)suwt) / (float)neq;
                 if (nan > 0) { status = 1; break; }
@@ -713,22 +696,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             int ndf_add = 0;
             if (status == 0) {
                 // chi^2 cuts with REAL(4) thresholds (4106-4131)
-                float chichi;
-                {
-                    // chindl(3, ndf) (src/mpnum.f90:2078-2115)
-                    const float tab3[30] = {9.0000f, 5.9146f, 4.7184f, 4.0628f, 3.6410f, 3.3436f, 3.1209f, 2.9468f,
-                                            2.8063f, 2.6902f, 2.5922f, 2.5082f, 2.4352f, 2.3711f, 2.3143f, 2.2635f,
-                                            2.2178f, 2.1764f, 2.1386f, 2.1040f, 2.0722f, 2.0428f, 2.0155f, 1.9901f,
-                                            1.9665f, 1.9443f, 1.9235f, 1.9040f, 1.8855f, 1.8681f};
-                    float c;
-                    if (ndf < 1) c = 0.0f;
-                    else if (ndf <= 30) c = tab3[ndf - 1];
-                    else {
-                        float t = 2.782170f + sqrtf((float)(ndf + ndf - 1));
-                        c = t * t / (float)(ndf + ndf);
-                    }
-                    chichi = c * (float)ndf;
-                }
+                const float chichi = three_sigma_chi2(ndf);
                 if (o.chicut >= 0.0f) {
                     if (summ > (double)(o.chhuge * chichi)) status = 5;
                     else if (o.chicut > 0.0f) {

@@ -133,18 +133,6 @@ __device__ void sqminv_small(double *v, double *b, int n, int *nrank, double *di
     for (int i = 1; i <= (n * n + n) / 2; i++) v[i] = -v[i];
 }
 
-// wavefront-wide order of LDS accesses (one wavefront's LDS operations complete in order)
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-__device__ __forceinline__ double readlane_d(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l), hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
 // Equations in order, 64 at a time, by one wavefront: lane q gets word q of the equation (its local
 // or total position and its value), the words of the next equations are in flight, and
 // f(i, words) does equation i.  Every equation has at most 64 words.
@@ -279,8 +267,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
     int32_t *gpos = gv + P.max_gl;                 // [max_gl]
     int32_t *gvl = gpos + P.max_gl;                // [max_var]
     int32_t *segof = gvl + P.max_var;              // [max_var]
-    int32_t *seggr = segof + P.max_var;            // [max_var]
-    int32_t *clsof = seggr + P.max_var;            // [max_var]
+    int32_t *clsof = segof + P.max_var;            // [max_var]
     int32_t *gptr = clsof + P.max_var;             // [max_var + 1]
     int32_t *cls0 = gptr + P.max_var + 1;          // [max_var + 1] first global of each class
     int32_t *sptr = cls0 + P.max_var + 1;          // [max_var + 1] support offsets of each class
@@ -366,7 +353,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
         const bool eq1 = sh[7] == 0, one = nmb <= 64 && mbnd <= 10;
         const int tn = one ? 64 : BNT;
         auto tsync = [&]() {
-            if (one) wave_sync();
+            if (one) wave_order();
             else __syncthreads();
         };
         if (nalg > P.max_var || nalc > NA || nalc <= 0 || nmb <= 0) {
@@ -424,7 +411,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
                     const double wght = lw[i];
                     if (rhs) bl[ij] = bl[ij] + wght * rm[i] * vj;
                     else if (tid < npair) put(ij, ik, wght * vj * vk);
-                    wave_sync();
+                    wave_order();
                 });
             for (int i = 0; i < (eq1 ? 0 : neq); i++) {
                 const int64_t sl = R.eq_sl[e0 + i];
@@ -632,21 +619,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
         double chi_add = 0.0;
         int ndf_add = 0;
         if (status == 0) {
-            float chichi;
-            {
-                const float tab3[30] = {9.0000f, 5.9146f, 4.7184f, 4.0628f, 3.6410f, 3.3436f, 3.1209f, 2.9468f,
-                                        2.8063f, 2.6902f, 2.5922f, 2.5082f, 2.4352f, 2.3711f, 2.3143f, 2.2635f,
-                                        2.2178f, 2.1764f, 2.1386f, 2.1040f, 2.0722f, 2.0428f, 2.0155f, 1.9901f,
-                                        1.9665f, 1.9443f, 1.9235f, 1.9040f, 1.8855f, 1.8681f};
-                float c;
-                if (ndf < 1) c = 0.0f;
-                else if (ndf <= 30) c = tab3[ndf - 1];
-                else {
-                    float t = 2.782170f + sqrtf((float)(ndf + ndf - 1));
-                    c = t * t / (float)(ndf + ndf);
-                }
-                chichi = c * (float)ndf;
-            }
+            const float chichi = three_sigma_chi2(ndf);
             if (o.chicut >= 0.0f) {
                 if (summ > (double)(o.chhuge * chichi)) status = 5;
                 else if (o.chicut > 0.0f) {
@@ -675,7 +648,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
                 bool st = (a < nalg) && (a == 0 || g != gprev);
                 unsigned long long m = __ballot(st);
                 int s = nseg + __popcll(m & ((2ull << tid) - 1ull)) - 1;
-                if (a < nalg) { segof[a] = s; if (st) { seggr[s] = g; segfn[s] = make_int2(M.gfirst[g], M.gfirst[g + 1] - M.gfirst[g]); } }
+                if (a < nalg) { segof[a] = s; if (st) segfn[s] = make_int2(M.gfirst[g], M.gfirst[g + 1] - M.gfirst[g]); }
                 nseg += __popcll(m);
             }
             int npair = (nseg * nseg + nseg) / 2;
@@ -880,7 +853,7 @@ __global__ __launch_bounds__(BNT, 4) void k_records_band(DevRecords R, DevModel 
                             }
                         }
                     }
-                    wave_sync();
+                    wave_order();
                 });
             for (int i = 0; i < (eq1 ? 0 : neq); i++) {
                 g_pairs(i, tid, BNT);
@@ -1026,7 +999,7 @@ int band_lds_bytes(BandPlan &P)
                2 * ((size_t)P.nbdr_max + 1) + (size_t)P.mp1_max * (NA + 1) + P.max_sup + 8;
     P.nwm = (P.nalc_max + 63) / 64;
     size_t u64 = (size_t)P.max_var * P.nwm;
-    size_t i32 = 2 * (size_t)P.max_gl + 4 * (size_t)P.max_var + 4 * ((size_t)P.max_var + 1) + P.max_sup + P.max_pair +
+    size_t i32 = 2 * (size_t)P.max_gl + 3 * (size_t)P.max_var + 4 * ((size_t)P.max_var + 1) + P.max_sup + P.max_pair +
                  P.nbdr_max + 1 + 32;
     size_t b = d * 8 + u64 * 8 + i32 * 4;
     // the local inverse in LDS behind the rest where four workgroups still fit a CU, else in memory

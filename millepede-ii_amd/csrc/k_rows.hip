@@ -37,22 +37,10 @@ namespace mpgpu {
 #define PERM_WINDOW 4096         // blocks whose order the gather may change
 #define MAXSEQ 4                 // equations of one group in a record
 
-__device__ __forceinline__ void rsync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __device__ __forceinline__ double rsum(double v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WV);
     return v;
-}
-__device__ __forceinline__ double rlane(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -115,7 +103,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_class(int64_t nrec, const i
             nl_max = max(nl_max, __shfl_xor(nl_max, o, WV));
             gs_max = max(gs_max, __shfl_xor(gs_max, o, WV));
         }
-        rsync();
+        wave_order();
         // groups of the record: runs of its (sorted) label list; a group has units when one of its
         // variables is in the list
         int nseg = 0, nu = 0;
@@ -154,7 +142,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_class(int64_t nrec, const i
             mx_nl = max(mx_nl, nl_max);
             mx_g = max(mx_g, gs_max);
         }
-        rsync();
+        wave_order();
     }
     if (lane == 0) {
         atomicMax(&maxes[0], mx_eq);
@@ -230,7 +218,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_fill(int64_t nq, const int6
             }
             nseg += __popcll(m);
         }
-        rsync();
+        wave_order();
         int nalc = 0;
         for (int i = lane; i < neq; i += WV) {
             const int64_t sl = eq_sl[e0 + i];
@@ -263,7 +251,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_fill(int64_t nq, const int6
             es[i] = (uint8_t)sgi;
         }
         for (int o = 32; o > 0; o >>= 1) nalc = max(nalc, __shfl_xor(nalc, o, WV));
-        rsync();
+        wave_order();
         // equations of each group, ascending, and their places in the units
         int before = 0, ubefore = 0;
         for (int b0 = 0; b0 < nseg; b0 += WV) {
@@ -307,7 +295,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_fill(int64_t nq, const int6
             h.nunit = ubefore;
             hdr[q] = h;
         }
-        rsync();
+        wave_order();
     }
 }
 
@@ -330,7 +318,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_incidence(int64_t q0, int64
                 for (int u = 0; u < un; u++) ug[u0 + u] = g;
             }
         }
-        rsync();
+        wave_order();
         const int64_t out = pr0[q] - pr0[q0];
         const int np = h.nunit * (h.nunit + 1) / 2;
         const uint32_t base = (uint32_t)(h.unit0 - ub);
@@ -343,7 +331,7 @@ __global__ __launch_bounds__(WV *RWAVES) void k_rows_incidence(int64_t q0, int64
             key[out + t] = (uint32_t)(wrank[o >> 5] + __popc(bits[o >> 5] & ((1u << (o & 31)) - 1u)));
             val[out + t] = make_uint2(base + a, base + b);
         }
-        rsync();
+        wave_order();
     }
 }
 
@@ -405,7 +393,7 @@ __device__ __forceinline__ int rows_gj(double acc, int nalc, int lane, int J, in
     const int L1 = lane < N ? lane : 0;
     double dg[N];
 #pragma unroll
-    for (int j = 0; j < N; j++) dg[j] = eps * fabs(rlane(cv, j * (j + 1) / 2 + j));
+    for (int j = 0; j < N; j++) dg[j] = eps * fabs(wave_lane(cv, j * (j + 1) / 2 + j));
     unsigned rem = (1u << nalc) - 1u;
     int nrank = 0;
     for (int step = 0; step < nalc; step++) {
@@ -413,7 +401,7 @@ __device__ __forceinline__ int rows_gj(double acc, int nalc, int lane, int J, in
         double vkk = 0.0;
 #pragma unroll
         for (int j = 0; j < N; j++) {
-            const double vjj = rlane(cv, j * (j + 1) / 2 + j);
+            const double vjj = wave_lane(cv, j * (j + 1) / 2 + j);
             if (((rem >> j) & 1u) && fabs(vjj) > fmax(fabs(vkk), dg[j])) { vkk = vjj; k = j; }
         }
         k = __builtin_amdgcn_readfirstlane(k);
@@ -429,7 +417,7 @@ __device__ __forceinline__ int rows_gj(double acc, int nalc, int lane, int J, in
         const double coJ = __shfl(cv, pk(J, k), WV);
         const double coK = __shfl(cv, pk(K, k), WV);
         const double coL = __shfl(cv, pk(L1, k), WV);
-        const double bk = rlane(bv, k) * vinv;
+        const double bk = wave_lane(bv, k) * vinv;
         if (lane < N) st[step].mu[lane] = ((rem >> lane) & 1u) ? coL * vinv : 0.0;
         if (lane == 0) { st[step].pivot = vkk; st[step].k = k; }
         double nv;
@@ -445,21 +433,6 @@ __device__ __forceinline__ int rows_gj(double acc, int nalc, int lane, int J, in
     return nrank;
 }
 
-__device__ __forceinline__ float rows_chichi(int ndf)
-{
-    // chindl(3, ndf) * ndf (src/mpnum.f90:2078-2115)
-    const float tab3[30] = {9.0000f, 5.9146f, 4.7184f, 4.0628f, 3.6410f, 3.3436f, 3.1209f, 2.9468f, 2.8063f, 2.6902f,
-                            2.5922f, 2.5082f, 2.4352f, 2.3711f, 2.3143f, 2.2635f, 2.2178f, 2.1764f, 2.1386f, 2.1040f,
-                            2.0722f, 2.0428f, 2.0155f, 1.9901f, 1.9665f, 1.9443f, 1.9235f, 1.9040f, 1.8855f, 1.8681f};
-    float c;
-    if (ndf < 1) c = 0.0f;
-    else if (ndf <= 30) c = tab3[ndf - 1];
-    else {
-        float t = 2.782170f + sqrtf((float)(ndf + ndf - 1));
-        c = t * t / (float)(ndf + ndf);
-    }
-    return c * (float)ndf;
-}
 
 // LDS of one wavefront (bytes): weights and products [mq], the local inverse and solution, the
 // elimination steps, local derivatives and (without BUILD) group derivatives of the equations
@@ -564,7 +537,7 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
                 wt[c] = wght;
                 w[i] = wght;
             }
-            rsync();
+            wave_order();
             double acc = 0.0;
             if (lane < NE) {
                 // equations in order; the products are rounded before they are added, as the
@@ -591,7 +564,7 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
                 }
             }
             nrank = rows_gj<N>(acc, nalc, lane, J, K, cb, st);
-            rsync();
+            wave_order();
             double b[N];
 #pragma unroll
             for (int k = 0; k < N; k++) b[k] = cb[NPK + k];
@@ -645,7 +618,7 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
         int ndf_add = 0;
         if (status == 0) {
             // chi^2 cuts with REAL(4) thresholds (4106-4131)
-            const float chichi = rows_chichi(ndf);
+            const float chichi = three_sigma_chi2(ndf);
             if (o.chicut >= 0.0f) {
                 if (summ > (double)(o.chhuge * chichi)) status = 5;
                 else if (o.chicut > 0.0f) {
@@ -749,7 +722,7 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
         summ = rsum(s_chi);
         if (lane == 0) { out.status[h.rec] = 0; out.chi2[h.rec] = summ; out.ndf[h.rec] = ndf; }
-        rsync();
+        wave_order();
         if (BUILD) continue;
         // ---- vector and counters (4184-4186): one lane per parameter of the record's groups ----
         for (int base = 0; base < h.nseg * GP; base += VL) {
@@ -769,7 +742,7 @@ __global__ __launch_bounds__(WV *RWAVES) __attribute__((amdgpu_waves_per_eu(4)))
             atomicAdd(&M.vec[d.x + j - 1], v);
             atomicAdd(&M.cnt[d.x + j - 1], (unsigned long long)cnt);
         }
-        rsync();
+        wave_order();
     }
 }
 

@@ -632,9 +632,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int64_t npart, const R
             sd[w][lane] = R.o;
             sd[w][8 + lane] = R.n;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_order();
         if (t + 2 < nsteps) load(t + 2, R);
         if (k < kn) {
             const int off = sd[w][k], nc = sd[w][8 + k];
@@ -654,9 +652,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_st(int64_t npart, const R
                 tb[(g0 + k) * tbw + j] = sv;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_order();
     };
     StepRegs RA, RB;
     if (nsteps > 0) load(0, RA);
@@ -768,9 +764,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int64_t npart, const Ro
             for (int i = 0; i < NV; i++) st[w][min(lane + 64 * i, max(len, 1) - 1)] = R.v[i];
         }
         sx[w][lane] = R.x;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_order();
         {
             const int64_t t2 = min(t + 2, nsteps - 1), t3 = min(t + 3, nsteps - 1);
             col_next = ld_col(t3);
@@ -789,9 +783,7 @@ __global__ __launch_bounds__(64 * W) void k_bsymv_rows_u(int64_t npart, const Ro
         for (int r = 0; r < G; r++) tv += B[r * G + min(j, G - 1)] * xa[r];
         const bool ok = k < kn && j < G;
         tb[ok ? (g0 + k) * G + j : tb_spare + lane] = tv;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_order();
     };
     for (int64_t t = 0; t < nsteps; t += 2) {
         step(t, RA);
@@ -1850,21 +1842,12 @@ __global__ void k_band_h(int32_t m, const int *cb, const int64_t *koff, const do
         if (threadIdx.x < 64) {
             const int lane = threadIdx.x;
             const double eps = 16.0 * DBL_EPSILON;
-            auto pick = [](double v, int l) {
-                return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
-                                        __builtin_amdgcn_readlane(__double2loint(v), l));
-            };
-            auto order = [] {
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            };
             int nr = 0;
             const double h0 = hs[0];
             if (!(h0 > 0.0)) nr = -1;
-            order();
+            wave_order();
             if (lane == 0) hs[0] = h0 > 0.0 ? 1.0 / sqrt(h0) : 0.0;
-            order();
+            wave_order();
             for (int k = 1; k < m; k++) {
                 const int rk = (k * k + k) / 2, j1 = lane + 64;
                 const int q0 = min(lane, k), q1 = min(j1, k);
@@ -1875,21 +1858,21 @@ __global__ void k_band_h(int32_t m, const int *cb, const int64_t *koff, const do
                 for (int i = 0; i < k; i++) {
                     const double di = hs[(i * i + i) / 2 + i];
                     const double a0 = hs[o0 + min(i, q0)], a1 = hs[o1 + min(i, q1)];
-                    const double v = pick(i < 64 ? c0 : c1, i & 63) * di;
+                    const double v = wave_lane(i < 64 ? c0 : c1, i & 63) * di;
                     c0 = lane == i ? v : lane > i ? c0 - v * (lane >= k ? v : a0) : c0;
                     c1 = j1 == i ? v : j1 > i ? c1 - v * (j1 >= k ? v : a1) : c1;
                 }
-                const double ck = pick(k < 64 ? c0 : c1, k & 63);
+                const double ck = wave_lane(k < 64 ? c0 : c1, k & 63);
                 const bool ok = ck > eps * dk;
                 const double piv = 1.0 / sqrt(ck);
                 if (!ok) {
                     if (nr == 0) nr = -(k + 1);
                     else { if (nr < 0) nr = 1; nr++; }
                 }
-                order();
+                wave_order();
                 if (lane <= k) hs[rk + lane] = !ok ? 0.0 : lane == k ? piv : c0;
                 if (j1 <= k) hs[rk + j1] = !ok ? 0.0 : j1 == k ? piv : c1;
-                order();
+                wave_order();
             }
             if (lane == 0) *nrkd2 = nr;
         }
@@ -2526,12 +2509,6 @@ __global__ __launch_bounds__(64) void k_spk_local(int n, int nch, const double *
 // boundary row per lane (lane i < w: its row of S and value of x in registers, the next chunk's
 // row read ahead) and the carried values broadcast with readlane.
 #define SPK_LDS_DOUBLES 6144
-__device__ __forceinline__ double spk_rdlane(double v, int l)
-{
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
 template <int W>
 __global__ __launch_bounds__(256) void k_spk_carry(int n, int nch, const double *x, const double *S, double *t, int backward)
 {
@@ -2578,7 +2555,7 @@ __global__ __launch_bounds__(256) void k_spk_carry(int n, int nch, const double 
                 double v = xa;
                 if (coupled) {
 #pragma unroll
-                    for (int q = 0; q < W; q++) v += sa[q] * spk_rdlane(cur, q);
+                    for (int q = 0; q < W; q++) v += sa[q] * wave_lane(cur, q);
                 }
                 if (L < w) {
                     // chunk shorter than w (the last one): rows outside it carry through
@@ -2745,13 +2722,13 @@ __global__ __launch_bounds__(64) void k_eqs_small(int n, int m, const double *h,
             const int fk = k - indk + indk1 + 1;       // first column of row k
             for (int j = 1; j <= m; j++) {
                 if (lane == j - 1) xv = xv * sh_h[indk - 1];
-                const double xj = spk_rdlane(xv, j - 1);
+                const double xj = wave_lane(xv, j - 1);
                 if (lane < m && k > j && j >= fk) xv = xv - sh_h[indk - k + j - 1] * xj;
             }
             for (int kk = m; kk >= 2; kk--) {
                 const int ik = sh_i[kk - 1], ik1 = sh_i[kk - 2];
                 if (lane == kk - 1) xv = xv * sh_h[ik - 1];
-                const double xk = spk_rdlane(xv, kk - 1);
+                const double xk = wave_lane(xv, kk - 1);
                 const int fkk = kk - ik + ik1 + 1;
                 if (k < kk && k >= fkk) xv = xv - sh_h[ik - kk + k - 1] * xk;
             }

@@ -25,12 +25,6 @@ namespace mpgpu {
 #define SW 64
 #define STRUCT_WAVES 4
 
-__device__ __forceinline__ void wsync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (SW - 1); }
 template <typename T> __device__ __forceinline__ T wmax(T v)
 {
@@ -293,7 +287,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_labels(int64_t nrec, i
         }
         for (int i = m + lane; i < P; i += SW) keys[i] = ~0ull;
         for (int i = lane; i < m; i += SW) unz[i] = 0;
-        wsync();
+        wave_order();
         // bitonic sort of keys[0, P)
         for (int k = 2; k <= P; k <<= 1)
             for (int j = k >> 1; j > 0; j >>= 1) {
@@ -307,7 +301,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_labels(int64_t nrec, i
                         }
                     }
                 }
-                wsync();
+                wave_order();
             }
         // runs of equal total index: the record's distinct labels
         int nrun = 0;
@@ -328,7 +322,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_labels(int64_t nrec, i
             }
             nrun += __popcll(sm);
         }
-        wsync();
+        wave_order();
         if (lane == 0) ngl[r] = nrun;
         for (int k = lane; k < nrun; k += SW) tmp_gl[mofs[r] + k] = U[k];
         if (PER_RECORD) {
@@ -352,12 +346,12 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_labels(int64_t nrec, i
                 const uint32_t n = eq_n[e];
                 const int ng = (int)(n >> 16);
                 const int64_t sg = eq_sl[e] + (n & 0xffff) + 1;
-                wsync();
+                wave_order();
                 for (int j = lane; j < ng; j += SW) {
                     const int64_t wd = sg + 1 + j;
                     sc[j] = val[wd] != T(0) ? tix_of(L, I[wd]) : -1;
                 }
-                wsync();
+                wave_order();
                 for (int j = lane; j < ng; j += SW) {
                     const int32_t x = sc[j];
                     if (x < 0) continue;
@@ -374,7 +368,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_labels(int64_t nrec, i
                 }
             }
         }
-        wsync();
+        wave_order();
     }
 }
 
@@ -419,7 +413,7 @@ __device__ int record_segments(int64_t g0, int64_t g1, const int32_t *gl_tix, co
         const int glast = __shfl(g, live ? 63 - __clzll(live) : 0, SW);
         if (live) lastg = glast;
     }
-    wsync();
+    wave_order();
     for (int s0 = 0; s0 < nseg; s0 += SW) {
         const int s = s0 + lane;
         int a = 0, b = 0;
@@ -427,9 +421,9 @@ __device__ int record_segments(int64_t g0, int64_t g1, const int32_t *gl_tix, co
             a = sz[s];
             b = s + 1 < nseg ? sz[s + 1] : nlive;
         }
-        wsync();
+        wave_order();
         if (s < nseg) sz[s] = b - a;
-        wsync();
+        wave_order();
     }
     nv = nlive;
     return nseg;
@@ -459,7 +453,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_stats(int64_t nrec, in
         const int nseg = record_segments(g0, g1, gl_tix, var, group_of, s_g, s_z, nv);
         const int ngl = (int)(g1 - g0);
         for (int k = lane; k < ngl; k += SW) qc[k] = 0;
-        wsync();
+        wave_order();
         int nalc = 0;
         int64_t sup = 0;
         for (int64_t eb = e0; eb < e1; eb += SW) {
@@ -478,7 +472,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_stats(int64_t nrec, in
         }
         nalc = wmax(nalc);
         sup = wsum(sup);
-        wsync();
+        wave_order();
         int qe = 0;
         for (int k = lane; k < ngl; k += SW) qe = max(qe, qc[k]);
         qe = wmax(qe);
@@ -507,7 +501,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_rec_stats(int64_t nrec, in
                 set_bit(pbits, pair_bit(s_g[a], s_g[b]));
             }
         }
-        wsync();
+        wave_order();
     }
 }
 
@@ -611,7 +605,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_pair_blocks(int64_t nrec, 
             pair_of(t, a, b);
             pair_blk[rec_pb[r] + t] = (int32_t)bit_rank(pair_bit(s_g[a], s_g[b]), bits, wrank);
         }
-        wsync();
+        wave_order();
     }
 }
 
@@ -676,7 +670,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_incidence(int64_t q0, int6
                 reg += (int64_t)s_z[a] * upto + ((s_z[a] + 3) & ~3);
             }
         }
-        wsync();
+        wave_order();
         const int64_t out = pos[q - q0], np = (int64_t)nseg * (nseg + 1) / 2;
         for (int64_t t = lane; t < np; t += SW) {
             int a, b;
@@ -684,7 +678,7 @@ __global__ __launch_bounds__(SW *STRUCT_WAVES) void k_incidence(int64_t q0, int6
             key[out + t] = (uint32_t)pair_blk[rec_pb[r] + t];
             val[out + t] = rec_cb[r] + s_reg[a] + (int64_t)s_col[b] * s_z[a];
         }
-        wsync();
+        wave_order();
     }
 }
 

@@ -126,6 +126,37 @@ struct BandPlan {
     int32_t bytes;
 };
 
+// Order of the LDS accesses of one wavefront's lanes: a wavefront executes its LDS operations in
+// order, so this has no wait for its outstanding global accesses, unlike a workgroup barrier
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// value of a lane-held double at a uniform lane
+__device__ __forceinline__ double wave_lane(double v, int l)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+    return __hiloint2double(hi, lo);
+}
+// chindl(3, ndf) * ndf (src/mpnum.f90:2078-2115) in REAL(4): the three-sigma limit of chi^2
+__device__ __forceinline__ float three_sigma_chi2(int ndf)
+{
+    const float tab3[30] = {9.0000f, 5.9146f, 4.7184f, 4.0628f, 3.6410f, 3.3436f, 3.1209f, 2.9468f, 2.8063f, 2.6902f,
+                            2.5922f, 2.5082f, 2.4352f, 2.3711f, 2.3143f, 2.2635f, 2.2178f, 2.1764f, 2.1386f, 2.1040f,
+                            2.0722f, 2.0428f, 2.0155f, 1.9901f, 1.9665f, 1.9443f, 1.9235f, 1.9040f, 1.8855f, 1.8681f};
+    float c;
+    if (ndf < 1) c = 0.0f;
+    else if (ndf <= 30) c = tab3[ndf - 1];
+    else {
+        float t = 2.782170f + sqrtf((float)(ndf + ndf - 1));
+        c = t * t / (float)(ndf + ndf);
+    }
+    return c * (float)ndf;
+}
+
 // MINRES recurrence state in device memory (src/minresModule.f90:294-660): the dot products of an
 // iteration land here, one thread advances the scalar recurrence and the vector kernels read
 // their coefficients from it; once istop is set the remaining launched iterations do nothing
