@@ -13,6 +13,9 @@
 // carried boundary, the constraint block and the backward solve share one kernel, the constraint
 // factor's inverse (m x m, formed once per matrix) replaces its two substitutions (20 us for 60
 // constraints), and the backward correction is left to the kernel that takes MINRES's dot product.
+//
+// Contexts with eliminated constraints keep the substitutions of k_spk_*: their solves may end at the
+// iteration limit, where another order of sums shows in the result (mpgpu_ctx::elim).
 #include "mpgpu_internal.h"
 
 namespace mpgpu {

@@ -24,7 +24,7 @@
 // the next four equations in flight, and as many records as possible are in flight beside each
 // other: 128 registers for four workgroups a CU, though some values spill (three without spills: 8.4
 // against 5.4 ms), and a grid of what is resident.  20,000 broken-lines tracks of up to 44 local
-// parameters: pass 14.8 -> 5.4 ms, without the matrix 4.2 -> 2.1 ms.
+// parameters: 12.2 -> 5.3 ms.
 #include "mpgpu_device.h"
 #include <float.h>
 
